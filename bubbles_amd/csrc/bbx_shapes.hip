@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -22,8 +23,8 @@ struct bbx_sdf {
 
 namespace {
 
-constexpr int kTriTile = 128;  // triangles staged per LDS round (9 doubles each)
-constexpr int kSdfBlock = 256;
+constexpr int kSdfWaves = 4;  // waves that share a brick of 4 x 4 x 4 nodes
+constexpr int kSdfBlock = 64 * kSdfWaves;
 
 __device__ __forceinline__ double sgn_d(double a) { return a > 0 ? 1.0 : (a < 0 ? -1.0 : 0.0); }
 __device__ __forceinline__ double clamp_d(double v, double lo, double hi) {
@@ -77,43 +78,242 @@ __device__ double tri_solid_angle(const double *t, double px, double py, double 
     return 2.0 * atan2(det, den);
 }
 
+__device__ __forceinline__ double det3(double ax, double ay, double az, double bx, double by, double bz, double cx,
+                                       double cy, double cz) {
+    return ax * (by * cz - bz * cy) - ay * (bx * cz - bz * cx) + az * (bx * cy - by * cx);
+}
+
+// By how much the winding number of a mesh changes from q to p through
+// triangle abc: 0, or +-1 where the segment crosses it (tri_solid_angle is
+// positive on the side where det(a - p, b - p, c - p) is).  A determinant
+// within eps of zero tells nothing; *sure = 0 where the answer needs it.
+__device__ __forceinline__ double tri_crossing(const double *t, double px, double py, double pz, double qx, double qy,
+                                               double qz, double eps, int *sure) {
+    const double ax = t[0] - px, ay = t[1] - py, az = t[2] - pz;
+    const double bx = t[3] - px, by = t[4] - py, bz = t[5] - pz;
+    const double cx = t[6] - px, cy = t[7] - py, cz = t[8] - pz;
+    const double dx = qx - px, dy = qy - py, dz = qz - pz;
+    // signed volumes: p and q against the plane, the segment against the edges
+    const double sp = det3(ax, ay, az, bx, by, bz, cx, cy, cz);
+    const double sq = det3(ax - dx, ay - dy, az - dz, bx - dx, by - dy, bz - dz, cx - dx, cy - dy, cz - dz);
+    const double e0 = det3(dx, dy, dz, ax, ay, az, bx, by, bz);
+    const double e1 = det3(dx, dy, dz, bx, by, bz, cx, cy, cz);
+    const double e2 = det3(dx, dy, dz, cx, cy, cz, ax, ay, az);
+    const bool beside = (fmax(fmax(e0, e1), e2) > eps && fmin(fmin(e0, e1), e2) < -eps) ||  // the line misses it
+                        fmin(sp, sq) > eps || fmax(sp, sq) < -eps;                          // one side of the plane
+    const bool through = (fmin(fmin(e0, e1), e2) > eps || fmax(fmax(e0, e1), e2) < -eps) &&
+                         fmin(sp, sq) < -eps && fmax(sp, sq) > eps;
+    *sure = beside || through;
+    return beside || !through ? 0.0 : (sp > 0.0 ? 1.0 : -1.0);
+}
+
+__device__ __forceinline__ float lane_of(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// A triangle's bounding sphere (centroid and radius, FP32, relative to the
+// grid's origin).  `slack` covers the FP32 rounding of a position inside the
+// grid.  A triangle that tri_dist2 cannot measure (an edge of no length, no
+// area, coordinates that are not finite) gets an infinite radius: it is never
+// passed over and bounds nothing.
+__global__ void __launch_bounds__(256) k_tri_spheres(const double *__restrict__ tri, int ntri, double ox, double oy,
+                                                     double oz, float slack, float4 *__restrict__ sphere) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= ntri) return;
+    const double *v = tri + 9 * (size_t)t;
+    const double cx = (v[0] + v[3] + v[6]) / 3.0, cy = (v[1] + v[4] + v[7]) / 3.0, cz = (v[2] + v[5] + v[8]) / 3.0;
+    double r2 = 0.0, e2 = DBL_MAX;
+    for (int k = 0; k < 3; k++) {
+        const double *a = v + 3 * k, *b = v + 3 * ((k + 1) % 3);
+        r2 = fmax(r2, (a[0] - cx) * (a[0] - cx) + (a[1] - cy) * (a[1] - cy) + (a[2] - cz) * (a[2] - cz));
+        e2 = fmin(e2, (a[0] - b[0]) * (a[0] - b[0]) + (a[1] - b[1]) * (a[1] - b[1]) + (a[2] - b[2]) * (a[2] - b[2]));
+    }
+    const double ux = v[3] - v[0], uy = v[4] - v[1], uz = v[5] - v[2];
+    const double wx = v[6] - v[0], wy = v[7] - v[1], wz = v[8] - v[2];
+    const double nx = uy * wz - uz * wy, ny = uz * wx - ux * wz, nz = ux * wy - uy * wx;
+    const bool sound = e2 > 0.0 && nx * nx + ny * ny + nz * nz > 0.0 && r2 < 1e30 && fabs(cx) + fabs(cy) + fabs(cz) < 1e30;
+    sphere[t] = make_float4((float)(cx - ox), (float)(cy - oy), (float)(cz - oz),
+                            sound ? (float)sqrt(r2) * 1.000001f + slack : __builtin_inff());
+}
+
 // SetNodeSDFKernel (src/core/shape.cpp:411-424) for a mesh: distance to the
 // closest triangle, at least 1e-5, negative inside.  Inside is decided by
-// the winding number of the closed mesh (the reference counts ray hits
-// towards the mesh's bounds centre, src/core/shape.cpp:356-373).
-__global__ void __launch_bounds__(kSdfBlock) k_sdf_from_mesh(const double *__restrict__ tri, int ntri, int nx,
+// the winding number of the mesh (the reference counts ray hits towards the
+// mesh's bounds centre, src/core/shape.cpp:356-373).
+//
+// A workgroup holds a brick of 4 x 4 x 4 nodes, one per lane in each of its
+// waves, and splits the triangles between the waves.  FP64 distances and solid angles
+// of every (node, triangle) pair bounded the kernel (4.03 ms at 229k nodes
+// and 1,280 triangles, about 2,100 cycles per pair of a wave), so most pairs
+// get neither (0.31 ms; 34 to 2.1 ms at 572k nodes and 5,120 triangles of a
+// ball, whose centre no bound helps and one wave alone took 4.6 ms over):
+//  - Centroids bound the brick's distances from above, bounding spheres bound
+//    them from below: FP32, a triangle per lane.  Only triangles that some
+//    node of the brick may be closest to go on to a test per node and then
+//    to tri_dist2.  The minimum is over the same values as before.
+//  - The winding number of a closed mesh changes by one where a path meets
+//    the surface.  The brick's farthest node is evaluated by the workgroup (a
+//    256th of the triangles per lane), the others by the triangles that
+//    the path from it crosses, of those that reach into the brick.
+//  - A node whose path is too close to an edge or a plane to tell, and every
+//    node of a mesh that is not closed (or has a triangle without area),
+//    takes the whole sum in triangle order: at the surface and in an opening
+//    the winding number is 1/2 up to its rounding.
+__global__ void __launch_bounds__(kSdfBlock) k_sdf_from_mesh(const double *__restrict__ tri,
+                                                             const float4 *__restrict__ sphere, int ntri, int nx,
                                                              int ny, int nz, double ox, double oy, double oz,
-                                                             double dx, float *__restrict__ out) {
+                                                             double dx, float slack, int closed,
+                                                             float *__restrict__ out) {
 #pragma clang fp contract(off)
-    __shared__ double st[kTriTile * 9];
-    const long long total = (long long)nx * ny * nz;
-    const long long node = (long long)blockIdx.x * kSdfBlock + threadIdx.x;
-    const bool live = node < total;
-    double px = 0, py = 0, pz = 0;
-    if (live) {
-        const long long i = node % nx, j = (node / nx) % ny, k = node / ((long long)nx * ny);
-        px = ox + dx * (double)i;
-        py = oy + dx * (double)j;
-        pz = oz + dx * (double)k;
+    __shared__ unsigned near_up[64];   // per node: bits of the smallest bound so far
+    __shared__ double part[kSdfWaves][64];
+    __shared__ float red[3][kSdfWaves];
+    __shared__ int red_at[kSdfWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int bx = (nx + 3) / 4, by = (ny + 3) / 4;
+    const int brick = (int)blockIdx.x;
+    const int i = brick % bx * 4 + (lane & 3), j = brick / bx % by * 4 + (lane >> 2 & 3),
+              k = brick / (bx * by) * 4 + (lane >> 4);
+    const bool live = i < nx && j < ny && k < nz;
+    const double px = ox + dx * (double)i, py = oy + dx * (double)j, pz = oz + dx * (double)k;
+    const float fx = (float)(px - ox), fy = (float)(py - oy), fz = (float)(pz - oz);
+    // the brick's centre and the radius that holds its nodes
+    const float half = 1.5f * (float)dx;
+    const float cx = __shfl(fx, 0, 64) + half, cy = __shfl(fy, 0, 64) + half, cz = __shfl(fz, 0, 64) + half;
+    const float brad = 1.7321f * half + slack;
+    float c2 = __builtin_inff(), rmax = 0.f, edge = 0.f;
+    int nearest = 0;
+    for (int t = wave * 64 + lane; t < ntri; t += kSdfBlock) {
+        const float4 s = sphere[t];
+        const float ax = cx - s.x, ay = cy - s.y, az = cz - s.z, d2 = ax * ax + ay * ay + az * az;
+        const bool sound = s.w < 3.4e38f;
+        if (sound && d2 < c2) {
+            c2 = d2;
+            nearest = t;
+        }
+        rmax = fmaxf(rmax, s.w);
+        edge = fmaxf(edge, sound ? s.w : 0.f);
     }
+    for (int off = 32; off > 0; off >>= 1) {
+        const float o2 = __shfl_xor(c2, off, 64);
+        const int ot = __shfl_xor(nearest, off, 64);
+        if (o2 < c2) {
+            c2 = o2;
+            nearest = ot;
+        }
+        rmax = fmaxf(rmax, __shfl_xor(rmax, off, 64));
+        edge = fmaxf(edge, __shfl_xor(edge, off, 64));
+    }
+    if (lane == 0) {
+        red[0][wave] = c2;
+        red[1][wave] = rmax;
+        red[2][wave] = edge;
+        red_at[wave] = nearest;
+    }
+    if (wave == 0) near_up[lane] = 0x7f800000u;
+    __syncthreads();
+    for (int w = 0; w < kSdfWaves; w++) {
+        if (red[0][w] < c2) {
+            c2 = red[0][w];
+            nearest = red_at[w];
+        }
+        rmax = fmaxf(rmax, red[1][w]);
+        edge = fmaxf(edge, red[2][w]);
+    }
+    // lanes of a wave may hold different triangles at equal distances
+    nearest = __builtin_amdgcn_readfirstlane(nearest);
+    // every node's distance is below `up`: the nearest centroid's, plus what
+    // the lower end of the edge parameters (1e-4 of an edge) can add
+    float up = sqrtf(c2) * 1.000001f + brad + slack + 1e-3f * edge;
+    const float brick_up = up + brad;
     double best = DBL_MAX;
-    double wind = 0.0;
-    for (int t0 = 0; t0 < ntri; t0 += kTriTile) {
-        const int cnt = min(kTriTile, ntri - t0);
-        __syncthreads();
-        for (int e = threadIdx.x; e < cnt * 9; e += kSdfBlock) st[e] = tri[(size_t)t0 * 9 + e];
-        __syncthreads();
-        if (live) {
-            for (int t = 0; t < cnt; t++) {
-                best = fmin(best, tri_dist2(&st[t * 9], px, py, pz));
-                wind += tri_solid_angle(&st[t * 9], px, py, pz);
+    auto measure = [&](int t) {
+        best = fmin(best, tri_dist2(tri + 9 * (size_t)t, px, py, pz));
+        up = fminf(up, (float)sqrt(best) * 1.000001f + slack);
+    };
+    measure(nearest);
+    for (int t0 = wave * 64; t0 < ntri; t0 += kSdfBlock) {
+        const float4 s = t0 + lane < ntri ? sphere[t0 + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float ax = cx - s.x, ay = cy - s.y, az = cz - s.z, reach = brick_up + s.w;
+        // both tests are written so that a NaN keeps the triangle
+        unsigned long long keep =
+            __ballot(t0 + lane < ntri && !(ax * ax + ay * ay + az * az > reach * reach * 1.00001f));
+        for (; keep; keep &= keep - 1) {
+            const int l = __builtin_ctzll(keep);
+            const float ux = fx - lane_of(s.x, l), uy = fy - lane_of(s.y, l), uz = fz - lane_of(s.z, l);
+            const float r = up + lane_of(s.w, l);
+            if (__ballot(live && !(ux * ux + uy * uy + uz * uz > r * r * 1.00001f))) {
+                measure(t0 + l);
+                // what one wave finds narrows the search of the others
+                up = fminf(up, __uint_as_float(atomicMin(&near_up[lane], __float_as_uint(up))));
             }
         }
     }
+    part[wave][lane] = best;
+    __syncthreads();
+    for (int w = 0; w < kSdfWaves; w++) best = fmin(best, part[w][lane]);
+    __syncthreads();
+    const double dist = sqrt(best);
+    bool interior = false;
+    unsigned long long todo = __ballot(live);
+    if (closed && rmax < 3.4e38f) {
+        // the brick's farthest node, by the whole workgroup
+        const float far = live ? (float)dist : -1.f;
+        float top = far;
+        for (int off = 32; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, 64));
+        const unsigned long long at = __ballot(live && far == top);
+        const int rep = at ? __builtin_ctzll(at) : 0;
+        const double qx = __shfl(px, rep, 64), qy = __shfl(py, rep, 64), qz = __shfl(pz, rep, 64);
+        double turns = 0.0;
+        for (int t = wave * 64 + lane; t < ntri; t += kSdfBlock) turns += tri_solid_angle(tri + 9 * (size_t)t, qx, qy, qz);
+        for (int off = 32; off > 0; off >>= 1) turns += __shfl_xor(turns, off, 64);
+        // the others by the triangles between them and it; each lane its own path
+        double number = 0.0;
+        bool unsure = false;
+        for (int t0 = wave * 64; t0 < ntri; t0 += kSdfBlock) {
+            const float4 s = t0 + lane < ntri ? sphere[t0 + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+            const float ax = cx - s.x, ay = cy - s.y, az = cz - s.z, reach = brad + s.w;
+            unsigned long long near = __ballot(t0 + lane < ntri && !(ax * ax + ay * ay + az * az > reach * reach * 1.00001f));
+            for (; near; near &= near - 1) {
+                const int l = __builtin_ctzll(near);
+                const double len = 2.0 * ((double)lane_of(s.w, l) + (double)brad);
+                int sure;
+                number += tri_crossing(tri + 9 * (size_t)(t0 + l), px, py, pz, qx, qy, qz,
+                                       1e-10 * len * len * (len + 1e6 * (double)slack), &sure);
+                unsure = unsure || (!sure && lane != rep);
+            }
+        }
+        // crossings are whole numbers: 1e6 marks a path that cannot tell
+        part[wave][lane] = (unsure ? 1e6 : 0.0) + number + turns / (4.0 * M_PI);
+        __syncthreads();
+        double sum = 0.0;
+        for (int w = 0; w < kSdfWaves; w++) sum += part[w][lane];
+        number = rint(sum);
+        interior = fabs(number) > 0.5;
+        todo &= __ballot(!(fabs(sum - number) < 1e-3) || fabs(number) > 5e5);
+    }
+    if (wave > 0) return;
+    if (__popcll(todo) > 24) {  // every node for itself is cheaper then
+        double wind = 0.0;
+        for (int t = 0; t < ntri; t++) wind += tri_solid_angle(tri + 9 * (size_t)t, px, py, pz);
+        if (todo >> lane & 1ull) interior = fabs(wind) > 2.0 * M_PI;  // |winding number| > 1/2
+        todo = 0ull;
+    }
+    for (; todo; todo &= todo - 1) {
+        const int rep = __builtin_ctzll(todo);
+        const double qx = __shfl(px, rep, 64), qy = __shfl(py, rep, 64), qz = __shfl(pz, rep, 64);
+        double wind = 0.0;
+        for (int t0 = 0; t0 < ntri; t0 += 64) {
+            const double a = t0 + lane < ntri ? tri_solid_angle(tri + 9 * (size_t)(t0 + lane), qx, qy, qz) : 0.0;
+            for (int l = 0; l < 64; l++)
+                wind += __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(a), l),
+                                         __builtin_amdgcn_readlane(__double2loint(a), l));
+        }
+        if (lane == rep) interior = fabs(wind) > 2.0 * M_PI;
+    }
     if (live) {
-        const bool interior = fabs(wind) > 2.0 * M_PI;  // |winding number| > 1/2
-        const double psd = fmax(sqrt(best), 0.00001);
-        out[node] = (float)(interior ? -psd : psd);
+        const double psd = fmax(dist, 0.00001);
+        out[(size_t)i + (size_t)nx * ((size_t)j + (size_t)ny * (size_t)k)] = (float)(interior ? -psd : psd);
     }
 }
 
@@ -237,6 +437,33 @@ int to_device(const bbx_collider &h, DevCollider &d) {
     return BBX_OK;
 }
 
+// Whether the triangles' directed edges cancel (each edge is walked as often
+// one way as the other), so that the winding number is the same along any
+// path off the surface.  Edges are compared by vertex index; a mesh whose
+// triangles do not share vertices counts as open (as does any without the
+// memory to tell).
+bool closed_mesh(const int *triangles, int ntriangles) try {
+    size_t cap = 64;
+    while (cap < 6 * (size_t)ntriangles) cap *= 2;
+    std::vector<unsigned long long> key(cap, 0);
+    std::vector<int> net(cap, 0);
+    for (int t = 0; t < ntriangles; t++)
+        for (int c = 0; c < 3; c++) {
+            const unsigned a = (unsigned)triangles[3 * (size_t)t + c], b = (unsigned)triangles[3 * (size_t)t + (c + 1) % 3];
+            if (a == b) continue;
+            const unsigned long long k = ((unsigned long long)(std::min(a, b) + 1) << 32) | (std::max(a, b) + 1);
+            size_t h = (size_t)((k * 0x9E3779B97F4A7C15ull) >> 20) & (cap - 1);
+            while (key[h] && key[h] != k) h = (h + 1) & (cap - 1);
+            key[h] = k;
+            net[h] += a < b ? 1 : -1;
+        }
+    for (int v : net)
+        if (v) return false;
+    return true;
+} catch (const std::bad_alloc &) {
+    return false;
+}
+
 int upload_colliders(const bbx_collider *list, int count, std::vector<DevCollider> &out) {
     if (count < 0 || count > kMaxColliders) return fail(BBX_E_RANGE, "collider count out of range (0..64)");
     if (count && !list) return fail(BBX_E_INVALID, "null collider list");
@@ -325,14 +552,22 @@ int bbx_sdf_from_mesh(const double *vertices, int nvertices, const int *triangle
         s->spacing[k] = sp;
     }
     const long long total = (long long)s->nodes[0] * s->nodes[1] * s->nodes[2];
+    // triangles, then their bounding spheres
     double *dtri = nullptr;
+    const size_t tri_bytes = (sizeof(double) * tri.size() + 255) / 256 * 256;
+    const bool closed = closed_mesh(triangles, ntriangles);
+    const float slack = (float)(1e-6 * (width + height + depth));
     hipError_t e = hipMalloc((void **)&s->field, sizeof(float) * (size_t)total);
-    if (e == hipSuccess) e = hipMalloc((void **)&dtri, sizeof(double) * tri.size());
+    if (e == hipSuccess) e = hipMalloc((void **)&dtri, tri_bytes + sizeof(float4) * (size_t)ntriangles);
     if (e == hipSuccess) e = hipMemcpy(dtri, tri.data(), sizeof(double) * tri.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) {
-        const unsigned blocks = (unsigned)((total + kSdfBlock - 1) / kSdfBlock);
-        k_sdf_from_mesh<<<blocks, kSdfBlock>>>(dtri, ntriangles, s->nodes[0], s->nodes[1], s->nodes[2], pmin[0],
-                                               pmin[1], pmin[2], sp, s->field);
+        float4 *sphere = (float4 *)((char *)dtri + tri_bytes);
+        k_tri_spheres<<<(unsigned)((ntriangles + 255) / 256), 256>>>(dtri, ntriangles, pmin[0], pmin[1], pmin[2],
+                                                                     slack, sphere);
+        const long long bricks = (long long)((s->nodes[0] + 3) / 4) * ((s->nodes[1] + 3) / 4) * ((s->nodes[2] + 3) / 4);
+        k_sdf_from_mesh<<<(unsigned)bricks, kSdfBlock>>>(
+            dtri, sphere, ntriangles, s->nodes[0], s->nodes[1], s->nodes[2], pmin[0], pmin[1], pmin[2], sp, slack,
+            closed ? 1 : 0, s->field);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipDeviceSynchronize();
