@@ -18,7 +18,41 @@
 namespace bbx {
 
 constexpr int kWaves = 4;         // waves per workgroup
-constexpr int kTilesPerWave = 4;  // training tiles per wave per step
+
+// Training weights in MFMA A layout: BF16 blocks of 64 lanes x 4 entries,
+// written by k_mlp_pack and kept up to date by the Adam update, so that a
+// wave fetches a block with one coalesced 8-byte load per lane.
+constexpr int kPackW1 = 0;                    // W1 block m: rows 16m + l%16, cols 4q..4q+3
+constexpr int kPackW2 = 4;                    // W2 block (m, kc): rows 16m + l%16, cols 16kc + 4q..
+constexpr int kPackW2T = 20;                  // W2^T block (kc, m): rows 16kc + l%16, cols 16m + 4q..
+constexpr int kPackBlocks = 36;
+constexpr int kPackEntries = kPackBlocks * 256;  // unsigned short
+
+// entries of parameter p in the packed layout (-1: none)
+__device__ __forceinline__ void pack_at(int p, int &a, int &b) {
+    a = b = -1;
+    if (p < OFF_B1) {
+        const int r = p / kF, c = p % kF;
+        a = (kPackW1 + r / 16) * 256 + ((r % 16) + 16 * (c / 4)) * 4 + c % 4;
+    } else if (p >= OFF_W2 && p < OFF_B2) {
+        const int r = (p - OFF_W2) / kH, c = (p - OFF_W2) % kH;
+        a = (kPackW2 + (r / 16) * 4 + c / 16) * 256 + ((r % 16) + 16 * (c % 16 / 4)) * 4 + c % 4;
+        b = (kPackW2T + (c / 16) * 4 + r / 16) * 256 + ((c % 16) + 16 * (r % 16 / 4)) * 4 + r % 4;
+    }
+}
+
+__device__ __forceinline__ void pack_store(unsigned short *__restrict__ wp, int p, float v) {
+    int a, b;
+    pack_at(p, a, b);
+    const unsigned short h = f2bf(v);
+    if (a >= 0) wp[a] = h;
+    if (b >= 0) wp[b] = h;
+}
+
+__global__ void __launch_bounds__(256) k_mlp_pack(const float *__restrict__ P, unsigned short *__restrict__ wp) {
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < kTrainable) pack_store(wp, p, P[p]);
+}
 
 // Weights in MFMA A layout, loaded once per wave.
 struct Weights {
@@ -29,27 +63,29 @@ struct Weights {
     float mean[4], istd[4];  // features 4q..4q+3
 };
 
-__device__ __forceinline__ void load_weights(const float *__restrict__ P, Weights &w, int lane) {
-    const int r = lane & 15, q = lane >> 4;
+__device__ __forceinline__ void load4(const float *__restrict__ p, float (&v)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = p[k];
+}
+
+__device__ __forceinline__ void load_weights(const float *__restrict__ P, const bf16x4 *__restrict__ wp, Weights &w,
+                                             bf16x4 (&w2t)[4][4], int lane) {
+    const int q = lane >> 4;
+#pragma unroll
     for (int m = 0; m < 4; m++) {
-        const float *row = P + OFF_W1 + (16 * m + r) * kF + 4 * q;
-        w.w1[m] = pack4(row[0], row[1], row[2], row[3]);
+        w.w1[m] = wp[(kPackW1 + m) * 64 + lane];
+#pragma unroll
         for (int kc = 0; kc < 4; kc++) {
-            const float *r2 = P + OFF_W2 + (16 * m + r) * kH + 16 * kc + 4 * q;
-            w.w2[m][kc] = pack4(r2[0], r2[1], r2[2], r2[3]);
+            w.w2[m][kc] = wp[(kPackW2 + 4 * m + kc) * 64 + lane];
+            w2t[m][kc] = wp[(kPackW2T + 4 * m + kc) * 64 + lane];
         }
-        for (int v = 0; v < 4; v++) {
-            int h = 16 * m + 4 * q + v;
-            w.b1[m][v] = P[OFF_B1 + h];
-            w.b2[m][v] = P[OFF_B2 + h];
-            w.w3[m][v] = P[OFF_W3 + h];
-        }
+        load4(P + OFF_B1 + 16 * m + 4 * q, w.b1[m]);
+        load4(P + OFF_B2 + 16 * m + 4 * q, w.b2[m]);
+        load4(P + OFF_W3 + 16 * m + 4 * q, w.w3[m]);
     }
     w.b3 = P[OFF_B3];
-    for (int v = 0; v < 4; v++) {
-        w.mean[v] = P[OFF_MEAN + 4 * q + v];
-        w.istd[v] = P[OFF_ISTD + 4 * q + v];
-    }
+    load4(P + OFF_MEAN + 4 * q, w.mean);
+    load4(P + OFF_ISTD + 4 * q, w.istd);
 }
 
 struct Acts {
@@ -148,9 +184,15 @@ __global__ void __launch_bounds__(64 * kWaves) k_mlp_infer(const float *__restri
 }
 
 // ---------------------------------------------------------------------------
-// training: forward + backward over kTilesPerWave tiles per wave; per-wave
-// gradient partials, reduced in a fixed order by k_mlp_reduce.
+// training: forward + backward of one 16-sample tile per wave, the weight
+// gradients of a workgroup's four tiles split between its waves; one partial
+// gradient per workgroup, reduced in a fixed order by k_mlp_reduce.
 // Loss = 0.5 / B * sum (y_j - t_j / out_scale)^2 over the batch.
+//
+// A batch is small (4,096 samples are 256 tiles), so the time is the chain
+// of latencies of one wave: four tiles in turn per wave, and the weights
+// gathered as FP32 with strides, took 26.6 us for 4,096 samples.  A tile per
+// wave and packed weights take 9.2 us.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ unsigned long long mix64(unsigned long long z) {
     z += 0x9E3779B97F4A7C15ull;
@@ -160,152 +202,183 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long z) {
 }
 
 __global__ void __launch_bounds__(64 * kWaves) k_mlp_grad(const float *__restrict__ P,
+                                                          const bf16x4 *__restrict__ wp,
                                                           const float *__restrict__ xs,
                                                           const float *__restrict__ ts, int n,
                                                           int batch, int random, unsigned long long seed,
                                                           float expectile,
                                                           float *__restrict__ gpart,
                                                           float *__restrict__ lpart) {
-    __shared__ unsigned short lds[kWaves][3][kH * 16];  // dz2, h1, dz1 tiles [hidden][sample]
-    __shared__ unsigned short ldx[kWaves][kF * 16];     // x tile [feature][sample]
+    // the four tiles' dz2, h1, dz1 [hidden][sample] and x [feature][sample]
+    __shared__ __align__(16) unsigned short lds[kWaves][3][kH * 16];
+    __shared__ __align__(16) unsigned short ldx[kWaves][kF * 16];
+    // bias and output-layer gradients (result layout), loss terms: one tile
+    // after the other adds to them
+    __shared__ f32x4 lb[3][4][64];
+    __shared__ float ldy[2][64];
     const int lane = threadIdx.x & 63, wl = threadIdx.x >> 6;
-    const int wave = blockIdx.x * kWaves + wl;
     const int q = lane >> 4, j = lane & 15;
+    const int bpos = (blockIdx.x * kWaves + wl) * 16 + j;  // position in the batch
+    const bool valid = bpos < batch;
+    int idx = 0;
+    if (valid) idx = random ? (int)(mix64(seed ^ ((unsigned long long)bpos << 20)) % (unsigned long long)n) : bpos;
+    float x4[4];
+    load4(xs + (size_t)idx * kF + 4 * q, x4);
+#pragma unroll
+    for (int v = 0; v < 4; v++) x4[v] = valid ? x4[v] : 0.f;
+    const float traw = ts[idx];
     Weights w;
-    load_weights(P, w, lane);
-    // W2^T in A layout for dH1 = W2^T dZ2: block (kc, m2), rows 16kc + l%16
     bf16x4 w2t[4][4];
-    for (int kc = 0; kc < 4; kc++)
-        for (int m2 = 0; m2 < 4; m2++) {
-            float e[4];
-            for (int v = 0; v < 4; v++) e[v] = P[OFF_W2 + (16 * m2 + 4 * q + v) * kH + 16 * kc + j];
-            w2t[kc][m2] = pack4(e[0], e[1], e[2], e[3]);
-        }
+    load_weights(P, wp, w, w2t, lane);
     const float inv_os = 1.f / P[OFF_OSCALE];
     const float inv_b = 1.f / (float)batch;
-    f32x4 gW2[4][4], gW1[4];
-    for (int a = 0; a < 4; a++) {
-        gW1[a] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int b = 0; b < 4; b++) gW2[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    float gb1[4][4] = {}, gb2[4][4] = {}, gw3[4][4] = {};
-    float gb3 = 0.f, loss = 0.f;
+    Acts a;
+    forward_tile(w, x4, a, lane);
+    const float tj = valid ? traw * inv_os : 0.f;
+    const float diff = valid ? (a.y - tj) : 0.f;
+    // expectile weight: 2 (1 - tau) above the target, 2 tau below (1 at tau = 0.5)
+    const float wgt = diff > 0.f ? 2.f * (1.f - expectile) : 2.f * expectile;
+    const float dy = wgt * diff * inv_b;
+    // layer 3 and layer-2 activations; dH1 = W2^T dZ2 (dz2 already in B layout)
     unsigned short *T2 = lds[wl][0], *T1 = lds[wl][1], *T3 = lds[wl][2], *TX = ldx[wl];
-    for (int tt = 0; tt < kTilesPerWave; tt++) {
-        const int bpos = (wave * kTilesPerWave + tt) * 16 + j;  // position in the batch
-        const bool valid = bpos < batch;
-        int idx = 0;
-        if (valid) idx = random ? (int)(mix64(seed ^ ((unsigned long long)bpos << 20)) % (unsigned long long)n) : bpos;
-        float x4[4];
-        for (int v = 0; v < 4; v++) x4[v] = valid ? xs[(size_t)idx * kF + 4 * q + v] : 0.f;
-        Acts a;
-        forward_tile(w, x4, a, lane);
-        const float tj = valid ? ts[idx] * inv_os : 0.f;
-        const float diff = valid ? (a.y - tj) : 0.f;
-        // expectile weight: 2 (1 - tau) above the target, 2 tau below (1 at tau = 0.5)
-        const float wgt = diff > 0.f ? 2.f * (1.f - expectile) : 2.f * expectile;
-        const float dy = wgt * diff * inv_b;
-        if (lane < 16) {
-            loss += 0.5f * wgt * diff * diff * inv_b;
-            gb3 += dy;
-        }
-        // layer 3 and layer-2 activations
-        float dz2[4][4];
-        for (int m2 = 0; m2 < 4; m2++)
-            for (int v = 0; v < 4; v++) {
-                gw3[m2][v] += dy * a.g2[m2][v];
-                dz2[m2][v] = w.w3[m2][v] * dy * a.d2[m2][v];
-                gb2[m2][v] += dz2[m2][v];
-            }
-        // dH1 = W2^T dZ2 (dz2 already in B layout)
-        bf16x4 dz2b[4];
-        for (int m2 = 0; m2 < 4; m2++) dz2b[m2] = pack4(dz2[m2][0], dz2[m2][1], dz2[m2][2], dz2[m2][3]);
-        float dz1[4][4];
-        for (int kc = 0; kc < 4; kc++) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            for (int m2 = 0; m2 < 4; m2++) acc = mfma(w2t[kc][m2], dz2b[m2], acc);
-            for (int v = 0; v < 4; v++) {
-                dz1[kc][v] = acc[v] * a.d1[kc][v];
-                gb1[kc][v] += dz1[kc][v];
-            }
-        }
-        // transpose dz2, h1, dz1, x through LDS: tile[hidden][sample]
-        __syncthreads();
-        for (int m = 0; m < 4; m++)
-            for (int v = 0; v < 4; v++) {
-                const int hrow = 16 * m + 4 * q + v;
-                T2[hrow * 16 + j] = f2bf(dz2[m][v]);
-                T1[hrow * 16 + j] = f2bf(a.g1[m][v]);
-                T3[hrow * 16 + j] = f2bf(dz1[m][v]);
-            }
-        for (int v = 0; v < 4; v++) TX[(4 * q + v) * 16 + j] = f2bf(a.xn[v]);
-        __syncthreads();
-        // A operands: rows (hidden) 16m + l%16, cols (samples) 4q..4q+3
-        bf16x4 A2[4], A3[4], B1[4];
-        for (int m = 0; m < 4; m++) {
-            const int hrow = 16 * m + j;
-            for (int v = 0; v < 4; v++) {
-                A2[m][v] = (short)T2[hrow * 16 + 4 * q + v];
-                A3[m][v] = (short)T3[hrow * 16 + 4 * q + v];
-                B1[m][v] = (short)T1[hrow * 16 + 4 * q + v];  // B: rows samples 4q.., col hidden 16m + l%16
-            }
-        }
-        bf16x4 BX;
-        for (int v = 0; v < 4; v++) BX[v] = (short)TX[j * 16 + 4 * q + v];
-        // dW2[i][k] += sum_j dz2[i][j] h1[k][j]
-        for (int m2 = 0; m2 < 4; m2++)
-            for (int kc = 0; kc < 4; kc++) gW2[m2][kc] = mfma(A2[m2], B1[kc], gW2[m2][kc]);
-        // dW1[i][f] += sum_j dz1[i][j] x[f][j]
-        for (int m = 0; m < 4; m++) gW1[m] = mfma(A3[m], BX, gW1[m]);
-    }
-    // per-wave partials
-    float *g = gpart + (size_t)wave * kTrainable;
-    for (int m = 0; m < 4; m++)
+    bf16x4 dz2b[4];
+    f32x4 dh1[4];
+#pragma unroll
+    for (int m2 = 0; m2 < 4; m2++) {
+        float dz[4];
+#pragma unroll
         for (int v = 0; v < 4; v++) {
-            const int row = 16 * m + 4 * q + v;
-            g[OFF_W1 + row * kF + j] = gW1[m][v];
-            for (int kc = 0; kc < 4; kc++) g[OFF_W2 + row * kH + 16 * kc + j] = gW2[m][kc][v];
+            dz[v] = w.w3[m2][v] * dy * a.d2[m2][v];
+            T2[(16 * m2 + 4 * q + v) * 16 + j] = f2bf(dz[v]);
         }
-    // reduce per-hidden-unit sums over the 16 samples (lanes sharing q)
-    for (int m = 0; m < 4; m++)
-        for (int v = 0; v < 4; v++) {
-            float s1 = gb1[m][v], s2 = gb2[m][v], s3 = gw3[m][v];
-            for (int off = 1; off < 16; off <<= 1) {
-                s1 += __shfl_xor(s1, off, 64);
-                s2 += __shfl_xor(s2, off, 64);
-                s3 += __shfl_xor(s3, off, 64);
-            }
-            if (j == 0) {
-                const int h = 16 * m + 4 * q + v;
-                g[OFF_B1 + h] = s1;
-                g[OFF_B2 + h] = s2;
-                g[OFF_W3 + h] = s3;
-            }
-        }
-    for (int off = 1; off < 64; off <<= 1) {
-        gb3 += __shfl_xor(gb3, off, 64);
-        loss += __shfl_xor(loss, off, 64);
+        dz2b[m2] = pack4(dz[0], dz[1], dz[2], dz[3]);
     }
-    if (lane == 0) {
-        g[OFF_B3] = gb3;
-        lpart[wave] = loss;
+#pragma unroll
+    for (int kc = 0; kc < 4; kc++) {
+        dh1[kc] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m2 = 0; m2 < 4; m2++) dh1[kc] = mfma(w2t[kc][m2], dz2b[m2], dh1[kc]);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int at = (16 * kc + 4 * q + v) * 16 + j;
+            T3[at] = f2bf(dh1[kc][v] * a.d1[kc][v]);
+            T1[at] = f2bf(a.g1[kc][v]);
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++) TX[(4 * q + v) * 16 + j] = f2bf(a.xn[v]);
+    for (int t = 0; t < kWaves; t++) {
+        if (wl == t) {
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+                f32x4 b1 = t ? lb[0][m][lane] : zero, b2 = t ? lb[1][m][lane] : zero, w3 = t ? lb[2][m][lane] : zero;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    b1[v] = fmaf(dh1[m][v], a.d1[m][v], b1[v]);
+                    b2[v] = fmaf(w.w3[m][v] * dy, a.d2[m][v], b2[v]);
+                    w3[v] = fmaf(dy, a.g2[m][v], w3[v]);
+                }
+                lb[0][m][lane] = b1;
+                lb[1][m][lane] = b2;
+                lb[2][m][lane] = w3;
+            }
+            const float wd = wgt * diff;
+            ldy[0][lane] = lane < 16 ? fmaf(wd, inv_b, t ? ldy[0][lane] : 0.f) : 0.f;
+            ldy[1][lane] = lane < 16 ? fmaf(0.5f * wgt * diff * diff, inv_b, t ? ldy[1][lane] : 0.f) : 0.f;
+        }
+        __syncthreads();
+    }
+    // Wave wl takes hidden rows 16 wl .. 16 wl + 15 over the workgroup's
+    // tiles in order: dW2[i][k] += sum_j dz2[i][j] h1[k][j] and
+    // dW1[i][f] += sum_j dz1[i][j] x[f][j].  A operands: rows (hidden)
+    // 16 wl + l%16, cols (samples) 4q..4q+3; B: rows samples, col l%16.
+    f32x4 gW2[4], gW1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kc = 0; kc < 4; kc++) gW2[kc] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const f32x4 s1 = lb[0][wl][lane], s2 = lb[1][wl][lane], s3 = lb[2][wl][lane];
+#pragma unroll
+    for (int t = 0; t < kWaves; t++) {
+        const int at = (16 * wl + j) * 16 + 4 * q;
+        const bf16x4 A2 = *reinterpret_cast<const bf16x4 *>(&lds[t][0][at]);
+        const bf16x4 A3 = *reinterpret_cast<const bf16x4 *>(&lds[t][2][at]);
+        const bf16x4 BX = *reinterpret_cast<const bf16x4 *>(&ldx[t][j * 16 + 4 * q]);
+#pragma unroll
+        for (int kc = 0; kc < 4; kc++)
+            gW2[kc] = mfma(A2, *reinterpret_cast<const bf16x4 *>(&lds[t][1][(16 * kc + j) * 16 + 4 * q]), gW2[kc]);
+        gW1 = mfma(A3, BX, gW1);
+    }
+    float *g = gpart + (size_t)blockIdx.x * kTrainable;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int row = 16 * wl + 4 * q + v;
+        g[OFF_W1 + row * kF + j] = gW1[v];
+#pragma unroll
+        for (int kc = 0; kc < 4; kc++) g[OFF_W2 + row * kH + 16 * kc + j] = gW2[kc][v];
+        // the hidden unit's sums over the 16 samples (lanes sharing q)
+        float b1 = s1[v], b2 = s2[v], w3 = s3[v];
+#pragma unroll
+        for (int off = 1; off < 16; off <<= 1) {
+            b1 += __shfl_xor(b1, off, 64);
+            b2 += __shfl_xor(b2, off, 64);
+            w3 += __shfl_xor(w3, off, 64);
+        }
+        if (j == 0) {
+            g[OFF_B1 + row] = b1;
+            g[OFF_B2 + row] = b2;
+            g[OFF_W3 + row] = w3;
+        }
+    }
+    if (wl == 0) {
+        float gb3 = ldy[0][lane], loss = ldy[1][lane];
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            gb3 += __shfl_xor(gb3, off, 64);
+            loss += __shfl_xor(loss, off, 64);
+        }
+        if (lane == 0) {
+            g[OFF_B3] = gb3;
+            lpart[blockIdx.x] = loss;
+        }
     }
 }
 
-// grad[p] = sum over waves in index order (deterministic); optional Adam step
-__global__ void k_mlp_reduce(const float *__restrict__ gpart, const float *__restrict__ lpart,
-                             int nwaves, float *__restrict__ grad, float *__restrict__ loss_out,
-                             float *__restrict__ P, float *__restrict__ m1, float *__restrict__ m2,
-                             int adam, float lr, float bc1, float bc2) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p == 0) {
+// grad[p] = sum over the partials in index order (deterministic); optional
+// Adam step, which also renews the packed weights.  One wave per workgroup:
+// 84 of them spread the loads over the chip, and a thread has sixteen in
+// flight (18.5 us with four-wave workgroups and a load at a time, 4.4 us
+// now, for the 64 partials of 4,096 samples).  The last workgroup sums the
+// loss, a partial per lane, in index order too.
+constexpr int kReduceBlocks = (kTrainable + 63) / 64;
+__global__ void __launch_bounds__(64) k_mlp_reduce(const float *__restrict__ gpart, const float *__restrict__ lpart,
+                                                   int parts, float *__restrict__ grad, float *__restrict__ loss_out,
+                                                   float *__restrict__ P, unsigned short *__restrict__ wp,
+                                                   float *__restrict__ m1, float *__restrict__ m2, int adam, float lr,
+                                                   float bc1, float bc2) {
+    const int lane = threadIdx.x;
+    if (blockIdx.x == kReduceBlocks) {
         float l = 0.f;
-        for (int w = 0; w < nwaves; w++) l += lpart[w];
-        *loss_out = l;
+        for (int w0 = 0; w0 < parts; w0 += 64) {
+            const float v = w0 + lane < parts ? lpart[w0 + lane] : 0.f;
+            const int m = min(64, parts - w0);
+            for (int k = 0; k < m; k++) l += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
+        }
+        if (lane == 0) *loss_out = l;
+        return;
     }
+    const int p = blockIdx.x * 64 + lane;
     if (p >= kTrainable) return;
+    constexpr int kAhead = 16;
     float s = 0.f;
-    for (int w = 0; w < nwaves; w++) s += gpart[(size_t)w * kTrainable + p];
+    int w = 0;
+    for (; w + kAhead <= parts; w += kAhead) {
+        float v[kAhead];
+#pragma unroll
+        for (int k = 0; k < kAhead; k++) v[k] = gpart[(size_t)(w + k) * kTrainable + p];
+#pragma unroll
+        for (int k = 0; k < kAhead; k++) s += v[k];
+    }
+    for (; w < parts; w++) s += gpart[(size_t)w * kTrainable + p];
     grad[p] = s;
     if (adam) {
         const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
@@ -313,7 +386,9 @@ __global__ void k_mlp_reduce(const float *__restrict__ gpart, const float *__res
         float b = b2 * m2[p] + (1.f - b2) * s * s;
         m1[p] = a;
         m2[p] = b;
-        P[p] -= lr * (a / bc1) / (sqrtf(b / bc2) + eps);
+        const float v = P[p] - lr * (a / bc1) / (sqrtf(b / bc2) + eps);
+        P[p] = v;
+        pack_store(wp, p, v);
     }
 }
 
@@ -324,10 +399,11 @@ using namespace bbx;
 struct bbx_mlp {
     float *params = nullptr;   // kParams FP32 (device)
     float *m1 = nullptr, *m2 = nullptr, *grad = nullptr, *loss = nullptr;
+    unsigned short *wpack = nullptr;  // BF16 weights in MFMA layout (training)
     float *gpart = nullptr, *lpart = nullptr;
-    int gpart_waves = 0;
+    int gpart_parts = 0;
     float *data_x = nullptr, *data_t = nullptr;  // resident training set (sample-major)
-    int data_n = 0;
+    int data_n = 0;                              // samples the two buffers hold
     float *tmp_x = nullptr, *tmp_y = nullptr;
     int tmp_n = 0;
     int adam_t = 0;
@@ -351,15 +427,23 @@ static int ensure_tmp(bbx_mlp *m, int n) {
     return BBX_OK;
 }
 
-static int ensure_gpart(bbx_mlp *m, int waves) {
-    if (waves <= m->gpart_waves) return BBX_OK;
+static int ensure_gpart(bbx_mlp *m, int parts) {
+    if (parts <= m->gpart_parts) return BBX_OK;
     if (m->gpart) (void)hipFree(m->gpart);
     if (m->lpart) (void)hipFree(m->lpart);
     m->gpart = m->lpart = nullptr;
-    m->gpart_waves = 0;
-    BBX_HIP_CHECK(hipMalloc((void **)&m->gpart, sizeof(float) * (size_t)waves * kTrainable));
-    BBX_HIP_CHECK(hipMalloc((void **)&m->lpart, sizeof(float) * (size_t)waves));
-    m->gpart_waves = waves;
+    m->gpart_parts = 0;
+    BBX_HIP_CHECK(hipMalloc((void **)&m->gpart, sizeof(float) * (size_t)parts * kTrainable));
+    BBX_HIP_CHECK(hipMalloc((void **)&m->lpart, sizeof(float) * (size_t)parts));
+    m->gpart_parts = parts;
+    return BBX_OK;
+}
+
+// the packed weights of the current parameters; before the first gradient
+// pass of a call (the Adam update keeps them up to date within one)
+static int pack_launch(bbx_mlp *m) {
+    k_mlp_pack<<<(kTrainable + 255) / 256, 256, 0, m->stream>>>(m->params, m->wpack);
+    BBX_HIP_CHECK(hipGetLastError());
     return BBX_OK;
 }
 
@@ -380,13 +464,10 @@ static int infer_launch(bbx_mlp *m, const float *x, int n, int fstride, int sstr
 static int grad_launch(bbx_mlp *m, const float *xs, const float *ts, int n, int batch, int random,
                        unsigned long long seed, int adam, float lr) {
     const int tiles = (batch + 15) / 16;
-    const int waves_needed = (tiles + kTilesPerWave - 1) / kTilesPerWave;
-    const int blocks = (waves_needed + kWaves - 1) / kWaves;
-    const int nwaves = blocks * kWaves;
-    BBX_CHECK(ensure_gpart(m, nwaves));
-    k_mlp_grad<<<blocks, 64 * kWaves, 0, m->stream>>>(m->params, xs, ts, n, batch, random, seed,
-                                                       m->expectile,
-                                                       m->gpart, m->lpart);
+    const int parts = (tiles + kWaves - 1) / kWaves;
+    BBX_CHECK(ensure_gpart(m, parts));
+    k_mlp_grad<<<parts, 64 * kWaves, 0, m->stream>>>(m->params, (const bf16x4 *)m->wpack, xs, ts, n, batch, random,
+                                                      seed, m->expectile, m->gpart, m->lpart);
     BBX_HIP_CHECK(hipGetLastError());
     float bc1 = 1.f, bc2 = 1.f;
     if (adam) {
@@ -394,9 +475,8 @@ static int grad_launch(bbx_mlp *m, const float *xs, const float *ts, int n, int 
         bc1 = 1.f - powf(0.9f, (float)m->adam_t);
         bc2 = 1.f - powf(0.999f, (float)m->adam_t);
     }
-    k_mlp_reduce<<<(kTrainable + 255) / 256, 256, 0, m->stream>>>(m->gpart, m->lpart, nwaves, m->grad,
-                                                                  m->loss, m->params, m->m1, m->m2,
-                                                                  adam, lr, bc1, bc2);
+    k_mlp_reduce<<<kReduceBlocks + 1, 64, 0, m->stream>>>(m->gpart, m->lpart, parts, m->grad, m->loss, m->params,
+                                                          m->wpack, m->m1, m->m2, adam, lr, bc1, bc2);
     BBX_HIP_CHECK(hipGetLastError());
     return BBX_OK;
 }
@@ -453,6 +533,7 @@ int bbx_mlp_create(int seed, bbx_mlp **out) {
     p[OFF_RESID] = 0.f;
     hipError_t e = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc((void **)&m->params, sizeof(float) * kParams);
+    if (e == hipSuccess) e = hipMalloc((void **)&m->wpack, sizeof(unsigned short) * kPackEntries);
     if (e == hipSuccess) e = hipMalloc((void **)&m->m1, sizeof(float) * kTrainable);
     if (e == hipSuccess) e = hipMalloc((void **)&m->m2, sizeof(float) * kTrainable);
     if (e == hipSuccess) e = hipMalloc((void **)&m->grad, sizeof(float) * kTrainable);
@@ -474,6 +555,7 @@ static void mlp_free(bbx_mlp *m) {
                      m->data_x, m->data_t, m->tmp_x, m->tmp_y};
     for (float *b : bufs)
         if (b) (void)hipFree(b);
+    if (m->wpack) (void)hipFree(m->wpack);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
 }
@@ -530,6 +612,7 @@ static int upload_batch(bbx_mlp *m, const float *x, const float *t, int n) {
 int bbx_mlp_gradients(bbx_mlp *m, const float *x, const float *t, int n, float *grad, float *loss) {
     if (!m || n <= 0 || !x || !t || !grad) return fail(BBX_E_INVALID, "bad arguments");
     BBX_CHECK(upload_batch(m, x, t, n));
+    BBX_CHECK(pack_launch(m));
     BBX_CHECK(grad_launch(m, m->tmp_x, m->tmp_y, n, n, 0, 0, 0, 0.f));
     std::vector<float> g(kTrainable);
     BBX_HIP_CHECK(hipMemcpyAsync(g.data(), m->grad, sizeof(float) * kTrainable, hipMemcpyDeviceToHost, m->stream));
@@ -544,6 +627,7 @@ int bbx_mlp_gradients(bbx_mlp *m, const float *x, const float *t, int n, float *
 int bbx_mlp_train_step(bbx_mlp *m, const float *x, const float *t, int n, float lr, float *loss) {
     if (!m || n <= 0 || !x || !t) return fail(BBX_E_INVALID, "bad arguments");
     BBX_CHECK(upload_batch(m, x, t, n));
+    BBX_CHECK(pack_launch(m));
     BBX_CHECK(grad_launch(m, m->tmp_x, m->tmp_y, n, n, 0, 0, 1, lr));
     float l = 0.f;
     BBX_HIP_CHECK(hipMemcpyAsync(&l, m->loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
@@ -555,14 +639,18 @@ int bbx_mlp_train_step(bbx_mlp *m, const float *x, const float *t, int n, float 
 int bbx_mlp_train(bbx_mlp *m, const float *x, const float *t, int n, int steps, int batch, float lr,
                   int seed, float *final_loss) {
     if (!m || n <= 0 || !x || !t || steps < 0 || batch <= 0) return fail(BBX_E_INVALID, "bad arguments");
-    if (m->data_x) (void)hipFree(m->data_x);
-    if (m->data_t) (void)hipFree(m->data_t);
-    m->data_x = m->data_t = nullptr;
-    BBX_HIP_CHECK(hipMalloc((void **)&m->data_x, sizeof(float) * (size_t)n * kF));
-    BBX_HIP_CHECK(hipMalloc((void **)&m->data_t, sizeof(float) * (size_t)n));
+    if (n > m->data_n) {
+        if (m->data_x) (void)hipFree(m->data_x);
+        if (m->data_t) (void)hipFree(m->data_t);
+        m->data_x = m->data_t = nullptr;
+        m->data_n = 0;
+        BBX_HIP_CHECK(hipMalloc((void **)&m->data_x, sizeof(float) * (size_t)n * kF));
+        BBX_HIP_CHECK(hipMalloc((void **)&m->data_t, sizeof(float) * (size_t)n));
+        m->data_n = n;
+    }
     BBX_HIP_CHECK(hipMemcpy(m->data_x, x, sizeof(float) * (size_t)n * kF, hipMemcpyHostToDevice));
     BBX_HIP_CHECK(hipMemcpy(m->data_t, t, sizeof(float) * (size_t)n, hipMemcpyHostToDevice));
-    m->data_n = n;
+    if (steps > 0) BBX_CHECK(pack_launch(m));
     for (int s = 0; s < steps; s++) {
         unsigned long long sd = ((unsigned long long)(unsigned)seed << 32) ^ (unsigned long long)s * 0x2545F4914F6CDD1Dull;
         BBX_CHECK(grad_launch(m, m->data_x, m->data_t, n, batch, 1, sd, 1, lr));
