@@ -20,7 +20,7 @@ BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libbubbles_amd.so")
 
 SOURCES = ["bbx_abi.hip", "bbx_grid.hip", "bbx_sph.hip", "bbx_mlp.hip", "bbx_stream.hip", "bbx_io.hip",
-           "bbx_shapes.hip"]
+           "bbx_shapes.hip", "bbx_fetch.hip"]
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "bbx_common.h"
+#include "bbx_fetch.h"
 
 namespace bbx {
 
@@ -397,9 +398,7 @@ static void free_all(bbx_solver *s) {
     s->loop = nullptr; s->max_force = nullptr; s->counters = nullptr;
     dfree(s->coll);
     s->ncoll = 0;
-    if (s->h_step) (void)hipHostFree(s->h_step);
-    if (s->h_flag) (void)hipHostFree(s->h_flag);
-    if (s->h_signal) (void)hipHostFree(s->h_signal);
+    if (s->h_signal) (void)hipHostFree(s->h_signal);  // the pinned block
     s->h_step = nullptr; s->h_flag = nullptr;
     s->h_signal = nullptr; s->d_signal = nullptr;
     s->h_loop = nullptr; s->h_counters = nullptr; s->h_max_force = nullptr;
@@ -413,6 +412,7 @@ static void free_all(bbx_solver *s) {
         if (s->mark[k]) (void)hipEventDestroy(s->mark[k]);
         s->mark[k] = nullptr;
     }
+    fetch_free(s);
     s->prof.destroy();
     if (s->stream) (void)hipStreamDestroy(s->stream);
     s->stream = nullptr;
@@ -550,22 +550,28 @@ int bbx_solver_create(int kind, const bbx_params *params, const double *pos, con
         s->counters = s->step->counters;
     }
     if (!rc) rc = dalloc(&s->flag, 1);
-    if (!rc && hipHostMalloc((void **)&s->h_step, sizeof(StepBlock)) != hipSuccess)
-        rc = fail(BBX_E_NOMEM, "pinned alloc");
-    if (!rc && hipHostMalloc((void **)&s->h_flag, sizeof(int)) != hipSuccess)
-        rc = fail(BBX_E_NOMEM, "pinned alloc");
-    if (!rc && hipHostMalloc((void **)&s->h_signal, sizeof(LoopSignal), hipHostMallocMapped | hipHostMallocCoherent) !=
+    // one pinned block (an allocation costs about 100 us): the loop signal,
+    // the step block's copy, a flag, and the ring of the field downloads
+    const size_t pin_step = 256, pin_flag = pin_step + (sizeof(StepBlock) + 255) / 256 * 256, pin_ring = pin_flag + 256;
+    static_assert(sizeof(LoopSignal) <= 256, "pinned block layout");
+    char *pin = nullptr, *d_pin = nullptr;
+    if (!rc && hipHostMalloc((void **)&pin, pin_ring + fetch_ring_bytes(N) + 64, hipHostMallocMapped | hipHostMallocCoherent) !=
                    hipSuccess)
         rc = fail(BBX_E_NOMEM, "pinned alloc");
     if (!rc) {
+        s->h_signal = (LoopSignal *)pin;  // the block's address: free_all frees it
+        s->h_step = (StepBlock *)(pin + pin_step);
+        s->h_flag = (int *)(pin + pin_flag);
         std::memset(s->h_signal, 0, sizeof(LoopSignal));
-        if (hipHostGetDevicePointer((void **)&s->d_signal, s->h_signal, 0) != hipSuccess)
+        if (hipHostGetDevicePointer((void **)&d_pin, pin, 0) != hipSuccess)
             rc = fail(BBX_E_HIP, "device address of the loop signal");
+        s->d_signal = (LoopSignal *)d_pin;
         // BBX_LOOP_SIGNAL=0: no published decisions; the host reads every
         // decision back through a copy (the fallback path, for tests)
         if (const char *e = std::getenv("BBX_LOOP_SIGNAL"))
             if (std::atoi(e) == 0) s->d_signal = nullptr;
     }
+    if (!rc) rc = fetch_init(s, pin + pin_ring, d_pin + pin_ring, fetch_ring_bytes(N));
     if (!rc) {
         s->h_loop = &s->h_step->loop;
         s->h_max_force = s->h_step->max_force;
@@ -600,33 +606,21 @@ int bbx_solver_create(int kind, const bbx_params *params, const double *pos, con
     }
     hipError_t e = hipMemcpy(s->posA, hp.data(), sizeof(float4) * N, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(s->velA, hv.data(), sizeof(float4) * N, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemset(s->force, 0, sizeof(float4) * N);
-    if (e == hipSuccess) e = hipMemset(s->fp, 0, sizeof(float4) * N);
-    if (e == hipSuccess) e = hipMemset(s->xstar, 0, sizeof(float4) * N);
-    if (e == hipSuccess) e = hipMemset(s->rho, 0, sizeof(float) * N);
-    if (e == hipSuccess) e = hipMemset(s->pres, 0, sizeof(float) * N);
-    if (e == hipSuccess) e = hipMemset(s->rho_star, 0, sizeof(float) * N);
-    if (e == hipSuccess) e = hipMemset(s->xq, 0, sizeof(float4) * N);
-    if (e == hipSuccess) e = hipMemset(s->nbr_cnt, 0, sizeof(int) * N);
-    if (e == hipSuccess) e = hipMemset(s->tile_tab, 0, sizeof(int) * (size_t)s->ntiles * kTabIntsHost);
-    if (e == hipSuccess) e = hipMemset(s->feat, 0, sizeof(float) * N * BBX_NFEAT);
-    if (e == hipSuccess) e = hipMemset(s->max_force, 0, sizeof(unsigned) * kSlots);
-    if (e == hipSuccess) e = hipMemset(s->loop, 0, sizeof(LoopState));
+    if (e == hipSuccess) e = hipMemset(s->step, 0, sizeof(StepBlock));
     if (e == hipSuccess) e = hipMemset(s->flag, 0, sizeof(int));
-    if (e == hipSuccess) e = hipMemset(s->counters, 0, sizeof(int) * CNT_N);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // before work on the solver's stream
     if (e != hipSuccess) {
         free_all(s);
         delete s;
         return fail(BBX_E_HIP, std::string("upload: ") + hipGetErrorString(e));
     }
-    // every slot starts in no chain until Setup distributes
-    std::vector<int> none(N, (int)s->grid.total);
-    e = hipMemcpy(s->cellA, none.data(), sizeof(int) * N, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(s->home, none.data(), sizeof(int) * N, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
+    // fields at zero, and every slot in no chain until Setup distributes
+    rc = launch_init_fields(s);
+    if (rc == BBX_OK && hipStreamSynchronize(s->stream) != hipSuccess) rc = fail(BBX_E_HIP, "field initialisation");
+    if (rc) {
         free_all(s);
         delete s;
-        return fail(BBX_E_HIP, std::string("upload: ") + hipGetErrorString(e));
+        return rc;
     }
     fill_sim_const(s);
     *out = s;
@@ -674,49 +668,55 @@ int bbx_solver_info(bbx_solver *s, bbx_info *out) {
     return BBX_OK;
 }
 
+}  // extern "C"
+namespace {
+// what a fetch does with a range of the id-ordered field
+struct Widen final : FetchTake {
+    double *out;
+    explicit Widen(double *o) : out(o) {}
+    void run(const float *p, size_t first, size_t count) const override {
+        double *o = out + first;
+        for (size_t k = 0; k < count; k++) o[k] = p[k];
+    }
+};
+struct Keep final : FetchTake {
+    float *out;
+    explicit Keep(float *o) : out(o) {}
+    void run(const float *p, size_t first, size_t count) const override {
+        std::memcpy(out + first, p, sizeof(float) * count);
+    }
+};
+struct Ratio final : FetchTake {  // value / ref, 0 for a zero ref
+    float *out;
+    double ref;
+    Ratio(float *o, double r) : out(o), ref(r) {}
+    void run(const float *p, size_t first, size_t count) const override {
+        for (size_t k = 0; k < count; k++) out[first + k] = ref != 0 ? (float)(p[k] / ref) : 0.f;
+    }
+};
+}  // namespace
+extern "C" {
+
 int bbx_solver_download(bbx_solver *s, int field, double *out) {
     BBX_CHECK(check_solver(s));
     if (!out) return fail(BBX_E_INVALID, "null output");
     if (s->n == 0) return BBX_OK;
-    std::vector<int> ids;
-    BBX_CHECK(slot_ids(s, ids));
-    const size_t n = (size_t)s->n;
-    auto vec4 = [&](const float4 *src) -> int {
-        std::vector<float4> h(n);
-        BBX_HIP_CHECK(hipMemcpy(h.data(), src, sizeof(float4) * n, hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < n; i++) {
-            double *o = &out[3 * (size_t)ids[i]];
-            o[0] = h[i].x; o[1] = h[i].y; o[2] = h[i].z;
-        }
-        return BBX_OK;
-    };
-    auto scal = [&](const float *src) -> int {
-        std::vector<float> h(n);
-        BBX_HIP_CHECK(hipMemcpy(h.data(), src, sizeof(float) * n, hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < n; i++) out[ids[i]] = h[i];
-        return BBX_OK;
-    };
+    FieldSource f{1, nullptr, nullptr};
+    auto vec = [&](const float4 *v) { f = FieldSource{3, v, nullptr}; };
     switch (field) {
-        case BBX_FIELD_POSITION: return vec4(s->posA);
-        case BBX_FIELD_VELOCITY: return vec4(s->velA);
-        case BBX_FIELD_FORCE: return vec4(s->force);
-        case BBX_FIELD_PRESSURE_FORCE: return vec4(s->fp);
-        case BBX_FIELD_TEMP_POSITION: return vec4(s->xstar);
-        case BBX_FIELD_DENSITY: return scal(s->rho);
-        case BBX_FIELD_PRESSURE: return scal(s->pres);
-        case BBX_FIELD_DENSITY_PREDICTED: return scal(s->rho_star);
-        case BBX_FIELD_WARM_PRESSURE: return scal(s->pwarm);
-        case BBX_FIELD_FEATURES: {
-            std::vector<float> h(n * BBX_NFEAT);
-            for (int f = 0; f < BBX_NFEAT; f++)
-                BBX_HIP_CHECK(hipMemcpy(&h[f * n], s->feat + (size_t)f * s->stride, sizeof(float) * n,
-                                        hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < n; i++)
-                for (int f = 0; f < BBX_NFEAT; f++) out[(size_t)ids[i] * BBX_NFEAT + f] = h[f * n + i];
-            return BBX_OK;
-        }
+        case BBX_FIELD_POSITION: vec(s->posA); break;
+        case BBX_FIELD_VELOCITY: vec(s->velA); break;
+        case BBX_FIELD_FORCE: vec(s->force); break;
+        case BBX_FIELD_PRESSURE_FORCE: vec(s->fp); break;
+        case BBX_FIELD_TEMP_POSITION: vec(s->xstar); break;
+        case BBX_FIELD_DENSITY: f.scal = s->rho; break;
+        case BBX_FIELD_PRESSURE: f.scal = s->pres; break;
+        case BBX_FIELD_DENSITY_PREDICTED: f.scal = s->rho_star; break;
+        case BBX_FIELD_WARM_PRESSURE: f.scal = s->pwarm; break;
+        case BBX_FIELD_FEATURES: f = FieldSource{BBX_NFEAT, nullptr, s->feat}; break;
         default: return fail(BBX_E_INVALID, "unknown field");
     }
+    return fetch_by_id(s, f, Widen(out));
 }
 
 // ---------------------------------------------------------------------------
@@ -797,7 +797,7 @@ int bbx_solver_reserve(bbx_solver *s, int capacity) {
     BBX_HIP_CHECK(hipMemcpy(s->home + n, none.data(), sizeof(int) * none.size(), hipMemcpyHostToDevice));
     s->stride = (int)S1;
     fill_sim_const(s);
-    return BBX_OK;
+    return fetch_grow(s, S1);
 }
 
 int bbx_solver_capacity(bbx_solver *s, int *capacity) {
@@ -1588,7 +1588,6 @@ int bbx_pcisph_harvest(bbx_solver *s, double dt, int max_it, double tol, float *
                        float *targets, bbx_stats *stats) {
     BBX_CHECK(check_setup(s));
     if (!features || !targets) return fail(BBX_E_INVALID, "null output");
-    const size_t n = (size_t)s->n;
     // features at the start of the substep: distribute + density + non-pressure
     // with feature output, then the plain substep from the same state.
     // The features are computed on a throwaway pass that leaves the state
@@ -1600,22 +1599,11 @@ int bbx_pcisph_harvest(bbx_solver *s, double dt, int max_it, double tol, float *
     st.dt_over_m = (float)(dt / s->mass);
     st.delta = (float)delta;
     BBX_CHECK(distribute(s, false, true, false, -1, 1, &st));
-    std::vector<int> ids;
-    BBX_CHECK(slot_ids(s, ids));
-    std::vector<float> h(n * BBX_NFEAT);
-    for (int f = 0; f < BBX_NFEAT; f++)
-        BBX_HIP_CHECK(hipMemcpy(&h[f * n], s->feat + (size_t)f * s->stride, sizeof(float) * n,
-                                hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < n; i++)
-        for (int f = 0; f < BBX_NFEAT; f++) features[(size_t)ids[i] * BBX_NFEAT + f] = h[f * n + i];
+    BBX_CHECK(fetch_by_id(s, FieldSource{BBX_NFEAT, nullptr, s->feat}, Keep(features)));
     bbx_stats local{};
     BBX_CHECK(bbx_pcisph_substep(s, dt, max_it, tol, BBX_MODE_TEXTBOOK, BBX_WARM_NONE, &local));
-    // converged pressure / (delta rho0), by id (slots moved only inside the substep's distribute)
-    BBX_CHECK(slot_ids(s, ids));
-    std::vector<float> p(n);
-    BBX_HIP_CHECK(hipMemcpy(p.data(), s->pres, sizeof(float) * n, hipMemcpyDeviceToHost));
-    const double pref = delta * s->prm.target_density;
-    for (size_t i = 0; i < n; i++) targets[ids[i]] = pref != 0 ? (float)(p[i] / pref) : 0.f;
+    // converged pressure / (delta rho0), by id
+    BBX_CHECK(fetch_by_id(s, FieldSource{1, nullptr, s->pres}, Ratio(targets, delta * s->prm.target_density)));
     if (stats) *stats = local;
     return BBX_OK;
 }

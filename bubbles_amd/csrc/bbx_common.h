@@ -216,6 +216,9 @@ struct Profiler {
 // solver
 // ---------------------------------------------------------------------------
 struct bbx_mlp;
+namespace bbx {
+struct FetchRing;
+}
 
 struct bbx_solver {
     int kind = BBX_PCISPH;
@@ -291,7 +294,7 @@ struct bbx_solver {
     // kMarks - 1 substeps later, so the host never waits for a substep's end
     static constexpr int kMarks = 8;
     hipEvent_t mark[kMarks] = {};
-
+    bbx::FetchRing *fetch = nullptr;  // pinned ring of the field downloads
 
     bbx_mlp *mlp = nullptr;
     bbx::Profiler prof;
@@ -309,6 +312,7 @@ int compute_mass_and_delta(bbx_solver *s);
 void fill_sim_const(bbx_solver *s);
 
 int launch_fill_int(bbx_solver *s, int *p, int value, size_t n);
+int launch_init_fields(bbx_solver *s);
 int launch_scan(bbx_solver *s, const int *in, int *out, size_t n);
 // append_from >= 0: the append pass after new particles were placed in
 // slots append_from..n-1 (old chains kept, new particles at their tails)
