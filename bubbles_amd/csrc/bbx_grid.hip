@@ -461,12 +461,265 @@ struct WarmIn {
     float4 *__restrict__ xq;              // (x, p0 / rho^2)
 };
 
+// Acceptance mask of the candidates of one row (bit t: candidate t; len <=
+// 64): staged at `row` in LDS (with slack slots behind) or from storage index
+// a on.  Eight at a time with no branches.  The FP32 test uses
+// t = |pi - pj|^2 - band_c (the offset folded into the first FMA): t < 0
+// accepts; a candidate with |t| <= band_w (rare) makes the lane re-test its
+// row with the reference's FP64 rule.  The sign bits of a group enter a
+// 64-bit shift register {hi, lo} at its top.
+template <bool kStaged>
+__device__ __forceinline__ unsigned long long row_mask(const SimConst &c, float4 pi, const float4 *row,
+                                                       const float4 *__restrict__ pos, int a, int len) {
+    unsigned lo = 0u, hi = 0u;
+    float bdist = 3.4e38f;
+    int t0 = 0;
+    // Two groups of four per step: the second group's loads are in flight
+    // while the first group's arithmetic runs (one step of a row reads up to
+    // seven candidates past its end: slack slots when staged, clamped
+    // otherwise; their bits are cleared below).
+    for (; t0 < len; t0 += 8) {
+        float4 pc[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            if (kStaged)
+                pc[q] = row[t0 + q];
+            else
+                pc[q] = pos[min(a + t0 + q, c.n - 1)];
+        }
+        float tq[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) tq[q] = cut_offset(pi, pc[q], c.band_c);
+#pragma unroll
+        for (int q = 0; q < 8; q += 2) bdist = fminf(fminf(bdist, fabsf(tq[q])), fabsf(tq[q + 1]));
+        unsigned byte = __float_as_uint(tq[7]) >> 31;  // bit q: candidate t0 + q
+#pragma unroll
+        for (int q = 6; q >= 0; q--) byte = __builtin_amdgcn_alignbit(byte, __float_as_uint(tq[q]), 31);
+        lo = __builtin_amdgcn_alignbit(hi, lo, 8);
+        hi = __builtin_amdgcn_alignbit(byte, hi, 8);
+    }
+    // t0 = 8 * steps; candidate t sits at bit 64 - t0 + t
+    unsigned long long m = ((unsigned long long)hi << 32) | lo;
+    m = t0 > 0 ? m >> (64 - t0) : 0ull;
+    if (len < 64) m &= (1ull << len) - 1ull;
+    if (bdist <= c.band_w) {
+        // candidates inside the band: the exact FP64 rule
+        for (int t = 0; t < len; t++) {
+            const float4 pj = kStaged ? row[t] : pos[a + t];
+            if (fabsf(cut_offset(pi, pj, c.band_c)) <= c.band_w) {
+                const unsigned long long bit = 1ull << t;
+                m = within_std_fp64(pi, pj, c.h2d) ? (m | bit) : (m & ~bit);
+            }
+        }
+    }
+    return m;
+}
+
+// ComputePressureValue (src/equations/sph_equations3.cpp:7-18)
+__device__ __forceinline__ float tait_pressure(const SimConst &c, float d) {
+    float p = c.eos_scale / c.eos_exp * (powf(d / c.rho0, c.eos_exp) - 1.f);
+    if (p < 0.f) p *= c.nps;
+    return p;
+}
+
+// A bucket as it is emitted.  The current quad of entries.  Staged: a 64-bit
+// shift register of 16-bit entries held as two words (entry k of the quad
+// ends in bits 16k..16k+15); global: four 32-bit entries.
+template <bool kStaged>
+struct BucketWriter {
+    unsigned short *__restrict__ nbr16;
+    int *__restrict__ nbr32;
+    int stride, i;
+    int cnt = 0, dropped = 0;
+    unsigned qlo = 0u, qhi = 0u;
+    int e0 = 0, e1 = 0, e2 = 0, e3 = 0;
+
+    __device__ __forceinline__ BucketWriter(unsigned short *n16, int *n32, int str, int at)
+        : nbr16(n16), nbr32(n32), stride(str), i(at) {}
+    __device__ __forceinline__ void store_quad(int nfill) {  // nfill = entries in the quad
+        const size_t at = (size_t)((cnt - 1) >> 2) * stride + i;
+        if (kStaged) {
+            unsigned long long q = ((unsigned long long)qhi << 32) | qlo;
+            q >>= 16 * (4 - nfill);  // a partial quad moves down to slot 0
+            reinterpret_cast<uint2 *>(nbr16)[at] = make_uint2((unsigned)q, (unsigned)(q >> 32));
+        } else {
+            int4 v = make_int4(e0, e1, e2, e3);
+            if (nfill == 3) v = make_int4(e1, e2, e3, 0);
+            else if (nfill == 2) v = make_int4(e2, e3, 0, 0);
+            else if (nfill == 1) v = make_int4(e3, 0, 0, 0);
+            reinterpret_cast<int4 *>(nbr32)[at] = v;
+        }
+    }
+    // append accepted candidate j (storage index; LDS index j + sh) to the
+    // bucket (emit: up to the cap).  Only the index is handled here: the
+    // emission loops run as long as the wave's longest cell, so the density
+    // sum runs afterwards over the finished bucket, one uniform pass.
+    __device__ __forceinline__ void append(int j, int sh) {
+        if (kStaged) {  // the entry is the candidate's LDS byte offset
+            qlo = __builtin_amdgcn_alignbit(qhi, qlo, 16);
+            qhi = __builtin_amdgcn_alignbit((unsigned)(j + sh) << kSlotShift, qhi, 16);
+        } else {
+            e0 = e1;
+            e1 = e2;
+            e2 = e3;
+            e3 = j;
+        }
+        cnt++;
+        if ((cnt & 3) == 0) store_quad(4);
+    }
+    __device__ __forceinline__ void emit(int j, int sh) {
+        if (cnt >= kBucket)
+            dropped++;
+        else
+            append(j, sh);
+    }
+    __device__ __forceinline__ void finish() {
+        if (cnt & 3) store_quad(cnt & 3);
+    }
+};
+
+// The bucket cell by cell, in the reference's order and with its cap.
+// sh[r]: LDS index - storage index of row r (zero when not staged).
+template <bool kStaged>
+__device__ __forceinline__ void walk_cells(const SimConst &c, float4 pi, const int (&u)[3],
+                                           const int *__restrict__ start, const float4 *sx,
+                                           const float4 *__restrict__ pos, const int *sh, BucketWriter<kStaged> &bw) {
+    const int nx = c.g.n[0], ny = c.g.n[1], nz = c.g.n[2];
+    for (int dy = 0; dy < 3; dy++)
+        for (int dx = 0; dx < 3; dx++) {
+            const int x = u[0] + dx - 1;
+            if (x < 0 || x >= nx) continue;
+            for (int dz = 0; dz < 3; dz++) {
+                const int yy = u[1] + dy - 1, zz = u[2] + dz - 1;
+                if (yy < 0 || yy >= ny || zz < 0 || zz >= nz) continue;
+                const int cell = x + yy * nx + zz * nx * ny;
+                const int sr = sh[dz * 3 + dy];
+                const int e = start[cell + 1];
+                for (int j = start[cell]; j < e; j++) {
+                    const float4 pj = kStaged ? sx[j + sr] : pos[j];
+                    if (in_bucket(c, pi, pj)) bw.emit(j, sr);
+                }
+            }
+        }
+}
+
+// The features of particle i from its bucket's sums.
+__device__ __forceinline__ void finish_features(const SimConst &c, const WarmIn &wi, int i, float4 pi, float di,
+                                                int cnt, float m1, float m2, float m3, float cx, float cy, float cz,
+                                                float *fv) {
+    const float4 vi = wi.vel[i];
+    const float inv = 1.f / (cnt > 1 ? (float)(cnt - 1) : 1.f);
+    float wall = 3.4e38f;
+    const float p3[3] = {pi.x, pi.y, pi.z};
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const float lo = p3[a] - (c.tank_c[a] - c.tank_h[a]);
+        const float hi = (c.tank_c[a] + c.tank_h[a]) - p3[a];
+        wall = fminf(wall, fminf(lo, hi));
+    }
+    const float vs = wi.st.dt * c.inv_h;
+    const float s1 = c.inv_h * inv, s2 = s1 * c.inv_h, s3 = s2 * c.inv_h;
+    cx *= c.inv_h;
+    cy *= c.inv_h;
+    cz *= c.inv_h;
+    fv[BBX_F_DENSITY_ERR] = di / c.rho0 - 1.f;
+    fv[BBX_F_RESERVED1] = 0.f;
+    fv[BBX_F_COUNT] = (float)cnt;
+    fv[BBX_F_M1] = m1 * s1;
+    fv[BBX_F_M2] = m2 * s2;
+    fv[BBX_F_M3] = m3 * s3;
+    fv[BBX_F_CX] = cx * inv;
+    fv[BBX_F_CY] = cy * inv;
+    fv[BBX_F_CZ] = cz * inv;
+    fv[BBX_F_CNORM] = sqrtf(cx * cx + cy * cy + cz * cz) * inv;
+    fv[BBX_F_PPREV] = wi.st.delta != 0.f ? vi.w / (wi.st.delta * c.rho0) : 0.f;
+    fv[BBX_F_VY] = vi.y * vs;
+    fv[BBX_F_VNORM] = sqrtf(vi.x * vi.x + vi.y * vi.y + vi.z * vi.z) * vs;
+    fv[BBX_F_RESERVED2] = 0.f;
+    fv[BBX_F_RESERVED3] = 0.f;
+    fv[BBX_F_WALL] = fminf(fmaxf(wall * c.inv_h, 0.f), 4.f);
+}
+
+// Network pressures of a workgroup's kRows particles (thread t < kRows holds
+// particle t's features): the feature rows go through LDS (over the staged
+// candidates, which every thread has finished with) into the MFMA layout;
+// the waves share the rows in 16-sample tiles.
+// Returns the kRows pressures in LDS; the whole workgroup calls.
+template <int kRows>
+__device__ __forceinline__ const float *infer_block(const WarmIn &wi, float4 *sx, int row, bool valid,
+                                                    const float *fv) {
+    constexpr int kRow = BBX_NFEAT + 1;  // padded feature row
+    constexpr int kTiles = kRows * 4 / kBlock;  // 16-sample tiles per wave
+    constexpr int kT = kTiles > 1 ? 2 : 1;
+    float *lf = reinterpret_cast<float *>(sx);  // feature rows
+    float *lp = lf + kRows * kRow;              // warm-start pressures
+    float *lb = lp + kRows;                     // b1 | b2 | w3
+    unsigned short *lw = reinterpret_cast<unsigned short *>(lb + 3 * kH);  // BF16 weights of both layers
+    static_assert((kRows * (kRow + 1) + 3 * kH) * 4 + kLdsWeights * 2 <= (int)sizeof(float4) * kTileCap &&
+                      (kRows * (kRow + 1) + 3 * kH) % 4 == 0,
+                  "warm-start LDS layout over the staged candidates");
+    __syncthreads();
+    if (row >= 0) {
+#pragma unroll
+        for (int f = 0; f < BBX_NFEAT; f++) lf[row * kRow + f] = valid ? fv[f] : 0.f;
+    }
+    stage_infer_weights(wi.P, lw, lb, (int)threadIdx.x, kBlock);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int qq = lane >> 4, jj = lane & 15;
+    bf16x4 w1[4], w2[4][4];
+    load_weight_operands_lds(lw, lane, w1, w2);
+    float mean[4], istd[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        mean[v] = wi.P[OFF_MEAN + 4 * qq + v];
+        istd[v] = wi.P[OFF_ISTD + 4 * qq + v];
+    }
+    const float b3 = wi.P[OFF_B3], oscale = wi.P[OFF_OSCALE], alpha = wi.P[OFF_ALPHA];
+    const float pcap = wi.P[OFF_PCAP], resid = wi.P[OFF_RESID];
+#pragma unroll
+    for (int part = 0; part < kTiles / kT; part++) {  // pairs of tiles keep the registers below 128
+        float xv[kT][4];
+#pragma unroll
+        for (int t = 0; t < kT; t++) {
+            const int smp = (wv * kTiles + kT * part + t) * 16 + jj;
+#pragma unroll
+            for (int v = 0; v < 4; v++) xv[t][v] = lf[smp * kRow + 4 * qq + v];
+        }
+        float yn[kT];
+        forward_infer_tiles<kT>(w1, w2, lb, lb + kH, lb + 2 * kH, b3, xv, mean, istd, qq, yn);
+        if (lane < 16) {
+#pragma unroll
+            for (int t = 0; t < kT; t++) {
+                const int smp = (wv * kTiles + kT * part + t) * 16 + jj;
+                // the same expression as the standalone inference kernel
+                float y = yn[t] * oscale;
+                if (resid != 0.f) y += resid * lf[smp * kRow + BBX_F_PPREV];
+                y = alpha * fminf(fmaxf(y, 0.f), pcap);
+                lp[smp] = y * wi.st.warm_scale;
+            }
+        }
+    }
+    __syncthreads();
+    return lp;
+}
+
+// PredictVelocityAndPositionFor at k = 0 (src/equations/pcisph_equations3.cpp:3-28)
+// with the network's pressure p instead of 0: rho* = rho, p = p0
+__device__ __forceinline__ void warm_start_one(const WarmIn &wi, int i, float4 pi, float di, float p,
+                                               float *__restrict__ pres) {
+    const float d2 = di * di;
+    pres[i] = p;
+    wi.pwarm[i] = p;
+    wi.rho_star[i] = di;
+    wi.xq[i] = make_float4(pi.x, pi.y, pi.z, (fabsf(d2) < 1e-8f) ? 0.f : p / d2);
+}
+
 template <bool kPressure, int kFeat>
 __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
                                                             const float4 *__restrict__ pos,
                                                             const int *__restrict__ home,
                                                             const int *__restrict__ start,
-                                                            const int *__restrict__ count,
                                                             unsigned short *__restrict__ nbr16,
                                                             int *__restrict__ nbr32,
                                                             int *__restrict__ nbr_cnt,
@@ -555,112 +808,22 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
     // (that would compile to a slower generic load).
     auto per_particle = [&](auto staged_tag) {
         constexpr bool kStaged = decltype(staged_tag)::value;
-        int cnt = 0, dropped = 0;
         float sum = 0.f, comp = 0.f;
         float m1 = 0.f, m2 = 0.f, m3 = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;  // features
-        // The current quad of bucket entries.  Staged: a 64-bit shift
-        // register of 16-bit entries held as two words (entry k of the quad
-        // ends in bits 16k..16k+15); global: four 32-bit entries.
-        unsigned qlo = 0u, qhi = 0u;
-        int e0 = 0, e1 = 0, e2 = 0, e3 = 0;
-        auto store_quad = [&](int k, int nfill) {  // k = entries so far, nfill = entries in the quad
-            const size_t at = (size_t)((k - 1) >> 2) * c.stride + i;
-            if (kStaged) {
-                unsigned long long q = ((unsigned long long)qhi << 32) | qlo;
-                q >>= 16 * (4 - nfill);  // a partial quad moves down to slot 0
-                reinterpret_cast<uint2 *>(nbr16)[at] = make_uint2((unsigned)q, (unsigned)(q >> 32));
-            } else {
-                int4 v = make_int4(e0, e1, e2, e3);
-                if (nfill == 3) v = make_int4(e1, e2, e3, 0);
-                else if (nfill == 2) v = make_int4(e2, e3, 0, 0);
-                else if (nfill == 1) v = make_int4(e3, 0, 0, 0);
-                reinterpret_cast<int4 *>(nbr32)[at] = v;
-            }
-        };
-        // append accepted candidate j (storage index; LDS index j + sh) to the
-        // bucket (emit: up to the cap).  Only the index is handled here: the
-        // emission loops run as long as the wave's longest cell, so the
-        // density sum runs afterwards over the finished bucket, one uniform
-        // pass.
-        auto append = [&](int j, int sh) {
-            if (kStaged) {  // the entry is the candidate's LDS byte offset
-                qlo = __builtin_amdgcn_alignbit(qhi, qlo, 16);
-                qhi = __builtin_amdgcn_alignbit((unsigned)(j + sh) << kSlotShift, qhi, 16);
-            } else {
-                e0 = e1;
-                e1 = e2;
-                e2 = e3;
-                e3 = j;
-            }
-            cnt++;
-            if ((cnt & 3) == 0) store_quad(cnt, 4);
-        };
-        auto emit = [&](int j, int sh) {
-            if (cnt >= kBucket)
-                dropped++;
-            else
-                append(j, sh);
-        };
+        BucketWriter<kStaged> bw{nbr16, nbr32, c.stride, i};
         if (hc >= 0) {
             int sh[9];
 #pragma unroll
             for (int r = 0; r < 9; r++) sh[r] = kStaged ? tt.rdelta[r] : 0;
             bool emitted = false;
             if (narrow) {
-                // Pass 1: each row's candidates, four at a time with no
-                // branches, into an acceptance mask.  The FP32 test uses
-                // t = |pi - pj|^2 - band_c (the offset folded into the first
-                // FMA): t < 0 accepts; a candidate with |t| <= band_w (rare)
-                // makes the lane re-test its row with the reference's FP64
-                // rule.  The sign bits of a group form a nibble that enters a
-                // 64-bit shift register {hi, lo} at its top.
+                // Pass 1: each row's candidates into an acceptance mask
                 unsigned long long M[9];
                 int total = 0;
 #pragma unroll
                 for (int r = 0; r < 9; r++) {
-                    const int len = (int)(O[r] >> 24);
-                    unsigned lo = 0u, hi = 0u;
-                    float bdist = 3.4e38f;
-                    int t0 = 0;
-                    // Two groups of four per step: the second group's loads
-                    // are in flight while the first group's arithmetic runs
-                    // (one step of a row reads up to seven candidates past
-                    // its end: slack slots when staged, clamped otherwise;
-                    // their bits are cleared below).
-                    for (; t0 < len; t0 += 8) {
-                        float4 pc[8];
-#pragma unroll
-                        for (int q = 0; q < 8; q++) {
-                            if (kStaged)
-                                pc[q] = sx[A[r] + sh[r] + t0 + q];
-                            else
-                                pc[q] = pos[min(A[r] + t0 + q, c.n - 1)];
-                        }
-                        float tq[8];
-#pragma unroll
-                        for (int q = 0; q < 8; q++) tq[q] = cut_offset(pi, pc[q], c.band_c);
-#pragma unroll
-                        for (int q = 0; q < 8; q += 2) bdist = fminf(fminf(bdist, fabsf(tq[q])), fabsf(tq[q + 1]));
-                        unsigned byte = __float_as_uint(tq[7]) >> 31;  // bit q: candidate t0 + q
-#pragma unroll
-                        for (int q = 6; q >= 0; q--) byte = __builtin_amdgcn_alignbit(byte, __float_as_uint(tq[q]), 31);
-                        lo = __builtin_amdgcn_alignbit(hi, lo, 8);
-                        hi = __builtin_amdgcn_alignbit(byte, hi, 8);
-                    }
-                    // t0 = 8 * steps; candidate t sits at bit 64 - t0 + t
-                    unsigned long long m = ((unsigned long long)hi << 32) | lo;
-                    m = t0 > 0 ? m >> (64 - t0) : 0ull;
-                    if (len < 64) m &= (1ull << len) - 1ull;
-                    if (bdist <= c.band_w) {
-                        // candidates inside the band: the exact FP64 rule
-                        for (int t = 0; t < len; t++) {
-                            const float4 pj = kStaged ? sx[A[r] + sh[r] + t] : pos[A[r] + t];
-                            if (fabsf(cut_offset(pi, pj, c.band_c)) <= c.band_w) {
-                                const unsigned long long bit = 1ull << t;
-                                m = within_std_fp64(pi, pj, c.h2d) ? (m | bit) : (m & ~bit);
-                            }
-                        }
-                    }
+                    const unsigned long long m =
+                        row_mask<kStaged>(c, pi, sx + A[r] + sh[r], pos, A[r], (int)(O[r] >> 24));
                     M[r] = m;
                     total += __popcll(m);
                 }
@@ -689,32 +852,16 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
                                 while (m) {
                                     const int b = __builtin_ctz(m);
                                     m &= m - 1u;
-                                    append(A[r] + lo + b, sh[r]);
+                                    bw.append(A[r] + lo + b, sh[r]);
                                 }
                             }
                 }
             }
-            if (!emitted) {
-                // a wide row, a crowded cell or a bucket over the cap: cell by cell
-                for (int dy = 0; dy < 3; dy++)
-                    for (int dx = 0; dx < 3; dx++) {
-                        const int x = u[0] + dx - 1;
-                        if (x < 0 || x >= nx) continue;
-                        for (int dz = 0; dz < 3; dz++) {
-                            const int yy = u[1] + dy - 1, zz = u[2] + dz - 1;
-                            if (yy < 0 || yy >= ny || zz < 0 || zz >= nz) continue;
-                            const int cell = x + yy * nx + zz * nxy;
-                            const int sr = sh[dz * 3 + dy];
-                            const int b = start[cell], e = b + count[cell];
-                            for (int j = b; j < e; j++) {
-                                const float4 pj = kStaged ? sx[j + sr] : pos[j];
-                                if (in_bucket(c, pi, pj)) emit(j, sr);
-                            }
-                        }
-                    }
-            }
+            // a wide row, a crowded cell or a bucket over the cap
+            if (!emitted) walk_cells<kStaged>(c, pi, u, start, sx, pos, sh, bw);
         }
-        if (cnt & 3) store_quad(cnt, cnt & 3);
+        bw.finish();
+        const int cnt = bw.cnt;
         // ComputeDensityFor over the bucket in bucket order, read back from
         // the table this lane has just written (its own quads: no other lane
         // or wave writes them, and no earlier load in this kernel cached them)
@@ -747,37 +894,7 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
         di = sum * c.mass;
         rho[i] = di;
         if constexpr (kFeat > 0) {
-            const float4 vi = wi.vel[i];
-            const float inv = 1.f / (cnt > 1 ? (float)(cnt - 1) : 1.f);
-            float wall = 3.4e38f;
-            const float p3[3] = {pi.x, pi.y, pi.z};
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                const float lo = p3[a] - (c.tank_c[a] - c.tank_h[a]);
-                const float hi = (c.tank_c[a] + c.tank_h[a]) - p3[a];
-                wall = fminf(wall, fminf(lo, hi));
-            }
-            const float vs = wi.st.dt * c.inv_h;
-            const float s1 = c.inv_h * inv, s2 = s1 * c.inv_h, s3 = s2 * c.inv_h;
-            cx *= c.inv_h;
-            cy *= c.inv_h;
-            cz *= c.inv_h;
-            fv[BBX_F_DENSITY_ERR] = di / c.rho0 - 1.f;
-            fv[BBX_F_RESERVED1] = 0.f;
-            fv[BBX_F_COUNT] = (float)cnt;
-            fv[BBX_F_M1] = m1 * s1;
-            fv[BBX_F_M2] = m2 * s2;
-            fv[BBX_F_M3] = m3 * s3;
-            fv[BBX_F_CX] = cx * inv;
-            fv[BBX_F_CY] = cy * inv;
-            fv[BBX_F_CZ] = cz * inv;
-            fv[BBX_F_CNORM] = sqrtf(cx * cx + cy * cy + cz * cz) * inv;
-            fv[BBX_F_PPREV] = wi.st.delta != 0.f ? vi.w / (wi.st.delta * c.rho0) : 0.f;
-            fv[BBX_F_VY] = vi.y * vs;
-            fv[BBX_F_VNORM] = sqrtf(vi.x * vi.x + vi.y * vi.y + vi.z * vi.z) * vs;
-            fv[BBX_F_RESERVED2] = 0.f;
-            fv[BBX_F_RESERVED3] = 0.f;
-            fv[BBX_F_WALL] = fminf(fmaxf(wall * c.inv_h, 0.f), 4.f);
+            finish_features(c, wi, i, pi, di, cnt, m1, m2, m3, cx, cy, cz, fv);
             if (kFeat == 1 || wi.store_feat) {
                 const size_t S = (size_t)c.stride;
 #pragma unroll
@@ -785,77 +902,272 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
             }
         }
         if (kPressure) {
-            // ComputePressureValue (src/equations/sph_equations3.cpp:7-18)
-            float p = c.eos_scale / c.eos_exp * (powf(di / c.rho0, c.eos_exp) - 1.f);
-            if (p < 0.f) p *= c.nps;
-            pres[i] = p;
+            pres[i] = tait_pressure(c, di);
         }
-        if (dropped) atomicAdd(&counters[CNT_OVERFLOW], dropped);
+        if (bw.dropped) atomicAdd(&counters[CNT_OVERFLOW], bw.dropped);
     };
     if (valid) with_staging(staged, per_particle);
     if constexpr (kFeat == 2) {
-        // The block's 256 feature rows go through LDS (over the staged
-        // candidates, which every thread has finished with) into the MFMA
-        // layout; each wave infers its 64 particles as four 16-sample tiles.
-        constexpr int kRow = BBX_NFEAT + 1;  // padded feature row
-        float *lf = reinterpret_cast<float *>(sx);  // 256 rows
-        float *lp = lf + kBlock * kRow;             // 256 warm-start pressures
-        float *lb = lp + kBlock;                    // b1 | b2 | w3
-        unsigned short *lw = reinterpret_cast<unsigned short *>(lb + 3 * kH);  // BF16 weights of both layers
-        static_assert((kBlock * (kRow + 1) + 3 * kH) * 4 + kLdsWeights * 2 <= (int)sizeof(float4) * kTileCap &&
-                          (kBlock * (kRow + 1) + 3 * kH) % 4 == 0,
-                      "warm-start LDS layout over the staged candidates");
-        __syncthreads();
+        const float *lp = infer_block<kBlock>(wi, sx, (int)threadIdx.x, valid, fv);
+        if (valid) warm_start_one(wi, i, pi, di, lp[threadIdx.x], pres);
+    }
+}
+
+// The same with four lanes per particle and four workgroups per tile, for
+// sets that leave the chip idle otherwise: the kernel above is one long chain
+// per lane (nine rows of tests, the emission, the sum), 26 us for 2k
+// particles however few tiles there are.  Each lane of a particle takes rows
+// lane, lane + 4, lane + 8; the lanes exchange the cells' counts, so that
+// each knows where its entries go, and emit into LDS; then each sums (and
+// writes out) every fourth quad.  A workgroup stages its tile's candidates
+// like the others, so tile tables and entries are the same.  A particle with
+// a crowded row or more neighbours than the cap is walked cell by cell by its
+// first lane.
+//
+// Measured (us, one lane per particle / four): 25.2 / 12.5 at 2k, 28.3 / 13.9
+// at 16k, 29.7 / 19.0 at 35k, 37.6 / 34.0 at 94k; 62.6 / 206 at 255k, where
+// the chip is full and the four workgroups' staging and the longer emission
+// count.
+constexpr int kSplitUpTo = 98304;
+constexpr int kSplitLanes = 4;
+constexpr int kSplitRows = kBlock / kSplitLanes;  // particles per workgroup
+constexpr int kSplitMax = kBucket;                // bucket entries held in LDS
+constexpr int kSplitStride = kSplitMax / 2 + 1;   // words per particle (odd: its lanes spread over the banks)
+
+// value of lane k of the own group of four / of the lane across the mask
+template <int k>
+__device__ __forceinline__ int quad_lane(int v) {
+    return __builtin_amdgcn_mov_dpp(v, k * 0x55, 0xf, 0xf, true);
+}
+__device__ __forceinline__ int quad_xor1(int v) { return __builtin_amdgcn_mov_dpp(v, 0xb1, 0xf, 0xf, true); }
+__device__ __forceinline__ int quad_xor2(int v) { return __builtin_amdgcn_mov_dpp(v, 0x4e, 0xf, 0xf, true); }
+__device__ __forceinline__ float quad_sum(float v) {
+    v += __int_as_float(quad_xor1(__float_as_int(v)));
+    return v + __int_as_float(quad_xor2(__float_as_int(v)));
+}
+
+template <bool kPressure, int kFeat>
+__global__ void __launch_bounds__(kBlock) k_buckets_density_split(SimConst c,
+                                                                  const float4 *__restrict__ pos,
+                                                                  const int *__restrict__ home,
+                                                                  const int *__restrict__ start,
+                                                                  unsigned short *__restrict__ nbr16,
+                                                                  int *__restrict__ nbr32,
+                                                                  int *__restrict__ nbr_cnt,
+                                                                  float *__restrict__ rho,
+                                                                  float *__restrict__ pres,
+                                                                  const int *__restrict__ tile_tab,
+                                                                  int *__restrict__ counters,
+                                                                  WarmIn wi) {
+    __shared__ float4 sx[kTileCap + 8];
+    __shared__ unsigned ent[kSplitRows][kSplitStride];  // buckets of a staged tile, two entries a word
+    __shared__ TileTab tt;
+    const int unit = tile_of_block();
+    const int tile = unit / kSplitLanes, part = unit % kSplitLanes;
+    const int tw = tab_load_wave(tile_tab + (size_t)tile * kTabInts);
+    const int pl = threadIdx.x / kSplitLanes, sub = threadIdx.x % kSplitLanes;
+    const int i = tile * kBlock + part * kSplitRows + pl;
+    const bool valid = i < c.n;
+    const int hc = valid ? home[i] : -1;
+    const int nx = c.g.n[0], ny = c.g.n[1], nz = c.g.n[2], nxy = nx * ny;
+    float4 pi = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (valid) pi = pos[i];
+    int u[3] = {0, 0, 0};
+    // slot k holds row r = sub + 4k (k < 3, r < 9): bounds as in the kernel above
+    int A[3] = {0, 0, 0};
+    unsigned O[3] = {0u, 0u, 0u};
+    int b[3][4];
+    int wide = 0;
+    if (hc >= 0) {
+        unlinear_fast(c.g, c.inv_nx, c.inv_nxy, hc, u);
+        const int last = (int)c.g.total;
 #pragma unroll
-        for (int f = 0; f < BBX_NFEAT; f++) lf[threadIdx.x * kRow + f] = valid ? fv[f] : 0.f;
-        stage_infer_weights(wi.P, lw, lb, (int)threadIdx.x, kBlock);
-        __syncthreads();
-        const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-        const int qq = lane >> 4, jj = lane & 15;
-        bf16x4 w1[4], w2[4][4];
-        load_weight_operands_lds(lw, lane, w1, w2);
-        float mean[4], istd[4];
+        for (int k = 0; k < 3; k++) {
+            const int r = sub + 4 * k;
+            const int yy = u[1] + (r % 3) - 1, zz = u[2] + (r / 3) - 1;
+            const bool in = r < 9 && yy >= 0 && yy < ny && zz >= 0 && zz < nz;
+            const int cx = in ? u[0] + yy * nx + zz * nxy : 0;
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            mean[v] = wi.P[OFF_MEAN + 4 * qq + v];
-            istd[v] = wi.P[OFF_ISTD + 4 * qq + v];
+            for (int q = 0; q < 4; q++) b[k][q] = start[min(max(cx - 1 + q, 0), last)];
         }
-        const float b3 = wi.P[OFF_B3], oscale = wi.P[OFF_OSCALE], alpha = wi.P[OFF_ALPHA];
-        const float pcap = wi.P[OFF_PCAP], resid = wi.P[OFF_RESID];
+    }
+    if (threadIdx.x < kTabWords) reinterpret_cast<int *>(&tt)[threadIdx.x] = tw;
+    const bool staged = tab_word(tw, 1) != 0;
+    if (staged) tab_stage_dma_wave(tw, [&](int j, int e) { lds_dma16(pos + j, sx + e); });
+    if (hc >= 0) {
 #pragma unroll
-        for (int half = 0; half < 2; half++) {  // two pairs of tiles keep the registers below 128
-            float xv[2][4];
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const int smp = wv * 64 + (2 * half + t) * 16 + jj;
-#pragma unroll
-                for (int v = 0; v < 4; v++) xv[t][v] = lf[smp * kRow + 4 * qq + v];
+        for (int k = 0; k < 3; k++) {
+            const int r = sub + 4 * k;
+            const int yy = u[1] + (r % 3) - 1, zz = u[2] + (r / 3) - 1;
+            if (r < 9 && yy >= 0 && yy < ny && zz >= 0 && zz < nz) {
+                const int b1 = b[k][1], b2 = b[k][2];
+                const int b0 = u[0] > 0 ? b[k][0] : b1;
+                const int b3 = u[0] + 1 < nx ? b[k][3] : b2;
+                A[k] = b0;
+                O[k] = ((unsigned)(b1 - b0) << 8) | ((unsigned)(b2 - b0) << 16) | ((unsigned)(b3 - b0) << 24);
+                wide |= b3 - b0 > c.row_max || b1 - b0 > 32 || b2 - b1 > 32 || b3 - b2 > 32;
             }
-            float yn[2];
-            forward_infer_tiles<2>(w1, w2, lb, lb + kH, lb + 2 * kH, b3, xv, mean, istd, qq, yn);
-            if (lane < 16) {
+        }
+    }
+    wide |= quad_xor1(wide);
+    wide |= quad_xor2(wide);
+    lds_dma_wait();
+    __syncthreads();
+    if (kFeat != 2 && !valid) return;  // the inference below needs the whole block at its barriers
+    float fv[kFeat ? BBX_NFEAT : 1];
+    float di = 0.f;
+    // an unstaged tile's buckets: storage indices, in the candidates' place
+    static_assert(kSplitRows * (kSplitMax + 1) * sizeof(int) <= sizeof(sx), "unstaged buckets in LDS");
+    int *const far = reinterpret_cast<int *>(sx) + pl * (kSplitMax + 1);
+    auto per_particle = [&](auto staged_tag) {
+        constexpr bool kStaged = decltype(staged_tag)::value;
+        int cnt = 0, dropped = 0;
+        bool in_lds = false;
+        if (hc >= 0 && !wide) {
+            // acceptance masks and the accepted candidates of each cell, a byte a cell
+            unsigned long long M[3];
+            int P[3];
 #pragma unroll
-                for (int t = 0; t < 2; t++) {
-                    const int smp = wv * 64 + (2 * half + t) * 16 + jj;
-                    // the same expression as the standalone inference kernel
-                    float y = yn[t] * oscale;
-                    if (resid != 0.f) y += resid * lf[smp * kRow + BBX_F_PPREV];
-                    y = alpha * fminf(fmaxf(y, 0.f), pcap);
-                    lp[smp] = y * wi.st.warm_scale;
+            for (int k = 0; k < 3; k++) {
+                const int r = sub + 4 * k;
+                M[k] = row_mask<kStaged>(c, pi, sx + A[k] + (kStaged && r < 9 ? tt.rdelta[r] : 0), pos, A[k], (int)(O[k] >> 24));
+                const int b1 = (O[k] >> 8) & 0xff, b2 = (O[k] >> 16) & 0xff;
+                // b1 <= 32 and b2 <= 64; a shift by 64 is not defined
+                const unsigned long long from2 = b2 < 64 ? M[k] >> b2 : 0ull;
+                const int c0 = __popcll(M[k] & ((1ull << b1) - 1ull)), c2 = __popcll(from2);
+                P[k] = c0 | (__popcll(M[k]) - c0 - c2) << 8 | c2 << 16;
+            }
+            // every row's counts; r = dz * 3 + dy
+            const int R[9] = {quad_lane<0>(P[0]), quad_lane<1>(P[0]), quad_lane<2>(P[0]),
+                              quad_lane<3>(P[0]), quad_lane<0>(P[1]), quad_lane<1>(P[1]),
+                              quad_lane<2>(P[1]), quad_lane<3>(P[1]), quad_lane<0>(P[2])};
+            // the bucket's order is cells (y, x, z): where each row's three
+            // cells begin, a byte a cell (read only where the total is within
+            // the cap, so that every sum fits)
+            int at[9], total = 0;
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++) {
+                const int S = R[dy] + R[3 + dy] + R[6 + dy];
+                const int X = total * 0x010101 + ((S << 8) & 0xffff00) + ((S << 16) & 0xff0000);
+                at[dy] = X;
+                at[3 + dy] = X + R[dy];
+                at[6 + dy] = X + R[dy] + R[3 + dy];
+                total += (S & 0xff) + ((S >> 8) & 0xff) + ((S >> 16) & 0xff);
+            }
+            if (total <= kSplitMax) {
+                in_lds = true;
+                cnt = total;
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    const int lo = sub & 1 ? at[min(4 * k + 1, 8)] : at[4 * k], hi = sub & 1 ? at[min(4 * k + 3, 8)] : at[min(4 * k + 2, 8)];
+                    int to = sub & 2 ? hi : lo;
+                    const int r = sub + 4 * k;
+                    const int slot0 = A[k] + (kStaged && r < 9 ? tt.rdelta[r] : 0);
+                    const int b1 = (O[k] >> 8) & 0xff, b2 = (O[k] >> 16) & 0xff;
+                    unsigned long long m = M[k];
+                    while (m) {
+                        const int t = __builtin_ctzll(m);
+                        m &= m - 1ull;
+                        const int sh = t < b1 ? 0 : (t < b2 ? 8 : 16);
+                        if (kStaged)
+                            reinterpret_cast<unsigned short *>(ent[pl])[(to >> sh) & 0xff] =
+                                (unsigned short)((slot0 + t) << kSlotShift);
+                        else
+                            far[(to >> sh) & 0xff] = slot0 + t;
+                        to += 1 << sh;
+                    }
                 }
             }
         }
-        __syncthreads();
-        if (valid) {
-            // PredictVelocityAndPositionFor at k = 0 (src/equations/pcisph_equations3.cpp:3-28)
-            // with the network's pressure instead of 0: rho* = rho, p = p0
-            const float p = lp[threadIdx.x];
-            const float d2 = di * di;
-            pres[i] = p;
-            wi.pwarm[i] = p;
-            wi.rho_star[i] = di;
-            wi.xq[i] = make_float4(pi.x, pi.y, pi.z, (fabsf(d2) < 1e-8f) ? 0.f : p / d2);
+        if (!in_lds && sub == 0) {
+            int sh[9];
+#pragma unroll
+            for (int r = 0; r < 9; r++) sh[r] = kStaged ? tt.rdelta[r] : 0;
+            BucketWriter<kStaged> bw{nbr16, nbr32, c.stride, i};
+            if (hc >= 0) walk_cells<kStaged>(c, pi, u, start, sx, pos, sh, bw);
+            bw.finish();
+            cnt = bw.cnt;
+            dropped = bw.dropped;
         }
+        cnt = quad_lane<0>(cnt);
+        // the wave's entries are in LDS, its stores in the cache below
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_s_waitcnt(0);
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        // density (and features) over quads sub, sub + 4, ... of the bucket;
+        // dead entries read the particle itself, as in the kernel above
+        float sum = 0.f, comp = 0.f;
+        float m1 = 0.f, m2 = 0.f, m3 = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
+        const int self = kStaged ? (i + tt.rdelta[4]) << kSlotShift : i;
+        for (int q = sub; 4 * q < cnt; q += kSplitLanes) {
+            const int rem = cnt - 4 * q;
+            int4 e;
+            if (in_lds) {  // unused slots of the last quad are zero in the table
+                if (kStaged) {
+                    unsigned w0 = ent[pl][2 * q], w1 = ent[pl][2 * q + 1];
+                    w0 = rem > 1 ? w0 : w0 & 0xffffu;
+                    w1 = rem > 3 ? w1 : (rem > 2 ? w1 & 0xffffu : 0u);
+                    reinterpret_cast<uint2 *>(nbr16)[(size_t)q * c.stride + i] = make_uint2(w0, w1);
+                    e = quad_unpack(make_int4((int)w0, (int)w1, 0, 0), true);
+                } else {
+                    const int *f = far + 4 * q;
+                    e = make_int4(f[0], rem > 1 ? f[1] : 0, rem > 2 ? f[2] : 0, rem > 3 ? f[3] : 0);
+                    reinterpret_cast<int4 *>(nbr32)[(size_t)q * c.stride + i] = e;
+                }
+            } else {
+                e = quad_unpack(nbr_quad(nbr16, nbr32, kStaged, i, c.stride, q), kStaged);
+            }
+            const int j4[4] = {e.x, rem > 1 ? e.y : self, rem > 2 ? e.z : self, rem > 3 ? e.w : self};
+            float4 pj[4];
+#pragma unroll
+            for (int v = 0; v < 4; v++) pj[v] = kStaged ? lds_at(sx, j4[v]) : pos[j4[v]];
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float dx = pi.x - pj[v].x, dy = pi.y - pj[v].y, dz = pi.z - pj[v].z;
+                const float d2 = dx * dx + dy * dy + dz * dz;
+                const float w = poly6_w_member(c, d2);
+                kahan_add(sum, comp, v < rem ? w : 0.f);  // a dead entry adds an exact zero
+                if constexpr (kFeat > 0) {
+                    const float r = fast_sqrt(d2);
+                    m1 += r;
+                    m2 += d2;
+                    m3 = fmaf(r, d2, m3);
+                    cx -= dx;
+                    cy -= dy;
+                    cz -= dz;
+                }
+            }
+        }
+        // the lanes' compensated partial sums
+        di = quad_sum(sum - comp) * c.mass;
+        if constexpr (kFeat > 0) {
+            m1 = quad_sum(m1);
+            m2 = quad_sum(m2);
+            m3 = quad_sum(m3);
+            cx = quad_sum(cx);
+            cy = quad_sum(cy);
+            cz = quad_sum(cz);
+        }
+        if (sub == 0) {
+            nbr_cnt[i] = cnt;
+            rho[i] = di;
+            if constexpr (kFeat > 0) {
+                finish_features(c, wi, i, pi, di, cnt, m1, m2, m3, cx, cy, cz, fv);
+                if (kFeat == 1 || wi.store_feat) {
+                    const size_t S = (size_t)c.stride;
+#pragma unroll
+                    for (int f = 0; f < BBX_NFEAT; f++) wi.feat[(size_t)f * S + i] = fv[f];
+                }
+            }
+            if (kPressure) pres[i] = tait_pressure(c, di);
+            if (dropped) atomicAdd(&counters[CNT_OVERFLOW], dropped);
+        }
+    };
+    if (valid) with_staging(staged, per_particle);
+    if constexpr (kFeat == 2) {
+        const float *lp = infer_block<kSplitRows>(wi, sx, sub == 0 ? pl : -1, valid, fv);
+        if (valid && sub == 0) warm_start_one(wi, i, pi, di, lp[pl], pres);
     }
 }
 
@@ -966,19 +1278,24 @@ int build_buckets(bbx_solver *s, bool with_pressure, int feat_mode, const StepCo
         wi.xq = s->xq;
         BBX_PROF_BEGIN(feat_mode == 2 ? "buckets_density_warm"
                                       : (feat_mode == 1 ? "buckets_density_features" : "buckets_density"));
-#define BBX_BUCKETS(P, F)                                                                                   \
-    k_buckets_density<P, F><<<nblocks(n), kBlock, 0, s->stream>>>(c, s->posA, s->home, s->cell_start,       \
-                                                                   s->cell_count, s->nbr16, s->nbr32,      \
-                                                                   s->nbr_cnt, s->rho, s->pres,            \
-                                                                   s->tile_tab, s->counters, wi)
-        if (with_pressure)
+#define BBX_BUCKETS(P, F)                                                                                     \
+    if (n <= kSplitUpTo)                                                                                      \
+        k_buckets_density_split<P, F><<<nblocks(n) * kSplitLanes, kBlock, 0, s->stream>>>(                    \
+            c, s->posA, s->home, s->cell_start, s->nbr16, s->nbr32, s->nbr_cnt, s->rho, s->pres, s->tile_tab, \
+            s->counters, wi);                                                                                 \
+    else                                                                                                      \
+        k_buckets_density<P, F><<<nblocks(n), kBlock, 0, s->stream>>>(                                        \
+            c, s->posA, s->home, s->cell_start, s->nbr16, s->nbr32, s->nbr_cnt, s->rho, s->pres, s->tile_tab, \
+            s->counters, wi)
+        if (with_pressure) {
             BBX_BUCKETS(true, 0);
-        else if (feat_mode == 2)
+        } else if (feat_mode == 2) {
             BBX_BUCKETS(false, 2);
-        else if (feat_mode == 1)
+        } else if (feat_mode == 1) {
             BBX_BUCKETS(false, 1);
-        else
+        } else {
             BBX_BUCKETS(false, 0);
+        }
 #undef BBX_BUCKETS
         BBX_HIP_CHECK(hipGetLastError());
         BBX_PROF_END();
