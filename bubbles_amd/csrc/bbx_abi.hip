@@ -595,28 +595,14 @@ int bbx_solver_create(int kind, const bbx_params *params, const double *pos, con
         delete s;
         return rc;
     }
-    // upload: FP64 -> FP32, id in pos.w, velocity w = 0 (no previous pressure)
-    std::vector<float4> hp(N), hv(N);
-    for (int i = 0; i < n; i++) {
-        float idf;
-        std::memcpy(&idf, &i, sizeof(int));
-        hp[i] = make_float4((float)pos[3 * i], (float)pos[3 * i + 1], (float)pos[3 * i + 2], idf);
-        hv[i] = vel ? make_float4((float)vel[3 * i], (float)vel[3 * i + 1], (float)vel[3 * i + 2], 0.f)
-                    : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    hipError_t e = hipMemcpy(s->posA, hp.data(), sizeof(float4) * N, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(s->velA, hv.data(), sizeof(float4) * N, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemset(s->step, 0, sizeof(StepBlock));
-    if (e == hipSuccess) e = hipMemset(s->flag, 0, sizeof(int));
-    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // before work on the solver's stream
-    if (e != hipSuccess) {
-        free_all(s);
-        delete s;
-        return fail(BBX_E_HIP, std::string("upload: ") + hipGetErrorString(e));
-    }
+    // FP64 -> FP32, id in pos.w, velocity w = 0 (no previous pressure);
     // fields at zero, and every slot in no chain until Setup distributes
-    rc = launch_init_fields(s);
-    if (rc == BBX_OK && hipStreamSynchronize(s->stream) != hipSuccess) rc = fail(BBX_E_HIP, "field initialisation");
+    rc = upload_vec4(s, s->posA, pos, (size_t)n, N, true);
+    if (!rc) rc = upload_vec4(s, s->velA, vel, (size_t)n, N, false);
+    if (!rc) rc = launch_fill_int(s, (int *)s->step, 0, sizeof(StepBlock) / sizeof(int));
+    if (!rc) rc = launch_fill_int(s, s->flag, 0, 1);
+    if (!rc) rc = launch_init_fields(s);
+    if (!rc && hipStreamSynchronize(s->stream) != hipSuccess) rc = fail(BBX_E_HIP, "field initialisation");
     if (rc) {
         free_all(s);
         delete s;

@@ -1,4 +1,5 @@
-// bbx_fetch.hip -- particle fields to the host in particle-id order.
+// bbx_fetch.hip -- particle fields to the host in particle-id order, and a
+// new solver's particles to the device.
 //
 // A field lies in storage (cell) order.  Sorting it out on the host took a
 // download of the id table, one of the field, and a scatter through both:
@@ -10,6 +11,7 @@
 // half of the position ping-pong that holds nothing between calls, and comes
 // in chunks while the host widens those before.
 #include <atomic>
+#include <cstring>
 #include <exception>
 #include <thread>
 
@@ -219,6 +221,31 @@ int fetch_by_id(bbx_solver *s, const FieldSource &f, const FetchTake &take) {
         }
     }
     if (__atomic_load_n(bad, __ATOMIC_ACQUIRE)) return fail(BBX_E_INVALID, "corrupt particle id table");
+    return BBX_OK;
+}
+
+int upload_vec4(bbx_solver *s, float4 *dst, const double *xyz, size_t n, size_t rows, bool with_ids) {
+    FetchRing *r = s->fetch;
+    const size_t slot = r->bytes / kFetchSlots, per = slot / sizeof(float4);
+    size_t c = 0;
+    for (size_t lo = 0; lo < rows; lo += per, c++) {
+        const int k = (int)(c % kFetchSlots);
+        if (c >= (size_t)kFetchSlots) BBX_HIP_CHECK(hipEventSynchronize(r->ev[k]));  // its last chunk has gone
+        float4 *h = (float4 *)(r->ring + (size_t)k * slot);
+        const size_t hi = std::min(rows, lo + per);
+        for (size_t i = lo; i < hi; i++) {
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (i < n && xyz) v = make_float4((float)xyz[3 * i], (float)xyz[3 * i + 1], (float)xyz[3 * i + 2], 0.f);
+            if (i < n && with_ids) {
+                const int id = (int)i;
+                std::memcpy(&v.w, &id, sizeof(int));
+            }
+            h[i - lo] = v;
+        }
+        BBX_HIP_CHECK(hipMemcpyAsync(dst + lo, h, sizeof(float4) * (hi - lo), hipMemcpyHostToDevice, s->stream));
+        BBX_HIP_CHECK(hipEventRecord(r->ev[k], s->stream));
+    }
+    BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
     return BBX_OK;
 }
 
