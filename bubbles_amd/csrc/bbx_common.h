@@ -40,6 +40,10 @@ constexpr int kBucket = BBX_BUCKET_SIZE;   // reference bucket cap
 constexpr int kBlock = 256;                // threads per workgroup (4 wave64)
 constexpr int kScanItems = 8;              // items per thread in the cell scan
 constexpr int kTabIntsHost = 48;           // ints per tile table (see bbx_tile.h)
+// Up to this many particles the chip is not full with one lane per particle,
+// and what a kernel takes is one lane's chain of latencies: the bucket build
+// gives a particle four.
+constexpr int kSmallSet = 65536;
 // LDS tile capacity in particles (bbx_tile.h): 2528 float4 (+ the tile
 // table) lets four single-array or two two-array workgroups share a CU's
 // 160 KB of LDS

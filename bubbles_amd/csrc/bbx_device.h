@@ -132,6 +132,31 @@ __device__ __forceinline__ float poly6_w_member(const SimConst &c, float d2) {
     return c.poly6 * x * x * x;
 }
 
+// The same rule as a factor: 1 inside, 0 outside.  Clamping is a modifier of
+// the instruction (v_fma_f32 with clamp takes two cycles a wave; a compare
+// and a select take seven): the next value above -1e-8 maps to 0, -1e-8
+// itself to 2^60 of their distance, far above 1.
+__device__ __forceinline__ float cutoff_mask(float of) {
+    constexpr float kScale = 1152921504606846976.f;                            // 2^60
+    constexpr float kAbove = -__builtin_bit_cast(float, __builtin_bit_cast(unsigned, 1e-8f) - 1u);
+    return __builtin_amdgcn_fmed3f(fmaf(of, -kScale, kScale * kAbove), 0.f, 1.f);
+}
+
+// 1 - a, clamped to [0, 1].  The factor of the spiky kernels: bucket members
+// lie inside the radius by more than the spiky cutoff's 1e-8 (their squared
+// distance is at most h^2 - 1e-8) for every radius up to 0.5, and a factor
+// of 1e-8 is beyond a sum's precision for larger ones; so it only has to be
+// zero for an entry that is no neighbour (and for a NaN).
+__device__ __forceinline__ float one_minus(float a, float scale) {
+    return __builtin_amdgcn_fmed3f(fmaf(-a, scale, 1.f), 0.f, 1.f);
+}
+
+// poly6 W of the factor x = 1 - d^2 / h^2, rounded before it enters a sum
+__device__ __forceinline__ float poly6_of(const SimConst &c, float x) {
+#pragma clang fp contract(off)
+    return c.poly6 * x * x * x;
+}
+
 // spiky cutoff (src/core/kernel.cpp:181-226): zero when |r-h| < 1e-8 or r > h
 __device__ __forceinline__ bool spiky_in(const SimConst &c, float r) { return cutoff_in(r - c.h); }
 
@@ -153,6 +178,29 @@ __device__ __forceinline__ void kahan_add(float &s, float &comp, float v) {
     float t = s + y;
     comp = (t - s) - y;
     s = t;
+}
+
+// The same for a product: one rounding of a b - comp
+__device__ __forceinline__ void kahan_fma(float &s, float &comp, float a, float b) {
+    const float y = fmaf(a, b, -comp);
+    const float t = s + y;
+    comp = (t - s) - y;
+    s = t;
+}
+
+// Factors of the spiky gradient of a pair at offset d: x = 1 - r / h, clamped
+// (zero outside the radius), and ir = 1 / r, zero for pairs closer than 1e-8,
+// which the gradient leaves out (the particle itself among them).  1e-30 is
+// below half an ulp of any r^2 that counts and keeps 1 / r finite at r = 0;
+// the fma decides r^2 against 1e-16 by its sign.
+struct PairFactor {
+    float x, ir;
+};
+__device__ __forceinline__ PairFactor pair_factor(const SimConst &c, float dx, float dy, float dz) {
+    const float d2 = dx * dx + dy * dy + dz * dz + 1e-30f;
+    const float ir = fast_rsq(d2);
+    const float apart = __builtin_amdgcn_fmed3f(fmaf(d2, 1e30f, -1e14f), 0.f, 1.f);
+    return PairFactor{one_minus(d2 * ir, c.inv_h), ir * apart};
 }
 
 // Reversed-box collider (ColliderSet3 with one container; CollisionHandle,

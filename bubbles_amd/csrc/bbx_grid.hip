@@ -451,6 +451,7 @@ __global__ void __launch_bounds__(kBlock) k_tile_tables(SimConst c, const int *_
 // particle computes in this launch.  kFeat == 2 then infers the network on
 // the workgroup's 256 particles and starts the substep from its pressures.
 struct WarmIn {
+    float4 *__restrict__ vr;              // (v, 1 / rho) for the viscosity gather
     StepConst st;
     const float4 *__restrict__ vel;       // own velocity, w = previous converged pressure
     int store_feat;                       // write the features to feat
@@ -458,7 +459,7 @@ struct WarmIn {
     const float *__restrict__ P;          // network parameters (kFeat == 2)
     float *__restrict__ pwarm;            // network pressure
     float *__restrict__ rho_star;         // rho* = rho at k = 0
-    float4 *__restrict__ xq;              // (x, p0 / rho^2)
+    float4 *__restrict__ xq;              // (x, q): q = p0 / rho^2 (kFeat == 2), p / rho^2 (SPH), else 0
 };
 
 // Acceptance mask of the candidates of one row (bit t: candidate t; len <=
@@ -540,7 +541,10 @@ struct BucketWriter {
         const size_t at = (size_t)((cnt - 1) >> 2) * stride + i;
         if (kStaged) {
             unsigned long long q = ((unsigned long long)qhi << 32) | qlo;
-            q >>= 16 * (4 - nfill);  // a partial quad moves down to slot 0
+            if (nfill < 4) {  // a partial quad moves down to slot 0
+                q >>= 16 * (4 - nfill);
+                q |= (kFarEntry * 0x0001000100010001ull) << (16 * nfill);
+            }
             reinterpret_cast<uint2 *>(nbr16)[at] = make_uint2((unsigned)q, (unsigned)(q >> 32));
         } else {
             int4 v = make_int4(e0, e1, e2, e3);
@@ -631,7 +635,7 @@ __device__ __forceinline__ void finish_features(const SimConst &c, const WarmIn 
     fv[BBX_F_CX] = cx * inv;
     fv[BBX_F_CY] = cy * inv;
     fv[BBX_F_CZ] = cz * inv;
-    fv[BBX_F_CNORM] = sqrtf(cx * cx + cy * cy + cz * cz) * inv;
+    fv[BBX_F_CNORM] = sqrtf(fmaf(cz, cz, fmaf(cy, cy, cx * cx))) * inv;
     fv[BBX_F_PPREV] = wi.st.delta != 0.f ? vi.w / (wi.st.delta * c.rho0) : 0.f;
     fv[BBX_F_VY] = vi.y * vs;
     fv[BBX_F_VNORM] = sqrtf(vi.x * vi.x + vi.y * vi.y + vi.z * vi.z) * vs;
@@ -901,9 +905,15 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
                 for (int f = 0; f < BBX_NFEAT; f++) wi.feat[(size_t)f * S + i] = fv[f];
             }
         }
+        float p = 0.f;
         if (kPressure) {
-            pres[i] = tait_pressure(c, di);
+            p = tait_pressure(c, di);
+            pres[i] = p;
         }
+        // the positions of the pressure-force gather; q follows
+        if (kFeat != 2) wi.xq[i] = make_float4(pi.x, pi.y, pi.z, kPressure ? p / (di * di) : 0.f);
+        const float4 vo = wi.vel[i];
+        wi.vr[i] = make_float4(vo.x, vo.y, vo.z, fast_rcp(di));
         if (bw.dropped) atomicAdd(&counters[CNT_OVERFLOW], bw.dropped);
     };
     if (valid) with_staging(staged, per_particle);
@@ -918,17 +928,16 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
 // per lane (nine rows of tests, the emission, the sum), 26 us for 2k
 // particles however few tiles there are.  Each lane of a particle takes rows
 // lane, lane + 4, lane + 8; the lanes exchange the cells' counts, so that
-// each knows where its entries go, and emit into LDS; then each sums (and
-// writes out) every fourth quad.  A workgroup stages its tile's candidates
+// each knows where its entries go, and emit into LDS; then each evaluates
+// (and writes out) every fourth quad.  A workgroup stages its tile's candidates
 // like the others, so tile tables and entries are the same.  A particle with
 // a crowded row or more neighbours than the cap is walked cell by cell by its
 // first lane.
 //
-// Measured (us, one lane per particle / four): 25.2 / 12.5 at 2k, 28.3 / 13.9
-// at 16k, 29.7 / 19.0 at 35k, 37.6 / 34.0 at 94k; 62.6 / 206 at 255k, where
-// the chip is full and the four workgroups' staging and the longer emission
-// count.
-constexpr int kSplitUpTo = 98304;
+// Used up to kSmallSet.  Measured (us, one lane per particle / four): 25.2 / 12.3
+// at 2k, 28.3 / 14.5 at 16k, 29.7 / 23.2 at 35k, 37.6 / 41.2 at 94k, 62.6 /
+// over 200 at 255k, where the chip is full and the four workgroups' staging
+// and the longer emission count.
 constexpr int kSplitLanes = 4;
 constexpr int kSplitRows = kBlock / kSplitLanes;  // particles per workgroup
 constexpr int kSplitMax = kBucket;                // bucket entries held in LDS
@@ -941,9 +950,9 @@ __device__ __forceinline__ int quad_lane(int v) {
 }
 __device__ __forceinline__ int quad_xor1(int v) { return __builtin_amdgcn_mov_dpp(v, 0xb1, 0xf, 0xf, true); }
 __device__ __forceinline__ int quad_xor2(int v) { return __builtin_amdgcn_mov_dpp(v, 0x4e, 0xf, 0xf, true); }
-__device__ __forceinline__ float quad_sum(float v) {
-    v += __int_as_float(quad_xor1(__float_as_int(v)));
-    return v + __int_as_float(quad_xor2(__float_as_int(v)));
+template <int k>
+__device__ __forceinline__ float quad_lane_f(float v) {
+    return __int_as_float(quad_lane<k>(__float_as_int(v)));
 }
 
 template <bool kPressure, int kFeat>
@@ -1100,14 +1109,17 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density_split(SimConst c,
         float sum = 0.f, comp = 0.f;
         float m1 = 0.f, m2 = 0.f, m3 = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
         const int self = kStaged ? (i + tt.rdelta[4]) << kSlotShift : i;
-        for (int q = sub; 4 * q < cnt; q += kSplitLanes) {
-            const int rem = cnt - 4 * q;
-            int4 e;
-            if (in_lds) {  // unused slots of the last quad are zero in the table
+        for (int q0 = 0; 4 * q0 < cnt; q0 += kSplitLanes) {
+            const int q = q0 + sub, rem = cnt - 4 * q;
+            int4 e = make_int4(self, self, self, self);
+            if (rem <= 0) {
+                // a lane past the last quad adds zeros below
+            } else if (in_lds) {  // unused slots of the last quad as in BucketWriter
                 if (kStaged) {
+                    constexpr unsigned kTop = kFarEntry << 16;
                     unsigned w0 = ent[pl][2 * q], w1 = ent[pl][2 * q + 1];
-                    w0 = rem > 1 ? w0 : w0 & 0xffffu;
-                    w1 = rem > 3 ? w1 : (rem > 2 ? w1 & 0xffffu : 0u);
+                    w0 = rem > 1 ? w0 : (w0 & 0xffffu) | kTop;
+                    w1 = rem > 3 ? w1 : (rem > 2 ? w1 & 0xffffu : kFarEntry) | kTop;
                     reinterpret_cast<uint2 *>(nbr16)[(size_t)q * c.stride + i] = make_uint2(w0, w1);
                     e = quad_unpack(make_int4((int)w0, (int)w1, 0, 0), true);
                 } else {
@@ -1119,36 +1131,42 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density_split(SimConst c,
                 e = quad_unpack(nbr_quad(nbr16, nbr32, kStaged, i, c.stride, q), kStaged);
             }
             const int j4[4] = {e.x, rem > 1 ? e.y : self, rem > 2 ? e.z : self, rem > 3 ? e.w : self};
-            float4 pj[4];
-#pragma unroll
-            for (int v = 0; v < 4; v++) pj[v] = kStaged ? lds_at(sx, j4[v]) : pos[j4[v]];
+            float w[4], d2[4], dx[4], dy[4], dz[4];
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const float dx = pi.x - pj[v].x, dy = pi.y - pj[v].y, dz = pi.z - pj[v].z;
-                const float d2 = dx * dx + dy * dy + dz * dz;
-                const float w = poly6_w_member(c, d2);
-                kahan_add(sum, comp, v < rem ? w : 0.f);  // a dead entry adds an exact zero
-                if constexpr (kFeat > 0) {
-                    const float r = fast_sqrt(d2);
-                    m1 += r;
-                    m2 += d2;
-                    m3 = fmaf(r, d2, m3);
-                    cx -= dx;
-                    cy -= dy;
-                    cz -= dz;
-                }
+                const float4 pj = kStaged ? lds_at(sx, j4[v]) : pos[j4[v]];
+                dx[v] = pi.x - pj.x;
+                dy[v] = pi.y - pj.y;
+                dz[v] = pi.z - pj.z;
+                d2[v] = dx[v] * dx[v] + dy[v] * dy[v] + dz[v] * dz[v];
+                const float m = poly6_w_member(c, d2[v]);
+                w[v] = v < rem ? m : 0.f;  // a dead entry adds an exact zero
             }
+            // The terms are the lanes'; the sums run in bucket order, each
+            // lane the same one, so that they are those of the kernel above
+            // bit for bit.
+            auto add_quad = [&](auto lane) {
+                constexpr int L = decltype(lane)::value;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    kahan_add(sum, comp, quad_lane_f<L>(w[v]));
+                    if constexpr (kFeat > 0) {
+                        const float dd = quad_lane_f<L>(d2[v]), r = fast_sqrt(dd);
+                        m1 += r;
+                        m2 += dd;
+                        m3 = fmaf(r, dd, m3);
+                        cx -= quad_lane_f<L>(dx[v]);
+                        cy -= quad_lane_f<L>(dy[v]);
+                        cz -= quad_lane_f<L>(dz[v]);
+                    }
+                }
+            };
+            add_quad(std::integral_constant<int, 0>{});
+            add_quad(std::integral_constant<int, 1>{});
+            add_quad(std::integral_constant<int, 2>{});
+            add_quad(std::integral_constant<int, 3>{});
         }
-        // the lanes' compensated partial sums
-        di = quad_sum(sum - comp) * c.mass;
-        if constexpr (kFeat > 0) {
-            m1 = quad_sum(m1);
-            m2 = quad_sum(m2);
-            m3 = quad_sum(m3);
-            cx = quad_sum(cx);
-            cy = quad_sum(cy);
-            cz = quad_sum(cz);
-        }
+        di = sum * c.mass;
         if (sub == 0) {
             nbr_cnt[i] = cnt;
             rho[i] = di;
@@ -1160,7 +1178,14 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density_split(SimConst c,
                     for (int f = 0; f < BBX_NFEAT; f++) wi.feat[(size_t)f * S + i] = fv[f];
                 }
             }
-            if (kPressure) pres[i] = tait_pressure(c, di);
+            float p = 0.f;
+            if (kPressure) {
+                p = tait_pressure(c, di);
+                pres[i] = p;
+            }
+            if (kFeat != 2) wi.xq[i] = make_float4(pi.x, pi.y, pi.z, kPressure ? p / (di * di) : 0.f);
+            const float4 vo = wi.vel[i];
+            wi.vr[i] = make_float4(vo.x, vo.y, vo.z, fast_rcp(di));
             if (dropped) atomicAdd(&counters[CNT_OVERFLOW], dropped);
         }
     };
@@ -1178,10 +1203,11 @@ __global__ void __launch_bounds__(kBlock) k_density(SimConst c, const float4 *__
                                                     const int *__restrict__ nbr_cnt,
                                                     const int *__restrict__ tile_tab,
                                                     float *__restrict__ rho) {
-    __shared__ float4 sx[kTileCap];
+    __shared__ float4 sx[kFarSlot + 1];
     __shared__ TileTab tt;
     const int tile = tile_of_block();
     tab_load_shared(tile_tab + (size_t)tile * kTabInts, tt);
+    if (threadIdx.x == 0) sx[kFarSlot] = far_particle(0.f);
     __syncthreads();
     const bool staged = tt.staged != 0;
     if (staged) tab_stage(tt, sx, [&](int j) { return pos[j]; });
@@ -1270,6 +1296,7 @@ int build_buckets(bbx_solver *s, bool with_pressure, int feat_mode, const StepCo
         WarmIn wi{};
         if (st) wi.st = *st;
         wi.vel = s->velA;
+        wi.vr = s->velB;  // free until the integration writes it
         wi.store_feat = s->keep_features;
         wi.feat = s->feat;
         wi.P = feat_mode == 2 ? mlp_params_device(s->mlp) : nullptr;
@@ -1279,7 +1306,7 @@ int build_buckets(bbx_solver *s, bool with_pressure, int feat_mode, const StepCo
         BBX_PROF_BEGIN(feat_mode == 2 ? "buckets_density_warm"
                                       : (feat_mode == 1 ? "buckets_density_features" : "buckets_density"));
 #define BBX_BUCKETS(P, F)                                                                                     \
-    if (n <= kSplitUpTo)                                                                                      \
+    if (n <= kSmallSet)                                                                                       \
         k_buckets_density_split<P, F><<<nblocks(n) * kSplitLanes, kBlock, 0, s->stream>>>(                    \
             c, s->posA, s->home, s->cell_start, s->nbr16, s->nbr32, s->nbr_cnt, s->rho, s->pres, s->tile_tab, \
             s->counters, wi);                                                                                 \

@@ -46,34 +46,39 @@ struct NbrTab {
 
 // The tank alone takes the inlined reversed-box path; a collider list goes
 // through the collider-set rule (same result for the tank as its only entry).
+// Kernels are compiled for either (kList): the list's code alone takes the
+// pressure-force kernel from 63 registers to 127.
+template <bool kList>
 __device__ __forceinline__ void collide_any(const SimConst &c, float e, float3 &p, float3 &v) {
-    if (c.ncoll == 0)
-        collide(c, e, p, v);
-    else
+    if constexpr (kList)
         resolve_colliders(c.coll, c.ncoll, c.radius, e, p, v);
+    else
+        collide(c, e, p, v);
 }
 
 // PredictVelocityAndPositionFor (src/equations/pcisph_equations3.cpp:3-28):
 // v* = v + dt/m (f + f_p), x* = x + dt v*, collider with restitution 0.
+template <bool kList>
 __device__ __forceinline__ float4 predict_position(const SimConst &c, const StepConst &st,
                                                    float4 x, float4 v, float fx, float fy,
                                                    float fz) {
     float3 tv = make_float3(v.x + st.dt_over_m * fx, v.y + st.dt_over_m * fy,
                             v.z + st.dt_over_m * fz);
     float3 tp = make_float3(x.x + st.dt * tv.x, x.y + st.dt * tv.y, x.z + st.dt * tv.z);
-    collide_any(c, 0.f, tp, tv);
+    collide_any<kList>(c, 0.f, tp, tv);
     return make_float4(tp.x, tp.y, tp.z, 0.f);
 }
 
 // TimeIntegrationFor (src/equations/sph_equations3.cpp:283-339): symplectic
 // Euler, collider with restitution 0.6, clamp into the domain, 0.9-cell flag.
+template <bool kList>
 __device__ __forceinline__ void integrate_one(const SimConst &c, float dt, float4 xi, float4 vi,
                                               float Fx, float Fy, float Fz, float3 &p, float3 &v,
                                               int *__restrict__ flag) {
     const float inv_m = 1.f / c.mass;
     v = make_float3(vi.x + dt * (Fx * inv_m), vi.y + dt * (Fy * inv_m), vi.z + dt * (Fz * inv_m));
     p = make_float3(xi.x + dt * v.x, xi.y + dt * v.y, xi.z + dt * v.z);
-    collide_any(c, 0.6f, p, v);
+    collide_any<kList>(c, 0.6f, p, v);
     if (!inside_box(p.x, p.y, p.z, c.bmin, c.bmax)) {
         p.x = fminf(fmaxf(p.x, c.bmin[0] + c.radius), c.bmax[0] - c.radius);
         p.y = fminf(fmaxf(p.y, c.bmin[1] + c.radius), c.bmax[1] - c.radius);
@@ -89,7 +94,11 @@ __device__ __forceinline__ void integrate_one(const SimConst &c, float dt, float
 //       2 = + the warm start's pressure force f_p(p0) at rho* = rho, whose
 //           (x, q0 = p0 / rho^2) the bucket kernel wrote to xq, and
 //           predict(k=0) with it
-// LDS: neighbour position (mode 2: with q0), (velocity, density).
+// LDS: neighbour (position, q0) and (velocity, 1 / density), two LDS DMA
+// streams: the bucket kernel writes the pairs xq and vr (vr in the half of
+// the velocity ping-pong that the integration fills later), which costs it
+// 2 us at 1M particles.  Put together here, through registers, they cost this
+// kernel 15 us of 90.
 //
 // Two lanes per particle: the two LDS arrays allow only two workgroups per
 // CU, so each particle's bucket is split between lanes 2p and 2p + 1 (even
@@ -98,21 +107,26 @@ __device__ __forceinline__ void integrate_one(const SimConst &c, float dt, float
 // ---------------------------------------------------------------------------
 constexpr int kNpThreads = 2 * kBlock;
 
-template <int kMode>
+template <int kMode, bool kList>
 __global__ void __launch_bounds__(kNpThreads) __attribute__((amdgpu_waves_per_eu(4))) k_nonpressure(SimConst c, StepConst st, NbrTab nb,
                                                             const float4 *__restrict__ pos,
                                                             const float4 *__restrict__ vel,
                                                             const float *__restrict__ rho,
                                                             const float4 *__restrict__ xq,
+                                                            const float4 *__restrict__ vr,
                                                             float4 *__restrict__ force,
                                                             float4 *__restrict__ xstar,
                                                             float *__restrict__ rho_star) {
     constexpr bool kWarm = kMode == 2;
-    __shared__ float4 sx[kTileCap2];
-    __shared__ float4 sv[kTileCap2];
+    __shared__ float4 sx[kFarSlot + 1];
+    __shared__ float4 sv[kFarSlot + 1];
     __shared__ TileTab tt;
     const int tile = tile_of_block();
     tab_load_shared(nb.tab + (size_t)tile * kTabInts, tt);
+    if (threadIdx.x == 0) {
+        sx[kFarSlot] = far_particle(0.f);
+        sv[kFarSlot] = make_float4(0.f, 0.f, 0.f, 1.f);
+    }
     __syncthreads();
     const bool staged = tt.staged != 0;                  // buckets hold LDS-local indices
     const bool in_lds = staged && tt.total <= c.tile_cap2;  // and they fit this kernel's LDS
@@ -122,8 +136,6 @@ __global__ void __launch_bounds__(kNpThreads) __attribute__((amdgpu_waves_per_eu
     int cnt = 0;
     float4 xi = make_float4(0.f, 0.f, 0.f, 0.f), vi = xi;
     float rhoi = 0.f, qi = 0.f;
-    // (x, q0) in the warm mode, else the positions
-    const float4 *__restrict__ sxsrc = kWarm ? xq : pos;
     // this lane's first two quads: half, half + 2
     NbrQuads<2> first{};
     if (valid) {  // independent of the staging: requested before it
@@ -134,23 +146,12 @@ __global__ void __launch_bounds__(kNpThreads) __attribute__((amdgpu_waves_per_eu
         if (kWarm) qi = xq[i].w;
         first = nbr_prefetch<2, 2>(nb.n16, nb.n32, staged, i, c.stride, half);
     }
-    // staged through registers: the (velocity, 1 / density) pair is assembled on
-    // the way, and seven 4-byte LDS DMA streams measured slower here; both
-    // arrays in one pass, so each slot's storage index is found once
     if (in_lds) {
-        struct Slot {
-            float4 a, b;
-        };
-        tab_stage_with(
-            tt,
-            [&](int j) {
-                const float4 v = vel[j];
-                return Slot{sxsrc[j], make_float4(v.x, v.y, v.z, fast_rcp(rho[j]))};  // 1 / rho_j once
-            },
-            [&](int e, const Slot &v) {
-                sx[e] = v.a;
-                sv[e] = v.b;
-            });
+        tab_stage_dma(tt, [&](int j, int e) {
+            lds_dma16(xq + j, sx + e);
+            lds_dma16(vr + j, sv + e);
+        });
+        lds_dma_wait();
     }
     __syncthreads();
     if (!valid) return;  // the lane pair shares validity
@@ -166,38 +167,31 @@ __global__ void __launch_bounds__(kNpThreads) __attribute__((amdgpu_waves_per_eu
                 a = lds_at(sx, j);
                 b = lds_at(sv, j);
             } else {
-                const int g = staged ? tab_global(tt, j >> kSlotShift) : j;
-                a = sxsrc[g];
-                const float4 v = vel[g];
-                b = make_float4(v.x, v.y, v.z, fast_rcp(rho[g]));
+                const int g = staged ? (live ? tab_global(tt, j >> kSlotShift) : i) : j;
+                a = xq[g];
+                b = vr[g];
             }
             const float dx = xi.x - a.x, dy = xi.y - a.y, dz = xi.z - a.z;
+            // no branches and no masks: the cutoff is the clamped factor x,
+            // a dead entry (the far slot) has x = 0
             const float d2 = dx * dx + dy * dy + dz * dz;
-            const float r = fast_sqrt(d2);
-            // masks instead of branches: every pair's arithmetic runs, a
-            // dead pair contributes exact zeros, and the neighbour's LDS
-            // reads stay unconditional (so they are issued early)
-            const bool in = live & spiky_in(c, r);
-            const float x = keep_if(in, 1.f - r * c.inv_h);
+            float x = one_minus(fast_sqrt(d2), c.inv_h);
+            if (!kL) x = live ? x : 0.f;
             // viscosity term mu m^2 (v_j - v_i) d2W(r) / rho_j
             const float s = coef * (c.spiky_lap * x) * b.w;
-            fx += (b.x - vi.x) * s;
-            fy += (b.y - vi.y) * s;
-            fz += (b.z - vi.z) * s;
+            fx = fmaf(b.x - vi.x, s, fx);
+            fy = fmaf(b.y - vi.y, s, fy);
+            fz = fmaf(b.z - vi.z, s, fz);
             if constexpr (kWarm) {
                 // PredictPressureForceFor (src/equations/pcisph_equations3.cpp:114-155)
-                // at the current positions with rho* = rho: pairs j != i with
-                // 1e-8 <= r inside the spiky cutoff, the pressure-force
-                // kernel's pair rule (r = d2 rsqrt(d2) is NaN for d2 = 0);
-                // with d = x_i - x_j here, f_p = +sum g d
-                const float ir = fast_rsq(d2);
-                const float rp = d2 * ir;
-                const bool inp = live & spiky_in(c, rp) & (rp >= 1e-8f);
-                const float xp = 1.f - rp * c.inv_h;
-                const float g = keep_if(inp, kg * (qi + a.w) * xp * xp * ir);
-                kahan_add(px, epx, g * dx);
-                kahan_add(py, epy, g * dy);
-                kahan_add(pz, epz, g * dz);
+                // at the current positions with rho* = rho, the pressure-force
+                // kernel's pair rule; with d = x_i - x_j here, f_p = +sum g d
+                const PairFactor f = pair_factor(c, dx, dy, dz);
+                const float xp = kL || live ? f.x : 0.f;
+                const float g = kg * (qi + a.w) * xp * xp * f.ir;
+                kahan_fma(px, epx, g, dx);
+                kahan_fma(py, epy, g, dy);
+                kahan_fma(pz, epz, g, dz);
             }
         };
         // quads half, half + 2, half + 4, ... of the bucket, two in flight
@@ -223,7 +217,7 @@ __global__ void __launch_bounds__(kNpThreads) __attribute__((amdgpu_waves_per_eu
     if (half == 0) {
         force[i] = make_float4(fx, fy, fz, 0.f);
         if (kMode >= 1) {
-            xstar[i] = predict_position(c, st, xi, vi, fx + fpx, fy + fpy, fz + fpz);
+            xstar[i] = predict_position<kList>(c, st, xi, vi, fx + fpx, fy + fpy, fz + fpz);
             rho_star[i] = rhoi;
         }
     }
@@ -245,14 +239,13 @@ constexpr int kPpDepth = 1;
 __global__ void __launch_bounds__(kPpThreads) k_predict_pressure(SimConst c, StepConst st, double delta,
                                                                  NbrTab nb,
                                                                  const float4 *__restrict__ xstar,
-                                                                 const float4 *__restrict__ pos,
                                                                  float *__restrict__ pres,
                                                                  float *__restrict__ rho_star,
                                                                  float4 *__restrict__ xq,
                                                                  LoopState *__restrict__ loop, int k) {
     // predicted positions, copied by 16-byte LDS DMA (the w lane is the
     // unused fourth word of x*)
-    __shared__ float4 sx[kTileCap];
+    __shared__ float4 sx[kFarSlot + 1];
     __shared__ unsigned long long wmax[kPpThreads / 64];
     if (k > 0 && loop->done[k - 1]) return;  // uniform early exit
     const int tile = tile_of_block();
@@ -271,12 +264,13 @@ __global__ void __launch_bounds__(kPpThreads) k_predict_pressure(SimConst c, Ste
     const int ic = valid ? i : c.n - 1;  // the kernel runs only for n > 0
     NbrQuads<kPpDepth> first = nbr_prefetch<kPpDepth, 2>(nb.n16, nb.n32, true, ic, c.stride, half);
     const int cnt_ic = nb.cnt[ic];
-    const float4 xi = xstar[ic], pi = pos[ic];
+    const float4 xi = xstar[ic];
     const int cnt = valid ? cnt_ic : 0;
     const float pown = pres[ic];
     const float pold = (!st.first && half == 0) ? pown : 0.f;
     const bool staged = tab_word(tw, 1) != 0;
     if (staged) {
+        if (threadIdx.x == 0) sx[kFarSlot] = far_particle(0.f);
         tab_stage_dma_wave(tw, [&](int j, int e) { lds_dma16(xstar + j, sx + e); });
         lds_dma_wait();
     } else if (valid) {
@@ -297,9 +291,12 @@ __global__ void __launch_bounds__(kPpThreads) k_predict_pressure(SimConst c, Ste
                     const float4 g = xstar[j];
                     xj = make_float3(g.x, g.y, g.z);
                 }
-                float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-                const float w = poly6_w(c, dx * dx + dy * dy + dz * dz);
-                kahan_add(sum, comp, live ? w : 0.f);  // a dead entry adds an exact zero
+                const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+                // poly6; zero outside, and for a dead entry
+                const float d2 = dx * dx + dy * dy + dz * dz;
+                float x = (1.f - d2 * c.inv_h2) * cutoff_mask(d2 - c.h2);
+                if (!kS) x = live ? x : 0.f;
+                kahan_add(sum, comp, poly6_of(c, x));
             }, half);
         });
         // the pair's compensated partial sums; a + b == b + a, so both lanes
@@ -319,7 +316,8 @@ __global__ void __launch_bounds__(kPpThreads) k_predict_pressure(SimConst c, Ste
             pres[i] = p;
             rho_star[i] = density;
             float d2 = density * density;
-            xq[i] = make_float4(pi.x, pi.y, pi.z, (fabsf(d2) < 1e-8f) ? 0.f : p / d2);
+            // the position beside it is the substep's, written by the bucket kernel
+            xq[i].w = (fabsf(d2) < 1e-8f) ? 0.f : p / d2;
             // |err| with a cleared sign bit: -0.0 must not win the unsigned max
             // (the reference's AbsfMax keeps the first of equal squares)
             const double ae = fabs(err);
@@ -352,6 +350,7 @@ __global__ void __launch_bounds__(kPpThreads) k_predict_pressure(SimConst c, Ste
 // Quads in flight per lane in the pressure-force gather: 2 measured faster
 // than 3, 4 and 6 over the whole 1M run (0.4%, 1% and 3%).
 constexpr int kPfDepth = 2;
+template <bool kList>
 __global__ void __launch_bounds__(kBlock) k_pressure_force(SimConst c, StepConst st, NbrTab nb,
                                                            const float4 *__restrict__ pos,
                                                            const float4 *__restrict__ vel,
@@ -369,7 +368,7 @@ __global__ void __launch_bounds__(kBlock) k_pressure_force(SimConst c, StepConst
                                                            LoopSignal *sig, unsigned seq,
                                                            const int *__restrict__ counters) {
     // (position, q = p / rho*^2) of the neighbours, copied by 16-byte LDS DMA
-    __shared__ float4 sx[kTileCap];
+    __shared__ float4 sx[kFarSlot + 1];
     if (k > 0 && loop->done[k - 1]) {
         // an earlier iteration integrated: pass the flag on and exit (uniform)
         if (blockIdx.x == 0 && threadIdx.x == 0) loop->done[k] = 1;
@@ -391,8 +390,8 @@ __global__ void __launch_bounds__(kBlock) k_pressure_force(SimConst c, StepConst
     const int ic = valid ? i : c.n - 1;  // the kernel runs only for n > 0
     NbrQuads<kPfDepth> first = nbr_prefetch<kPfDepth>(nb.n16, nb.n32, true, ic, c.stride);
     const int cnt_ic = nb.cnt[ic];
-    const float4 xi = pos[ic];
-    const float qi = xq[ic].w;
+    const float4 xi = xq[ic];  // the position and its own q
+    const float qi = xi.w;
     const float4 fi = force[ic], vi = vel[ic];
     const int cnt = valid ? cnt_ic : 0;
     const bool staged = tab_word(tw, 1) != 0;
@@ -427,6 +426,7 @@ __global__ void __launch_bounds__(kBlock) k_pressure_force(SimConst c, StepConst
         }
     }
     if (staged) {
+        if (threadIdx.x == 0) sx[kFarSlot] = far_particle(0.f);
         tab_stage_dma_wave(tw, [&](int j, int e) { lds_dma16(xq + j, sx + e); });
         lds_dma_wait();
     } else {
@@ -435,42 +435,32 @@ __global__ void __launch_bounds__(kBlock) k_pressure_force(SimConst c, StepConst
     __syncthreads();
     unsigned fbits = 0u;
     if (valid) {
-        // pairs j != i with 1e-8 <= r and r inside the spiky cutoff
-        // (src/equations/pcisph_equations3.cpp:128-150); r = d2 * rsqrt(d2)
-        // is NaN for d2 = 0 (the particle itself or a coincident one), which
-        // fails both tests
+        // gradW(r, dir) = -dW(r) dir = spiky_grad x^2 (x_j - x_i) / r over
+        // pairs j != i with 1e-8 <= r and r inside the cutoff
+        // (src/equations/pcisph_equations3.cpp:128-150)
         const float kg = c.mass2 * c.spiky_grad;
         float tx = 0.f, ty = 0.f, tz = 0.f, ex = 0.f, ey = 0.f, ez = 0.f;
         with_staging(staged, [&](auto tag) {
             constexpr bool kS = decltype(tag)::value;
             for_each_neighbour_from<kPfDepth>(first, nb.n16, nb.n32, kS, i, cnt, c.stride, [&](int j, bool live) {
                 const float4 a = kS ? lds_at(sx, j) : xq[j];  // (x_j, q_j)
-                const float qj = a.w;
                 const float dx = a.x - xi.x, dy = a.y - xi.y, dz = a.z - xi.z;
-                const float d2 = dx * dx + dy * dy + dz * dz;
-                const float ir = fast_rsq(d2);
-                const float r = d2 * ir;
-                const bool in = live && spiky_in(c, r) && r >= 1e-8f;
-                const float x = 1.f - r * c.inv_h;
-                // gradW(r, dir) = -dW(r) dir = spiky_grad x^2 (x_j - x_i)/r;
-                // a dead pair adds an exact zero.  Masking the bits (rather
-                // than ?:) keeps the pair's arithmetic unconditional, so the
-                // compiler issues the neighbour's LDS read as one 16-byte
-                // load and does not branch per pair.
-                const float g = keep_if(in, kg * (qi + qj) * x * x * ir);
-                kahan_add(tx, ex, g * dx);
-                kahan_add(ty, ey, g * dy);
-                kahan_add(tz, ez, g * dz);
+                const PairFactor f = pair_factor(c, dx, dy, dz);
+                const float x = kS || live ? f.x : 0.f;  // zero outside, and for a dead entry
+                const float g = kg * (qi + a.w) * x * x * f.ir;
+                kahan_fma(tx, ex, g, dx);
+                kahan_fma(ty, ey, g, dy);
+                kahan_fma(tz, ez, g, dz);
             });
         });
         const float fpx = -tx, fpy = -ty, fpz = -tz;
         if (!integrate) {
-            xstar[i] = predict_position(c, st, xi, vi, fi.x + fpx, fi.y + fpy, fi.z + fpz);
+            xstar[i] = predict_position<kList>(c, st, xi, vi, fi.x + fpx, fi.y + fpy, fi.z + fpz);
         } else {
             const float Fx = fi.x + fpx, Fy = fi.y + fpy, Fz = fi.z + fpz;
             float3 p, v;
-            integrate_one(c, st.dt, xi, vi, Fx, Fy, Fz, p, v, flag);
-            pos_out[i] = make_float4(p.x, p.y, p.z, xi.w);
+            integrate_one<kList>(c, st.dt, xi, vi, Fx, Fy, Fz, p, v, flag);
+            pos_out[i] = make_float4(p.x, p.y, p.z, pos[i].w);
             vel_out[i] = make_float4(v.x, v.y, v.z, pres[i]);
             force[i] = make_float4(Fx, Fy, Fz, 0.f);  // the lane read force[i] above
             fp_out[i] = make_float4(fpx, fpy, fpz, 0.f);
@@ -491,11 +481,15 @@ __global__ void __launch_bounds__(kBlock) k_sph_force(SimConst c, NbrTab nb,
                                                       const float *__restrict__ rho,
                                                       const float *__restrict__ pres,
                                                       float4 *__restrict__ force) {
-    __shared__ float4 sx[kTileCap2];
-    __shared__ float4 sv[kTileCap2];
+    __shared__ float4 sx[kFarSlot + 1];
+    __shared__ float4 sv[kFarSlot + 1];
     __shared__ TileTab tt;
     const int tile = tile_of_block();
     tab_load_shared(nb.tab + (size_t)tile * kTabInts, tt);
+    if (threadIdx.x == 0) {
+        sx[kFarSlot] = far_particle(0.f);
+        sv[kFarSlot] = make_float4(0.f, 0.f, 0.f, 1.f);
+    }
     __syncthreads();
     const bool staged = tt.staged != 0;
     const bool in_lds = staged && tt.total <= c.tile_cap2;
@@ -533,7 +527,7 @@ __global__ void __launch_bounds__(kBlock) k_sph_force(SimConst c, NbrTab nb,
             xj = lds_at(sx, j);
             vj = lds_at(sv, j);
         } else {
-            const int g = staged ? tab_global(tt, j >> kSlotShift) : j;
+            const int g = staged ? (live ? tab_global(tt, j >> kSlotShift) : i) : j;
             xj = xq(g);
             vj = vr(g);
         }
@@ -555,6 +549,7 @@ __global__ void __launch_bounds__(kBlock) k_sph_force(SimConst c, NbrTab nb,
 }
 
 // TimeIntegrationFor as a separate pass (SPH two-phase form)
+template <bool kList>
 __global__ void __launch_bounds__(kBlock) k_integrate(SimConst c, StepConst st,
                                                       const float4 *__restrict__ pos,
                                                       const float4 *__restrict__ vel,
@@ -568,7 +563,7 @@ __global__ void __launch_bounds__(kBlock) k_integrate(SimConst c, StepConst st,
     if (i < c.n) {
         const float4 xi = pos[i], vi = vel[i], fi = force[i];
         float3 p, v;
-        integrate_one(c, st.dt, xi, vi, fi.x, fi.y, fi.z, p, v, flag);
+        integrate_one<kList>(c, st.dt, xi, vi, fi.x, fi.y, fi.z, p, v, flag);
         pos_out[i] = make_float4(p.x, p.y, p.z, xi.w);
         vel_out[i] = make_float4(v.x, v.y, v.z, vi.w);
         fbits = __float_as_uint(sqrtf(fi.x * fi.x + fi.y * fi.y + fi.z * fi.z));
@@ -583,11 +578,15 @@ __global__ void __launch_bounds__(kBlock) k_xsph(SimConst c, StepConst st, NbrTa
                                                  const float4 *__restrict__ vel,
                                                  const float *__restrict__ rho,
                                                  float4 *__restrict__ vel_out) {
-    __shared__ float4 sx[kTileCap2];
-    __shared__ float4 sv[kTileCap2];
+    __shared__ float4 sx[kFarSlot + 1];
+    __shared__ float4 sv[kFarSlot + 1];
     __shared__ TileTab tt;
     const int tile = tile_of_block();
     tab_load_shared(nb.tab + (size_t)tile * kTabInts, tt);
+    if (threadIdx.x == 0) {
+        sx[kFarSlot] = far_particle(0.f);
+        sv[kFarSlot] = make_float4(0.f, 0.f, 0.f, 1.f);
+    }
     __syncthreads();
     const bool staged = tt.staged != 0;
     const bool in_lds = staged && tt.total <= c.tile_cap2;
@@ -612,7 +611,7 @@ __global__ void __launch_bounds__(kBlock) k_xsph(SimConst c, StepConst st, NbrTa
             xj = lds_at(sx, j);
             vj = lds_at(sv, j);
         } else {
-            const int g = staged ? tab_global(tt, j >> kSlotShift) : j;
+            const int g = staged ? (live ? tab_global(tt, j >> kSlotShift) : i) : j;
             xj = pos[g];
             vj = vr(g);
         }
@@ -644,13 +643,34 @@ static NbrTab nbr_tab(const bbx_solver *s) {
     return NbrTab{s->nbr16, s->nbr32, s->nbr_cnt, s->tile_tab};
 }
 
+// the gather's inputs from the fields as they are now (a substep's come from
+// its bucket kernel)
+__global__ void __launch_bounds__(kBlock) k_pair_inputs(int n, const float4 *__restrict__ pos,
+                                                        const float4 *__restrict__ vel,
+                                                        const float *__restrict__ rho, float4 *__restrict__ xq,
+                                                        float4 *__restrict__ vr) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const float4 x = pos[i], v = vel[i];
+    xq[i] = make_float4(x.x, x.y, x.z, 0.f);
+    vr[i] = make_float4(v.x, v.y, v.z, fast_rcp(rho[i]));
+}
+
 int run_nonpressure(bbx_solver *s, const StepConst &st, int mode) {
     if (s->n == 0) return BBX_OK;
+    if (mode == 0) {
+        k_pair_inputs<<<nblocks(s->n), kBlock, 0, s->stream>>>(s->n, s->posA, s->velA, s->rho, s->xq, s->velB);
+        BBX_HIP_CHECK(hipGetLastError());
+    }
     const unsigned nb = nblocks(s->n);
     const NbrTab t = nbr_tab(s);
-#define BBX_NP(M)                                                                                     \
-    k_nonpressure<M><<<nb, kNpThreads, 0, s->stream>>>(s->sc, st, t, s->posA, s->velA, s->rho, s->xq, \
-                                                     s->force, s->xstar, s->rho_star)
+#define BBX_NP(M)                                                                                            \
+    if (s->ncoll)                                                                                            \
+        k_nonpressure<M, true><<<nb, kNpThreads, 0, s->stream>>>(s->sc, st, t, s->posA, s->velA, s->rho, s->xq, \
+                                                                 s->velB, s->force, s->xstar, s->rho_star);  \
+    else                                                                                                     \
+        k_nonpressure<M, false><<<nb, kNpThreads, 0, s->stream>>>(s->sc, st, t, s->posA, s->velA, s->rho, s->xq, \
+                                                                  s->velB, s->force, s->xstar, s->rho_star)
     if (mode == 2) {
         BBX_PROF_BEGIN("nonpressure_warm");
         BBX_NP(2);
@@ -677,7 +697,7 @@ int run_predict_pressure(bbx_solver *s, const StepConst &st, int k) {
     // the pressure increment uses the host's FP64 delta (s->delta64)
     BBX_PROF_BEGIN_IT("predict_pressure", k);
     k_predict_pressure<<<nblocks(s->n), kPpThreads, 0, s->stream>>>(s->sc, st, s->delta64, nbr_tab(s), s->xstar,
-                                                                s->posA, s->pres, s->rho_star, s->xq,
+                                                                s->pres, s->rho_star, s->xq,
                                                                 s->loop, k);
     BBX_HIP_CHECK(hipGetLastError());
     BBX_PROF_END();
@@ -688,7 +708,7 @@ int run_pressure_force(bbx_solver *s, const StepConst &st, int k, int max_it, in
     if (s->n == 0) return BBX_OK;
     if (k >= kMaxIt || max_it > kMaxIt) return fail(BBX_E_INVALID, "iteration index out of range");
     BBX_PROF_BEGIN_IT("pressure_force", k < 0 ? -1 : k);
-    k_pressure_force<<<nblocks(s->n), kBlock, 0, s->stream>>>(
+    (s->ncoll ? k_pressure_force<true> : k_pressure_force<false>)<<<nblocks(s->n), kBlock, 0, s->stream>>>(
         s->sc, st, nbr_tab(s), s->posA, s->velA, s->force, s->xq, s->pres, s->xstar, s->fp, s->posB,
         s->velB, s->flag, s->max_force, s->loop, k < 0 ? -1 : k, max_it, exact, tol, s->d_signal,
         s->loop_seq & 0x7fffffu, s->counters);
@@ -710,7 +730,7 @@ int run_sph_force(bbx_solver *s) {
 int run_integrate(bbx_solver *s, const StepConst &st) {
     if (s->n == 0) return BBX_OK;
     BBX_PROF_BEGIN("integrate");
-    k_integrate<<<nblocks(s->n), kBlock, 0, s->stream>>>(s->sc, st, s->posA, s->velA, s->force,
+    (s->ncoll ? k_integrate<true> : k_integrate<false>)<<<nblocks(s->n), kBlock, 0, s->stream>>>(s->sc, st, s->posA, s->velA, s->force,
                                                          s->posB, s->velB, s->flag, s->max_force);
     BBX_HIP_CHECK(hipGetLastError());
     BBX_PROF_END();

@@ -80,6 +80,13 @@ __device__ __forceinline__ int tab_local(const TileTab &t, int j) {
 // A staged tile's bucket entries are LDS byte offsets (slot << kSlotShift,
 // slot < kTileCap, so they fit 16 bits): a gather adds no shift per entry.
 constexpr int kSlotShift = 4;  // 16-byte slots
+// Unused entries of a staged bucket's last quad name a slot of their own,
+// where every gather keeps a particle so far away that its kernel factor
+// clamps to zero: the pair arithmetic needs no test for them.
+constexpr int kFarSlot = kTileCap;
+constexpr unsigned kFarEntry = (unsigned)kFarSlot << kSlotShift;
+static_assert(kFarEntry < 65536u, "entries are 16 bits");
+__device__ __forceinline__ float4 far_particle(float w) { return make_float4(1e15f, 1e15f, 1e15f, w); }
 __device__ __forceinline__ float4 lds_at(const float4 *base, int byte_off) {
     return *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(base) + byte_off);
 }
@@ -265,13 +272,14 @@ __device__ __forceinline__ NbrQuads<D> nbr_prefetch(const unsigned short *__rest
 // The four entries of one (unpacked) quad go through body(j, live) without
 // branches; live = false for an entry at or past the bucket count.  Every
 // slot of a quad the walk reaches holds a valid index: the bucket build
-// zero-fills the unused slots of a bucket's last quad, and index 0 is valid
-// in either index space.  So by default a dead entry keeps its slot's index
-// (no select per entry); with kSelect it gets `dead` instead (the particle's
-// own index: a sum over x_j - x_i then gets exact zeros from dead entries
-// unmasked).  Straight-line code lets the four entries' neighbour loads
-// issue together instead of one load-wait per entry.  The body must make a
-// dead entry contribute nothing (or an exact zero).
+// fills the unused slots of a bucket's last quad with kFarEntry (staged
+// tiles) or index 0 (storage indices).  So by default a dead entry keeps its
+// slot's index (no select per entry); with kSelect it gets `dead` instead
+// (the particle's own index: a sum over x_j - x_i then gets exact zeros from
+// dead entries unmasked).  Straight-line code lets the four entries'
+// neighbour loads issue together instead of one load-wait per entry.  The
+// body must make a dead entry contribute an exact zero; reading LDS slots, it
+// need not look at `live`.
 template <bool kSelect, typename Body>
 __device__ __forceinline__ void quad_body(const int4 &v, int k, int cnt, Body &body, int dead) {
     const int rem = cnt - k;  // entries of the bucket from this quad on

@@ -1,10 +1,10 @@
 """The bucket build's two kernels: four lanes per particle for small sets (up
-to 98,304 particles) and one lane per particle above.
+to 65,536 particles) and one lane per particle above.
 
 Buckets are exact against the FP64 oracle.  A density is an FP32 sum of at
 most 100 non-negative terms with compensation; each term has a few roundings
 of 2^-24, so 2e-6 relative bounds it (the tolerance of the other parity
-tests), and twice that bounds the difference of two sums in another order."""
+tests).  Both kernels add the same terms in the same order."""
 import dataclasses
 
 import numpy as np
@@ -51,9 +51,9 @@ def test_split_buckets_match_oracle(bbx, oracle, n, spacing):
 
 
 def test_both_kernels_agree_at_the_boundary(bbx):
-    """98,304 particles take the split kernel; the same with one more, far
+    """65,536 particles take the split kernel; the same with one more, far
     away, the other: the same buckets, features and network pressures."""
-    p = _points(98304, 0.01)
+    p = _points(65536, 0.01)
     extra = np.array([[0.9, 0.4, 0.9]], dtype=np.float32).astype(np.float64)
     assert np.abs(p).max() < 0.5
     res = []
@@ -64,25 +64,19 @@ def test_both_kernels_agree_at_the_boundary(bbx):
         s.distribute()
         counts, ids = s.buckets()
         s.pcisph_substep(5e-4, 1, 0.01, bbx.MODE_TEXTBOOK, bbx.WARM_MLP)
-        res.append([x[:98304] for x in (counts, ids, s.get("density"), s.get("features"), s.get("warm_pressure"))])
+        res.append([x[:65536] for x in (counts, ids, s.get("density"), s.get("features"), s.get("warm_pressure"))])
         s.close()
     a, b = res
     assert_buckets_equal((a[0], a[1]), (b[0], b[1]))
-    np.testing.assert_allclose(a[2], b[2], rtol=4e-6)
-    # sums of ~30 terms of order one in another order
-    np.testing.assert_allclose(a[3], b[3], rtol=1e-5, atol=2e-5)
-    # the network sees its features rounded to BF16: a feature at a rounding
-    # boundary moves by 2^-8 of its value
-    scale = np.abs(b[4]).max()
-    assert np.abs(a[4] - b[4]).max() <= 2e-2 * scale + 1e-12
-    assert np.abs(a[4] - b[4]).mean() <= 1e-4 * scale + 1e-12
+    for x, y in zip(a[2:], b[2:]):  # the same sums in the same order
+        np.testing.assert_array_equal(x, y)
 
 
 @pytest.mark.parametrize("env", [{"BBX_TILE_CAP": "0"}, {"BBX_TILE_CAP": "1500", "BBX_TILE_CAP2": "900"},
                                  {"BBX_BUCKET_ROW_MAX": "0"}, {"BBX_BUCKET_ROW_MAX": "20"}])
 def test_large_set_routes_bit_identical(bbx, monkeypatch, env):
     """Staged and unstaged tiles, row masks and cell walks above the boundary."""
-    sc = _scene(_points(99000, 0.01))
+    sc = _scene(_points(66000, 0.01))
     res = []
     for k in range(2):
         if k:
