@@ -627,7 +627,6 @@ int bbx_solver_setup(bbx_solver *s) {
     BBX_CHECK(check_solver(s));
     BBX_CHECK(compute_mass_and_delta(s));
     fill_sim_const(s);
-    BBX_CHECK(launch_fill_int(s, s->counters, 0, CNT_N));
     // full distribution into ascending-id chains; buckets come with the first substep
     BBX_CHECK(distribute(s, true, false, false));
     BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
@@ -823,7 +822,6 @@ int bbx_solver_append(bbx_solver *s, const double *pos, const double *vel, int c
     fill_sim_const(s);
     // DistributeByParticleList (src/core/grid.h:358-387): each new particle
     // goes to the tail of its cell's chain; buckets come with the next substep
-    BBX_CHECK(launch_fill_int(s, s->counters, 0, CNT_N));
     BBX_CHECK(distribute(s, false, false, false, n0));
     BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
     return BBX_OK;
@@ -930,7 +928,6 @@ static int read_stats(bbx_solver *s, bbx_stats *st, int loop_len = 0) {
 
 int bbx_grid_distribute(bbx_solver *s, bbx_stats *stats) {
     BBX_CHECK(check_setup(s));
-    BBX_CHECK(launch_fill_int(s, s->counters, 0, CNT_N));
     BBX_CHECK(distribute(s, false, true, s->kind == BBX_SPH));
     if (stats) std::memset(stats, 0, sizeof(*stats));
     BBX_CHECK(read_stats(s, stats));
@@ -997,11 +994,8 @@ int bbx_grid_set_chains(bbx_solver *s, const int *cell_start, const int *members
         BBX_HIP_CHECK(hipMemcpy(s->cellA, ncell.data(), sizeof(int) * n, hipMemcpyHostToDevice));
     }
     // cell table for the new order (buckets are rebuilt by the next distribute)
-    std::vector<int> cnt(total + 1, 0), st(total + 1, 0);
-    for (unsigned c = 0; c < total; c++) cnt[c] = cell_start[c + 1] - cell_start[c];
-    cnt[total] = s->n - in_chains;
+    std::vector<int> st(total + 1, 0);
     for (unsigned c = 0; c <= total; c++) st[c] = c < total ? cell_start[c] : in_chains;
-    BBX_HIP_CHECK(hipMemcpy(s->cell_count, cnt.data(), sizeof(int) * (total + 1), hipMemcpyHostToDevice));
     BBX_HIP_CHECK(hipMemcpy(s->cell_start, st.data(), sizeof(int) * (total + 1), hipMemcpyHostToDevice));
     s->setup_done = true;
     return BBX_OK;
@@ -1213,8 +1207,7 @@ static int check_substep(bbx_solver *s, double dt, int max_it, int warm) {
 static int substep_front(bbx_solver *s, hipEvent_t start) {
     s->maxf_cached = false;
     if (start) BBX_HIP_CHECK(hipEventRecord(start, s->stream));
-    // the step block is cleared by the launch that clears the cell counts
-    return distribute_grid(s, false, -1, (int *)s->step, sizeof(StepBlock) / sizeof(int));
+    return distribute_grid(s, false, -1, (int *)s->max_force, kStepClear);
 }
 
 struct SubstepPlan {
@@ -1514,8 +1507,8 @@ int bbx_sph_substep(bbx_solver *s, double dt, bbx_stats *stats) {
     if (!(dt > 0)) return fail(BBX_E_INVALID, "dt must be > 0");
     s->maxf_cached = false;
     BBX_HIP_CHECK(hipEventRecord(s->ev0[0], s->stream));
-    BBX_CHECK(launch_fill_int(s, (int *)s->step, 0, sizeof(StepBlock) / sizeof(int)));
-    BBX_CHECK(distribute(s, false, true, true));
+    BBX_CHECK(distribute_grid(s, false, -1, (int *)s->max_force, kStepClear));
+    BBX_CHECK(build_buckets(s, true, 0, nullptr));
     StepConst st{};
     st.dt = (float)dt;
     st.dt_over_m = (float)(dt / s->mass);
@@ -1578,7 +1571,6 @@ int bbx_pcisph_harvest(bbx_solver *s, double dt, int max_it, double tol, float *
     // with feature output, then the plain substep from the same state.
     // The features are computed on a throwaway pass that leaves the state
     // untouched (distribute is idempotent for unchanged positions).
-    BBX_CHECK(launch_fill_int(s, s->counters, 0, CNT_N));
     const double delta = compute_delta(s, dt);
     StepConst st{};
     st.dt = (float)dt;

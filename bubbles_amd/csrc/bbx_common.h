@@ -156,12 +156,11 @@ enum {
     CNT_OVERFLOW = 0,   // bucket inserts dropped by the cap
     CNT_LOST = 1,       // particles in no chain
     CNT_FULL = 2,       // last distribution was a full pass
-    CNT_BAD_HASH = 3,   // points hashing outside the grid
     CNT_N = 8
 };
 
-// The per-substep device state in one allocation: cleared by one fill at the
-// start of a substep and read back by one copy (the first kStepReadback
+// The per-substep device state in one allocation: cleared by the grid pass at
+// the start of a substep and read back by one copy (the first kStepReadback
 // bytes: counters, max-force slots, the loop's per-iteration errors and done
 // flags); the per-slot error maxima follow.
 struct StepBlock {
@@ -170,7 +169,10 @@ struct StepBlock {
     LoopState loop;
 };
 constexpr size_t kStepReadback = offsetof(StepBlock, loop) + offsetof(LoopState, slot);
-static_assert(sizeof(StepBlock) % sizeof(int) == 0, "StepBlock is cleared as ints");
+// what a substep clears: all behind the counters, as ints
+constexpr size_t kStepClear = (sizeof(StepBlock) - offsetof(StepBlock, max_force)) / sizeof(int);
+static_assert(sizeof(StepBlock) % sizeof(int) == 0 && offsetof(StepBlock, max_force) == CNT_N * sizeof(int),
+              "StepBlock is cleared as ints");
 
 // ---------------------------------------------------------------------------
 // kernel profiler (HIP events on the solver stream)
@@ -253,6 +255,7 @@ struct bbx_solver {
     int *home = nullptr;                       // hashed cell (neighbour lookups)
     // cell table (total + 1 entries, the last one collects particles in no chain)
     int *cell_count = nullptr, *cell_start = nullptr;
+    bool counts_clear = false;                 // cell_count is all zeros (k_scatter leaves it so)
     int *scan_tmp = nullptr;
     size_t scan_tmp_elems = 0;
     // sort scratch (indexed by old slot / new position)
@@ -328,10 +331,10 @@ int distribute(bbx_solver *s, bool force_full, bool buckets, bool with_pressure,
                int feat_mode = 0, const StepConst *st = nullptr);
 // the two halves of distribute: the grid (hash, scan, scatter, move) and the
 // tile tables + bucket build (the latter is where the warm start is chosen)
-// clear2 / clear2_n: a second int range set to zero by the same launch that
-// clears the cell counts (the substep's step block)
-int distribute_grid(bbx_solver *s, bool force_full, int append_from, int *clear2 = nullptr,
-                    size_t clear2_n = 0);
+// clear / clear_n: an int range set to zero on the way (the substep's step
+// block behind its counters, which this sets)
+int distribute_grid(bbx_solver *s, bool force_full, int append_from, int *clear = nullptr,
+                    size_t clear_n = 0);
 int build_buckets(bbx_solver *s, bool with_pressure, int feat_mode, const StepConst *st);
 int run_density_only(bbx_solver *s);
 // mode: 0 force only, 1 force + predict(k = 0), 2 force + the warm start's

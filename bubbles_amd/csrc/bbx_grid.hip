@@ -18,6 +18,8 @@
 // (DistributeToCellOpt) concatenates the 27 neighbour cells' old chains in
 // (y,x,z) order, i.e. key = (direction of the old cell seen from the new cell,
 // old storage slot), since storage is the old chain order.
+#include <algorithm>
+
 #include "bbx_mlp_device.h"
 #include "bbx_tile.h"
 
@@ -71,27 +73,6 @@ int launch_init_fields(bbx_solver *s) {
     k_init_fields<<<dim3((unsigned)blocks), dim3(kBlock), 0, s->stream>>>(
         n, (int)s->grid.total, s->force, s->fp, s->xstar, s->xq, s->rho, s->pres, s->rho_star, s->feat, s->nbr_cnt,
         s->cellA, s->home, s->tile_tab, ntab);
-    BBX_HIP_CHECK(hipGetLastError());
-    return BBX_OK;
-}
-
-// two int ranges set to zero by one launch: blocks [0, nb0) cover a, the
-// rest cover b
-__global__ void k_zero_int2(int *__restrict__ a, size_t na, size_t nb0, int *__restrict__ b, size_t nb) {
-    const size_t blk = blockIdx.x;
-    if (blk < nb0) {
-        const size_t i = blk * blockDim.x + threadIdx.x;
-        if (i < na) a[i] = 0;
-    } else {
-        const size_t i = (blk - nb0) * blockDim.x + threadIdx.x;
-        if (i < nb) b[i] = 0;
-    }
-}
-
-static int launch_zero_int2(bbx_solver *s, int *a, size_t na, int *b, size_t nb) {
-    if (!b || nb == 0) return launch_fill_int(s, a, 0, na);
-    const size_t ba = (na + kBlock - 1) / kBlock, bb = (nb + kBlock - 1) / kBlock;
-    k_zero_int2<<<dim3((unsigned)(ba + bb)), dim3(kBlock), 0, s->stream>>>(a, na, ba, b, nb);
     BBX_HIP_CHECK(hipGetLastError());
     return BBX_OK;
 }
@@ -173,6 +154,50 @@ __global__ void __launch_bounds__(kBlock) k_scan_add_reduce(int *__restrict__ ou
     }
 }
 
+// The whole scan in one launch for few blocks: every workgroup sums what
+// lies before its own elements itself (at most 30k ints) instead of a second
+// launch that adds block totals (4.0 + 3.0 us for 9k cells, 4.5 now).
+constexpr int kScanOneLaunch = 16;  // blocks
+__global__ void __launch_bounds__(kBlock) k_scan_small(const int *__restrict__ in, int *__restrict__ out, size_t n) {
+    __shared__ int before[kBlock / 64], wave_tot[kBlock / 64];
+    const size_t base = (size_t)blockIdx.x * kBlock * kScanItems;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int v[kScanItems], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kScanItems; k++) {
+        const size_t i = base + (size_t)threadIdx.x * kScanItems + k;
+        v[k] = i < n ? in[i] : 0;
+        sum += v[k];
+    }
+    int part = 0;
+    const int4 *in4 = reinterpret_cast<const int4 *>(in);  // base is a multiple of 4
+    const int lim = (int)(base / 4);
+    for (int t = (int)threadIdx.x; t < lim; t += 8 * kBlock) {
+        int4 q[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) q[k] = in4[min(t + k * kBlock, lim - 1)];
+#pragma unroll
+        for (int k = 0; k < 8; k++) part += t + k * kBlock < lim ? q[k].x + q[k].y + q[k].z + q[k].w : 0;
+    }
+    for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
+    int incl = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += o;
+    }
+    if (lane == 63) wave_tot[wave] = incl;
+    if (lane == 0) before[wave] = part;
+    __syncthreads();
+    int run = incl - sum;
+    for (int w = 0; w < kBlock / 64; w++) run += before[w] + (w < wave ? wave_tot[w] : 0);
+#pragma unroll
+    for (int k = 0; k < kScanItems; k++) {
+        const size_t i = base + (size_t)threadIdx.x * kScanItems + k;
+        if (i < n) out[i] = run;
+        run += v[k];
+    }
+}
+
 // Exclusive scan, recursive over block totals.  Needs scan_tmp sized by
 // scan_scratch_elems(n).
 static size_t blocks_for(size_t n) { return (n + (size_t)kBlock * kScanItems - 1) / ((size_t)kBlock * kScanItems); }
@@ -207,6 +232,12 @@ static int scan_rec(bbx_solver *s, const int *in, int *out, size_t n, int *tmp) 
 
 int launch_scan(bbx_solver *s, const int *in, int *out, size_t n) {
     if (n == 0) return BBX_OK;
+    const size_t b = blocks_for(n);
+    if (b <= (size_t)kScanOneLaunch) {
+        k_scan_small<<<dim3((unsigned)b), dim3(kBlock), 0, s->stream>>>(in, out, n);
+        BBX_HIP_CHECK(hipGetLastError());
+        return BBX_OK;
+    }
     if (scan_scratch_elems(n) > s->scan_tmp_elems) return fail(BBX_E_RANGE, "scan scratch too small");
     return scan_rec(s, in, out, n, s->scan_tmp);
 }
@@ -231,8 +262,7 @@ __global__ void __launch_bounds__(kBlock) k_hash(SimConst c, const float4 *__res
                                                  int *__restrict__ newc, int *__restrict__ hcell,
                                                  unsigned long long *__restrict__ key,
                                                  int *__restrict__ count,
-                                                 int *__restrict__ rank_tmp,
-                                                 int *__restrict__ counters) {
+                                                 int *__restrict__ rank_tmp) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     const int none = (int)c.g.total;
     const bool valid = s < c.n;
@@ -283,7 +313,6 @@ __global__ void __launch_bounds__(kBlock) k_hash(SimConst c, const float4 *__res
     if (head && valid) base = atomicAdd(&count[nc], next_head - lane);
     base = __shfl(base, head_lane, 64);
     if (!valid) return;
-    if (bad) atomicAdd(&counters[CNT_BAD_HASH], 1);
     newc[s] = nc;
     // a point outside the grid has no home cell: its bucket stays empty
     hcell[s] = bad ? -1 : cid;
@@ -294,24 +323,31 @@ __global__ void __launch_bounds__(kBlock) k_hash(SimConst c, const float4 *__res
 // ---------------------------------------------------------------------------
 // 3. scatter into cell segments (arrival order), record full/lost stats
 // ---------------------------------------------------------------------------
+// The cell counts have been read for the last time: this launch also leaves
+// them at zero for the next pass, and clears `clear` (a substep's step block
+// behind its counters), which took a launch of their own (4.2 us at 1M).
 __global__ void __launch_bounds__(kBlock) k_scatter(SimConst c, const int *__restrict__ newc,
                                                     const int *__restrict__ rank_tmp,
                                                     const int *__restrict__ start,
-                                                    const int *__restrict__ count,
+                                                    int *__restrict__ count, size_t cells,
                                                     int *__restrict__ tmp_idx,
                                                     int *__restrict__ flag, int force_full,
-                                                    int append,
-                                                    int *__restrict__ counters) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s == 0) {
-        counters[CNT_LOST] = count[c.g.total];
+                                                    int append, int *__restrict__ counters,
+                                                    int *__restrict__ clear, size_t clear_n) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0) {
+        counters[CNT_OVERFLOW] = 0;
+        counters[CNT_LOST] = c.n - start[c.g.total];
         if (!append) {  // an append leaves the higher-level flag to the next substep
             counters[CNT_FULL] = (force_full || *flag) ? 1 : 0;
             *flag = 0;  // ResetHigherLevel
+        } else {
+            counters[CNT_FULL] = 0;
         }
     }
-    if (s >= c.n) return;
-    tmp_idx[start[newc[s]] + rank_tmp[s]] = s;
+    if (t < cells) count[t] = 0;
+    if (t < clear_n) clear[t] = 0;
+    if (t < (size_t)c.n) tmp_idx[start[newc[t]] + rank_tmp[t]] = (int)t;
 }
 
 // ---------------------------------------------------------------------------
@@ -329,7 +365,6 @@ __global__ void __launch_bounds__(kBlock) k_rank_move(SimConst c, const int *__r
                                                       const int *__restrict__ hcell,
                                                       const unsigned long long *__restrict__ key,
                                                       const int *__restrict__ start,
-                                                      const int *__restrict__ count,
                                                       const float4 *__restrict__ pos_in,
                                                       const float4 *__restrict__ vel_in,
                                                       float4 *__restrict__ pos_out,
@@ -344,7 +379,8 @@ __global__ void __launch_bounds__(kBlock) k_rank_move(SimConst c, const int *__r
     const int cc = valid ? newc[s] : -1;
     const unsigned long long k = valid ? key[s] : 0ull;
     const int b = valid ? start[cc] : 0;
-    const int e = valid ? b + count[cc] : 0;
+    const int total = (int)c.g.total;  // start[total]: the particles in no chain, up to n
+    const int e = valid ? (cc < total ? start[cc + 1] : c.n) : 0;
     // thread 0 is valid in every launched workgroup (the grid is ceil(n / kBlock))
     if (threadIdx.x == 0) cell0 = cc;
     // Thread t holds the key of storage slot t, so the keys of the cell
@@ -356,7 +392,7 @@ __global__ void __launch_bounds__(kBlock) k_rank_move(SimConst c, const int *__r
     const bool uniform = __syncthreads_and(!valid || cc == cell0) != 0;
     const int c0 = cell0;
     const int bb = uniform ? start[c0] : 0;
-    const int ee = uniform ? bb + count[c0] : 0;
+    const int ee = uniform ? (c0 < total ? start[c0 + 1] : c.n) : 0;
     int rank = 0;
     if (uniform && ee - bb > kRankLds) {
         // every valid thread has [b, e) == [bb, ee); the trip count and the
@@ -396,18 +432,14 @@ __global__ void __launch_bounds__(kBlock) k_rank_move(SimConst c, const int *__r
 // particle is one of those, cmin and cmax are the homes of its first and
 // last particles (otherwise a wave reduction over the tile finds them).  The
 // row ranges of lanes 0-8 are gathered by shuffles and merged by lane 0.
-constexpr int kTabWaves = kBlock / 64;
-__global__ void __launch_bounds__(kBlock) k_tile_tables(SimConst c, const int *__restrict__ home,
-                                                        const int *__restrict__ start, int ntiles,
-                                                        int *__restrict__ tile_tab) {
-    __shared__ TileTab tt[kTabWaves];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int tile = blockIdx.x * kTabWaves + w;  // wave-uniform
-    if (tile >= ntiles) return;
+// (one wave; lane 0's table is complete when the wave has synchronised)
+__device__ __forceinline__ void tile_table(const SimConst &c, const int *__restrict__ home,
+                                           const int *__restrict__ start, int tile, int lane, TileTab &tt) {
     const int t0 = tile * kBlock, t1 = min(t0 + kBlock, c.n) - 1;
     int lo = 0x7fffffff, hi = home[t1];
+    const int first = home[t0];
     if (hi >= 0) {
-        lo = home[t0];
+        lo = first;
     } else {
 #pragma unroll
         for (int k = 0; k < kBlock / 64; k++) {
@@ -429,7 +461,18 @@ __global__ void __launch_bounds__(kBlock) k_tile_tables(SimConst c, const int *_
         ra[r] = __shfl(a, r, 64);
         rb[r] = __shfl(b, r, 64);
     }
-    if (lane == 0 && !tab_merge_ordered(ra, rb, c.tile_cap, tt[w])) tab_merge(ra, rb, c.tile_cap, tt[w]);
+    if (lane == 0 && !tab_merge_ordered(ra, rb, c.tile_cap, tt)) tab_merge(ra, rb, c.tile_cap, tt);
+}
+
+constexpr int kTabWaves = kBlock / 64;
+__global__ void __launch_bounds__(kBlock) k_tile_tables(SimConst c, const int *__restrict__ home,
+                                                        const int *__restrict__ start, int ntiles,
+                                                        int *__restrict__ tile_tab) {
+    __shared__ TileTab tt[kTabWaves];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int tile = blockIdx.x * kTabWaves + w;  // wave-uniform
+    if (tile >= ntiles) return;
+    tile_table(c, home, start, tile, lane, tt[w]);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -965,7 +1008,7 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density_split(SimConst c,
                                                                   int *__restrict__ nbr_cnt,
                                                                   float *__restrict__ rho,
                                                                   float *__restrict__ pres,
-                                                                  const int *__restrict__ tile_tab,
+                                                                  int *__restrict__ tile_tab,
                                                                   int *__restrict__ counters,
                                                                   WarmIn wi) {
     __shared__ float4 sx[kTileCap + 8];
@@ -973,7 +1016,6 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density_split(SimConst c,
     __shared__ TileTab tt;
     const int unit = tile_of_block();
     const int tile = unit / kSplitLanes, part = unit % kSplitLanes;
-    const int tw = tab_load_wave(tile_tab + (size_t)tile * kTabInts);
     const int pl = threadIdx.x / kSplitLanes, sub = threadIdx.x % kSplitLanes;
     const int i = tile * kBlock + part * kSplitRows + pl;
     const bool valid = i < c.n;
@@ -1000,9 +1042,14 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density_split(SimConst c,
             for (int q = 0; q < 4; q++) b[k][q] = start[min(max(cx - 1 + q, 0), last)];
         }
     }
-    if (threadIdx.x < kTabWords) reinterpret_cast<int *>(&tt)[threadIdx.x] = tw;
-    const bool staged = tab_word(tw, 1) != 0;
-    if (staged) tab_stage_dma_wave(tw, [&](int j, int e) { lds_dma16(pos + j, sx + e); });
+    // The tile's table, by the first wave while the loads above are under way
+    // (a kernel of its own takes 4.9 us); the later gathers read it from the
+    // first part's copy.
+    if (threadIdx.x < 64) tile_table(c, home, start, tile, (int)threadIdx.x, tt);
+    __syncthreads();
+    const bool staged = tt.staged != 0;
+    if (staged) tab_stage_dma(tt, [&](int j, int e) { lds_dma16(pos + j, sx + e); });
+    if (part == 0) tab_store(tile_tab + (size_t)tile * kTabInts, tt);
     if (hc >= 0) {
 #pragma unroll
         for (int k = 0; k < 3; k++) {
@@ -1232,50 +1279,54 @@ __global__ void __launch_bounds__(kBlock) k_density(SimConst c, const float4 *__
 static unsigned nblocks(int n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
 // UpdateGridDistribution: full or incremental chain update, then buckets.
-int distribute_grid(bbx_solver *s, bool force_full, int append_from, int *clear2, size_t clear2_n) {
+int distribute_grid(bbx_solver *s, bool force_full, int append_from, int *clear, size_t clear_n) {
     SimConst &c = s->sc;
     const int n = s->n;
     const size_t cells = (size_t)c.g.total + 1;
-    BBX_CHECK(launch_zero_int2(s, s->cell_count, cells, clear2, clear2_n));
-    if (n > 0) {
-        {
-            BBX_PROF_BEGIN("grid_hash");
-            k_hash<<<nblocks(n), kBlock, 0, s->stream>>>(c, s->posA, s->cellA, s->flag,
-                                                         force_full ? 1 : 0, append_from, s->newc,
-                                                         s->hash_tmp, s->key, s->cell_count,
-                                                         s->rank_tmp, s->counters);
-            BBX_HIP_CHECK(hipGetLastError());
-            BBX_PROF_END();
-        }
-        {
-            BBX_PROF_BEGIN("grid_scan");
-            BBX_CHECK(launch_scan(s, s->cell_count, s->cell_start, cells));
-            BBX_PROF_END();
-        }
-        {
-            BBX_PROF_BEGIN("grid_scatter");
-            k_scatter<<<nblocks(n), kBlock, 0, s->stream>>>(c, s->newc, s->rank_tmp,
-                                                            s->cell_start, s->cell_count,
-                                                            s->tmp_idx, s->flag,
-                                                            force_full ? 1 : 0, append_from >= 0 ? 1 : 0,
-                                                            s->counters);
-            BBX_HIP_CHECK(hipGetLastError());
-            BBX_PROF_END();
-        }
-        {
-            BBX_PROF_BEGIN("grid_rank_move");
-            k_rank_move<<<nblocks(n), kBlock, 0, s->stream>>>(c, s->tmp_idx, s->newc,
-                                                              s->hash_tmp, s->key,
-                                                              s->cell_start, s->cell_count,
-                                                              s->posA, s->velA, s->posB,
-                                                              s->velB, s->cellB, s->home);
-            BBX_HIP_CHECK(hipGetLastError());
-            BBX_PROF_END();
-        }
-        std::swap(s->posA, s->posB);
-        std::swap(s->velA, s->velB);
-        std::swap(s->cellA, s->cellB);
+    if (n == 0) {
+        BBX_CHECK(launch_fill_int(s, s->counters, 0, CNT_N));
+        return clear_n ? launch_fill_int(s, clear, 0, clear_n) : BBX_OK;
     }
+    // k_scatter leaves the counts at zero; not so before the first pass, or
+    // behind one that did not get that far
+    if (!s->counts_clear) BBX_CHECK(launch_fill_int(s, s->cell_count, 0, cells));
+    s->counts_clear = false;
+    {
+        BBX_PROF_BEGIN("grid_hash");
+        k_hash<<<nblocks(n), kBlock, 0, s->stream>>>(c, s->posA, s->cellA, s->flag,
+                                                     force_full ? 1 : 0, append_from, s->newc,
+                                                     s->hash_tmp, s->key, s->cell_count,
+                                                     s->rank_tmp);
+        BBX_HIP_CHECK(hipGetLastError());
+        BBX_PROF_END();
+    }
+    {
+        BBX_PROF_BEGIN("grid_scan");
+        BBX_CHECK(launch_scan(s, s->cell_count, s->cell_start, cells));
+        BBX_PROF_END();
+    }
+    {
+        const size_t items = std::max({(size_t)n, cells, clear_n});
+        BBX_PROF_BEGIN("grid_scatter");
+        k_scatter<<<(unsigned)((items + kBlock - 1) / kBlock), kBlock, 0, s->stream>>>(
+            c, s->newc, s->rank_tmp, s->cell_start, s->cell_count, cells, s->tmp_idx, s->flag, force_full ? 1 : 0,
+            append_from >= 0 ? 1 : 0, s->counters, clear, clear_n);
+        BBX_HIP_CHECK(hipGetLastError());
+        s->counts_clear = true;
+        BBX_PROF_END();
+    }
+    {
+        BBX_PROF_BEGIN("grid_rank_move");
+        k_rank_move<<<nblocks(n), kBlock, 0, s->stream>>>(c, s->tmp_idx, s->newc,
+                                                          s->hash_tmp, s->key, s->cell_start,
+                                                          s->posA, s->velA, s->posB,
+                                                          s->velB, s->cellB, s->home);
+        BBX_HIP_CHECK(hipGetLastError());
+        BBX_PROF_END();
+    }
+    std::swap(s->posA, s->posB);
+    std::swap(s->velA, s->velB);
+    std::swap(s->cellA, s->cellB);
     return BBX_OK;
 }
 
@@ -1286,7 +1337,7 @@ int build_buckets(bbx_solver *s, bool with_pressure, int feat_mode, const StepCo
     SimConst &c = s->sc;
     const int n = s->n;
     if (n > 0) {
-        {
+        if (n > kSmallSet) {  // smaller sets' bucket kernel makes its own
             BBX_PROF_BEGIN("tile_tables");
             k_tile_tables<<<(unsigned)((s->ntiles + kTabWaves - 1) / kTabWaves), kBlock, 0, s->stream>>>(
                 c, s->home, s->cell_start, s->ntiles, s->tile_tab);
