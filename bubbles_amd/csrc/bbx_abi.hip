@@ -392,7 +392,7 @@ static void free_all(bbx_solver *s) {
     dfree(s->cell_count); dfree(s->cell_start); dfree(s->scan_tmp);
     dfree(s->key); dfree(s->newc); dfree(s->rank_tmp); dfree(s->tmp_idx); dfree(s->hash_tmp);
     dfree(s->nbr16); dfree(s->nbr32); dfree(s->nbr_cnt); dfree(s->tile_tab);
-    dfree(s->rho); dfree(s->pres); dfree(s->rho_star); dfree(s->xq);
+    dfree(s->rho); dfree(s->pres); dfree(s->rho_star); dfree(s->xq); dfree(s->vr);
     dfree(s->force); dfree(s->fp); dfree(s->xstar); dfree(s->feat); dfree(s->pwarm);
     dfree(s->step); dfree(s->flag);
     s->loop = nullptr; s->max_force = nullptr; s->counters = nullptr;
@@ -538,6 +538,7 @@ int bbx_solver_create(int kind, const bbx_params *params, const double *pos, con
     if (!rc) rc = dalloc(&s->pres, N);
     if (!rc) rc = dalloc(&s->rho_star, N);
     if (!rc) rc = dalloc(&s->xq, N);
+    if (!rc && kind == BBX_SPH) rc = dalloc(&s->vr, N);
     if (!rc) rc = dalloc(&s->force, N);
     if (!rc) rc = dalloc(&s->fp, N);
     if (!rc) rc = dalloc(&s->xstar, N);
@@ -752,6 +753,7 @@ int bbx_solver_reserve(bbx_solver *s, int capacity) {
     BBX_CHECK(regrow(s, s->pwarm, S1, n));
     BBX_CHECK(regrow(s, s->posB, S1, 0));
     BBX_CHECK(regrow(s, s->velB, S1, 0));
+    if (s->vr) BBX_CHECK(regrow(s, s->vr, S1, 0));
     BBX_CHECK(regrow(s, s->cellB, S1, 0));
     BBX_CHECK(regrow(s, s->key, S1, 0));
     BBX_CHECK(regrow(s, s->newc, S1, 0));
@@ -1501,33 +1503,72 @@ int bbx_pcisph_advance(bbx_solver *s, double interval, int max_it, double tol, i
     return BBX_OK;
 }
 
-int bbx_sph_substep(bbx_solver *s, double dt, bbx_stats *stats) {
+}  // extern "C"
+// Words of the signal block that carry the current substep's number; true
+// once all `count` do.
+static bool signal_words(const bbx_solver *s, const int *which, int count, unsigned *out) {
+    const unsigned want = s->loop_seq & 0x7fffffu;
+    for (int q = 0; q < count; q++) {
+        const unsigned long long v = __atomic_load_n(&s->h_signal->stats[which[q]], __ATOMIC_ACQUIRE);
+        if ((unsigned)(v >> 32) != want) return false;
+        out[q] = (unsigned)v;
+    }
+    return true;
+}
+
+// The statistics and the largest force that the SPH step published: the host
+// spins on them, and it is an error if the stream drains without them.
+static int published_sph(bbx_solver *s, bbx_stats *st) {
+    const int which[4] = {PUB_OVERFLOW, PUB_LOST, PUB_FULL, PUB_MAXF};
+    unsigned w[4];
+    for (unsigned spin = 1; !signal_words(s, which, 4, w); spin++) {
+        if ((spin & 4095u) != 0u) continue;
+        const hipError_t q = hipStreamQuery(s->stream);
+        if (q == hipErrorNotReady) continue;
+        BBX_HIP_CHECK(q);
+        if (signal_words(s, which, 4, w)) break;
+        return fail(BBX_E_HIP, "the substep's statistics were not published");
+    }
+    st->bucket_overflows = (int)w[0];
+    st->lost_particles = (int)w[1];
+    st->full_redistribution = (int)w[2];
+    for (int k = 0; k < kSlots; k++) s->h_max_force[k] = k ? 0u : w[3];
+    return BBX_OK;
+}
+
+// timed: also measure the substep's device time, and return when it has
+// ended; without it the substep's last launch may still be running
+static int sph_substep(bbx_solver *s, double dt, bbx_stats *stats, bool timed) {
     BBX_CHECK(check_setup(s));
     if (s->kind != BBX_SPH) return fail(BBX_E_INVALID, "not an SPH solver");
     if (!(dt > 0)) return fail(BBX_E_INVALID, "dt must be > 0");
     s->maxf_cached = false;
-    BBX_HIP_CHECK(hipEventRecord(s->ev0[0], s->stream));
+    s->loop_seq++;  // numbers this substep's published words
+    if (timed) BBX_HIP_CHECK(hipEventRecord(s->ev0[0], s->stream));
     BBX_CHECK(distribute_grid(s, false, -1, (int *)s->max_force, kStepClear));
     BBX_CHECK(build_buckets(s, true, 0, nullptr));
     StepConst st{};
     st.dt = (float)dt;
     st.dt_over_m = (float)(dt / s->mass);
-    BBX_CHECK(run_sph_force(s));
-    BBX_CHECK(run_integrate(s, st));
+    BBX_CHECK(run_sph_step(s, st));
     BBX_CHECK(swap_after_integrate(s));
     BBX_CHECK(run_xsph(s, st));
-    BBX_HIP_CHECK(hipEventRecord(s->ev1[0], s->stream));
+    if (timed) BBX_HIP_CHECK(hipEventRecord(s->ev1[0], s->stream));
     bbx_stats local{};
-    BBX_CHECK(read_stats(s, &local));
+    if (s->d_signal && s->n > 0)
+        BBX_CHECK(published_sph(s, &local));
+    else
+        BBX_CHECK(read_stats(s, &local));
     s->maxf_cached = true;
     local.max_density_error = 0;
-    float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, s->ev0[0], s->ev1[0]);
-    local.gpu_ms = ms;
+    if (timed) BBX_CHECK(elapsed_ms(s->ev0[0], s->ev1[0], &local.gpu_ms));
     if (stats) *stats = local;
     if (s->prof.enabled) s->prof.resolve();
     return BBX_OK;
 }
+extern "C" {
+
+int bbx_sph_substep(bbx_solver *s, double dt, bbx_stats *stats) { return sph_substep(s, dt, stats, true); }
 
 int bbx_sph_advance(bbx_solver *s, double interval, int *substeps) {
     BBX_CHECK(check_setup(s));
@@ -1538,10 +1579,11 @@ int bbx_sph_advance(bbx_solver *s, double interval, int *substeps) {
         BBX_CHECK(time_steps(s, remaining, 1.0, &n));
         if (n == 0) return fail(BBX_E_INVALID, "time-step rule returned 0");
         double dt = remaining / (double)n;
-        BBX_CHECK(bbx_sph_substep(s, dt, nullptr));
+        BBX_CHECK(sph_substep(s, dt, nullptr, false));
         remaining -= dt;
         steps++;
     }
+    BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
     if (substeps) *substeps = steps;
     return BBX_OK;
 }

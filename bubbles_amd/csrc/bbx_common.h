@@ -144,11 +144,11 @@ struct LoopState {
 // `stats`, each word (seq << 32) | value: a word of another substep carries
 // another seq, so the host needs no ordering between the stores to tell
 // that all of them are current.
-enum { PUB_ERR_LO = 0, PUB_ERR_HI, PUB_OVERFLOW, PUB_LOST, PUB_FULL, kPubWords };
+enum { PUB_ERR_LO = 0, PUB_ERR_HI, PUB_OVERFLOW, PUB_LOST, PUB_FULL, kPubWords, PUB_MAXF = kPubWords };
 struct LoopSignal {
     unsigned word;
     unsigned pad;
-    unsigned long long stats[kPubWords];
+    unsigned long long stats[kPubWords + 1];  // the last one: SPH, FP32 bits of max |f|
 };
 
 // device-side counters
@@ -166,6 +166,7 @@ enum {
 struct StepBlock {
     int counters[CNT_N];
     unsigned max_force[kSlots];
+    int arrived[kSlots + 2];  // SPH: workgroups done per slot, slots done (and a pad)
     LoopState loop;
 };
 constexpr size_t kStepReadback = offsetof(StepBlock, loop) + offsetof(LoopState, slot);
@@ -270,6 +271,7 @@ struct bbx_solver {
     int ntiles = 0;
     // per-particle fields
     float *rho = nullptr, *pres = nullptr, *rho_star = nullptr;
+    float4 *vr = nullptr;        // SPH: velocity xyz and 1 / density (PCISPH keeps them in velB until it integrates)
     float4 *xq = nullptr;        // position xyz and q = p / rho*^2 (the pressure-force gather input)
     float4 *force = nullptr, *fp = nullptr, *xstar = nullptr;
     float *feat = nullptr;       // [16][stride]
@@ -344,8 +346,7 @@ int run_predict_pressure(bbx_solver *s, const StepConst &st, int k);
 // k < 0: predict only (warm start); otherwise integrate when iteration k is
 // converged (or k == max_it - 1, or exact), else predict iteration k + 1
 int run_pressure_force(bbx_solver *s, const StepConst &st, int k, int max_it, int exact, double tol);
-int run_sph_force(bbx_solver *s);
-int run_integrate(bbx_solver *s, const StepConst &st);
+int run_sph_step(bbx_solver *s, const StepConst &st);
 int run_xsph(bbx_solver *s, const StepConst &st);
 int swap_after_integrate(bbx_solver *s);
 const float *mlp_params_device(const bbx_mlp *m);

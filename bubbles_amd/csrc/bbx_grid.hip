@@ -1347,7 +1347,7 @@ int build_buckets(bbx_solver *s, bool with_pressure, int feat_mode, const StepCo
         WarmIn wi{};
         if (st) wi.st = *st;
         wi.vel = s->velA;
-        wi.vr = s->velB;  // free until the integration writes it
+        wi.vr = s->vr ? s->vr : s->velB;  // velB is free until the integration writes it
         wi.store_feat = s->keep_features;
         wi.feat = s->feat;
         wi.P = feat_mode == 2 ? mlp_params_device(s->mlp) : nullptr;

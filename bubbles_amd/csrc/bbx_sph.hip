@@ -471,19 +471,40 @@ __global__ void __launch_bounds__(kBlock) k_pressure_force(SimConst c, StepConst
 }
 
 // ---------------------------------------------------------------------------
-// SPH (WCSPH) forces: ComputeAllForcesFor without the in-loop integration
-// (src/equations/sph_equations3.cpp:184-278); integration is a separate pass.
-// LDS: (position, p / rho^2), (velocity, density).
+// SPH (WCSPH) step: ComputeAllForcesFor (src/equations/sph_equations3.cpp:184-278)
+// and TimeIntegrationFor in one launch.  All neighbours are read from the
+// state before the step and the new state goes to the other buffers, so it
+// is the two-phase form (all forces, then all moves) without a pass between.
+// LDS: (position, p / rho^2), (velocity, 1 / density), two lanes per
+// particle, as in the non-pressure gather: with one lane, the pairs put
+// together through registers (a division for every staged neighbour), IEEE
+// divisions per pair and a second launch for the moves it took 15.1 + 4.1 us
+// at 16k particles and 40.4 + 9.9 us at 241k; now 8.8 and 23.1 us.
+//
+// The last workgroup to finish publishes the substep's statistics and its
+// largest force to the host (LoopSignal), which waits for them to choose the
+// next time step: a copy and a stream synchronisation left the device idle
+// for about 25 us a substep.  Arrivals are counted in kSlots words and one
+// above them, so no word takes an atomic from every workgroup; a workgroup's
+// maximum has reached its slot before its arrival is counted.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kBlock) k_sph_force(SimConst c, NbrTab nb,
-                                                      const float4 *__restrict__ pos,
-                                                      const float4 *__restrict__ vel,
-                                                      const float *__restrict__ rho,
-                                                      const float *__restrict__ pres,
-                                                      float4 *__restrict__ force) {
+constexpr int kSphThreads = 2 * kBlock;
+
+template <bool kList>
+__global__ void __launch_bounds__(kSphThreads) k_sph_step(SimConst c, StepConst st, NbrTab nb,
+                                                          const float4 *__restrict__ pos,
+                                                          const float4 *__restrict__ vel,
+                                                          const float4 *__restrict__ xq,
+                                                          const float4 *__restrict__ vr,
+                                                          float4 *__restrict__ force,
+                                                          float4 *__restrict__ pos_out,
+                                                          float4 *__restrict__ vel_out,
+                                                          int *__restrict__ flag, StepBlock *step,
+                                                          LoopSignal *sig, unsigned seq) {
     __shared__ float4 sx[kFarSlot + 1];
     __shared__ float4 sv[kFarSlot + 1];
     __shared__ TileTab tt;
+    __shared__ unsigned wmax[kSphThreads / 64];
     const int tile = tile_of_block();
     tab_load_shared(nb.tab + (size_t)tile * kTabInts, tt);
     if (threadIdx.x == 0) {
@@ -493,82 +514,112 @@ __global__ void __launch_bounds__(kBlock) k_sph_force(SimConst c, NbrTab nb,
     __syncthreads();
     const bool staged = tt.staged != 0;
     const bool in_lds = staged && tt.total <= c.tile_cap2;
-    auto xq = [&](int j) {
-        float4 p = pos[j];
-        float d = rho[j];
-        return make_float4(p.x, p.y, p.z, pres[j] / (d * d));
-    };
-    auto vr = [&](int j) {
-        float4 v = vel[j];
-        return make_float4(v.x, v.y, v.z, rho[j]);
-    };
+    const int pl = threadIdx.x >> 1, half = threadIdx.x & 1;
+    const int i = tile * kBlock + pl;
+    const bool valid = i < c.n;
+    int cnt = 0;
+    float4 xi = make_float4(0.f, 0.f, 0.f, 0.f), vi = xi;
+    float pw = 0.f;
+    NbrQuads<2> first{};
+    if (valid) {  // independent of the staging: requested before it
+        cnt = nb.cnt[i];
+        xi = xq[i];
+        vi = vel[i];
+        pw = pos[i].w;
+        first = nbr_prefetch<2, 2>(nb.n16, nb.n32, staged, i, c.stride, half);
+    }
     if (in_lds) {
-        tab_stage(tt, sx, xq);
-        tab_stage(tt, sv, vr);
+        tab_stage_dma(tt, [&](int j, int e) {
+            lds_dma16(xq + j, sx + e);
+            lds_dma16(vr + j, sv + e);
+        });
+        lds_dma_wait();
     }
     __syncthreads();
-    const int i = tile * kBlock + threadIdx.x;
-    if (i >= c.n) return;
-    const int self = staged ? tab_local(tt, i) << kSlotShift : i;
-    const float4 xi = pos[i], vi = vel[i];
-    const float di = rho[i];
-    const float qi = pres[i] / (di * di);
-    const float coef = c.visc * c.mass2;
-    float fx = c.mass * c.gx - c.drag * vi.x;
-    float fy = c.mass * c.gy - c.drag * vi.y;
-    float fz = c.mass * c.gz - c.drag * vi.z;
-    float tx = 0.f, ty = 0.f, tz = 0.f, ex = 0.f, ey = 0.f, ez = 0.f;
-    const int cnt = nb.cnt[i];
-    for_each_neighbour<2>(nb.n16, nb.n32, staged, i, cnt, c.stride, [&](int j, bool live) {
-        // masks, not early returns: the pair's loads and arithmetic are
-        // unconditional and a skipped pair adds exact zeros
-        float4 xj, vj;
-        if (in_lds) {
-            xj = lds_at(sx, j);
-            vj = lds_at(sv, j);
-        } else {
-            const int g = staged ? (live ? tab_global(tt, j >> kSlotShift) : i) : j;
-            xj = xq(g);
-            vj = vr(g);
-        }
-        const float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
-        const float r = sqrtf(dx * dx + dy * dy + dz * dz);
-        const bool in = live & (j != self) & spiky_in(c, r);
-        const float x = 1.f - r * c.inv_h;
-        const bool pg = in & (r > 0.f) & !(fabsf(r) < 1e-8f);
-        const float g = keep_if(pg, c.mass2 * (qi + xj.w) * c.spiky_grad * x * x / r);
-        kahan_add(tx, ex, g * dx);
-        kahan_add(ty, ey, g * dy);
-        kahan_add(tz, ez, g * dz);
-        const float s = keep_if(in, coef * c.spiky_lap * x / vj.w);
-        fx += (vj.x - vi.x) * s;
-        fy += (vj.y - vi.y) * s;
-        fz += (vj.z - vi.z) * s;
-    });
-    force[i] = make_float4(fx - tx, fy - ty, fz - tz, 0.f);
-}
-
-// TimeIntegrationFor as a separate pass (SPH two-phase form)
-template <bool kList>
-__global__ void __launch_bounds__(kBlock) k_integrate(SimConst c, StepConst st,
-                                                      const float4 *__restrict__ pos,
-                                                      const float4 *__restrict__ vel,
-                                                      const float4 *__restrict__ force,
-                                                      float4 *__restrict__ pos_out,
-                                                      float4 *__restrict__ vel_out,
-                                                      int *__restrict__ flag,
-                                                      unsigned *__restrict__ max_force) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
     unsigned fbits = 0u;
-    if (i < c.n) {
-        const float4 xi = pos[i], vi = vel[i], fi = force[i];
-        float3 p, v;
-        integrate_one<kList>(c, st.dt, xi, vi, fi.x, fi.y, fi.z, p, v, flag);
-        pos_out[i] = make_float4(p.x, p.y, p.z, xi.w);
-        vel_out[i] = make_float4(v.x, v.y, v.z, vi.w);
-        fbits = __float_as_uint(sqrtf(fi.x * fi.x + fi.y * fi.y + fi.z * fi.z));
+    if (valid) {
+        const float coef = c.visc * c.mass2 * c.spiky_lap, kg = c.mass2 * c.spiky_grad;
+        const float qi = xi.w;
+        float fx = 0.f, fy = 0.f, fz = 0.f;
+        float tx = 0.f, ty = 0.f, tz = 0.f, ex = 0.f, ey = 0.f, ez = 0.f;
+        with_staging(in_lds, [&](auto tag) {
+            constexpr bool kL = decltype(tag)::value;
+            auto body = [&](int j, bool live) {
+                float4 a, b;
+                if (kL) {
+                    a = lds_at(sx, j);
+                    b = lds_at(sv, j);
+                } else {
+                    const int g = staged ? (live ? tab_global(tt, j >> kSlotShift) : i) : j;
+                    a = xq[g];
+                    b = vr[g];
+                }
+                // no branches and no masks, as in the non-pressure gather; the
+                // particle itself has no offset and no relative velocity
+                const float dx = a.x - xi.x, dy = a.y - xi.y, dz = a.z - xi.z;
+                const PairFactor f = pair_factor(c, dx, dy, dz);
+                const float x = kL || live ? f.x : 0.f;
+                const float g = kg * (qi + a.w) * x * x * f.ir;
+                kahan_fma(tx, ex, g, dx);
+                kahan_fma(ty, ey, g, dy);
+                kahan_fma(tz, ez, g, dz);
+                const float s = coef * x * b.w;
+                fx = fmaf(b.x - vi.x, s, fx);
+                fy = fmaf(b.y - vi.y, s, fy);
+                fz = fmaf(b.z - vi.z, s, fz);
+            };
+            for_each_neighbour_from<2, 2>(first, nb.n16, nb.n32, staged, i, cnt, c.stride, body, half);
+        });
+        // the pair's sums: viscosity, then the compensated pressure force
+        tx -= ex;
+        ty -= ey;
+        tz -= ez;
+        fx += __shfl_xor(fx, 1, 64);
+        fy += __shfl_xor(fy, 1, 64);
+        fz += __shfl_xor(fz, 1, 64);
+        tx += __shfl_xor(tx, 1, 64);
+        ty += __shfl_xor(ty, 1, 64);
+        tz += __shfl_xor(tz, 1, 64);
+        if (half == 0) {
+            const float Fx = c.mass * c.gx - c.drag * vi.x + fx - tx;
+            const float Fy = c.mass * c.gy - c.drag * vi.y + fy - ty;
+            const float Fz = c.mass * c.gz - c.drag * vi.z + fz - tz;
+            float3 p, v;
+            integrate_one<kList>(c, st.dt, xi, vi, Fx, Fy, Fz, p, v, flag);
+            force[i] = make_float4(Fx, Fy, Fz, 0.f);
+            pos_out[i] = make_float4(p.x, p.y, p.z, pw);
+            vel_out[i] = make_float4(v.x, v.y, v.z, vi.w);
+            fbits = __float_as_uint(sqrtf(Fx * Fx + Fy * Fy + Fz * Fz));
+        }
     }
-    block_max_to_slot(fbits, max_force);
+    fbits = wave_max_u32(fbits);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = fbits;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    bool last = false;
+    if (threadIdx.x == 0) {
+        unsigned m = wmax[0];
+        for (int w = 1; w < kSphThreads / 64; w++) m = wmax[w] > m ? wmax[w] : m;
+        const int slot = blockIdx.x & (kSlots - 1);
+        if (m) atomicMax(&step->max_force[slot], m);
+        if (sig) {
+            __builtin_amdgcn_s_waitcnt(0);  // the maximum is in its slot
+            const int nblk = (int)gridDim.x, in_slot = (nblk - slot + kSlots - 1) / kSlots;
+            if (atomicAdd(&step->arrived[slot], 1) + 1 == in_slot)
+                last = atomicAdd(&step->arrived[kSlots], 1) + 1 == min(nblk, kSlots);
+        }
+    }
+    if (!__any(last)) return;
+    // every workgroup has arrived
+    const int lane = threadIdx.x;
+    unsigned all = wave_max_u32(lane < kSlots ? atomicMax(&step->max_force[lane], 0u) : 0u);
+    if (lane < 4) {
+        const unsigned long long tag = (unsigned long long)seq << 32;
+        const int from[3] = {CNT_OVERFLOW, CNT_LOST, CNT_FULL};
+        const int at[4] = {PUB_OVERFLOW, PUB_LOST, PUB_FULL, PUB_MAXF};
+        const unsigned v = lane < 3 ? (unsigned)step->counters[from[lane]] : all;
+        __hip_atomic_store(&sig->stats[at[lane]], tag | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // XSPH velocity smoothing (src/equations/sph_equations3.cpp:341-382), active
@@ -717,21 +768,12 @@ int run_pressure_force(bbx_solver *s, const StepConst &st, int k, int max_it, in
     return BBX_OK;
 }
 
-int run_sph_force(bbx_solver *s) {
+int run_sph_step(bbx_solver *s, const StepConst &st) {
     if (s->n == 0) return BBX_OK;
-    BBX_PROF_BEGIN("sph_force");
-    k_sph_force<<<nblocks(s->n), kBlock, 0, s->stream>>>(s->sc, nbr_tab(s), s->posA, s->velA, s->rho,
-                                                         s->pres, s->force);
-    BBX_HIP_CHECK(hipGetLastError());
-    BBX_PROF_END();
-    return BBX_OK;
-}
-
-int run_integrate(bbx_solver *s, const StepConst &st) {
-    if (s->n == 0) return BBX_OK;
-    BBX_PROF_BEGIN("integrate");
-    (s->ncoll ? k_integrate<true> : k_integrate<false>)<<<nblocks(s->n), kBlock, 0, s->stream>>>(s->sc, st, s->posA, s->velA, s->force,
-                                                         s->posB, s->velB, s->flag, s->max_force);
+    BBX_PROF_BEGIN("sph_step");
+    (s->ncoll ? k_sph_step<true> : k_sph_step<false>)<<<nblocks(s->n), kSphThreads, 0, s->stream>>>(
+        s->sc, st, nbr_tab(s), s->posA, s->velA, s->xq, s->vr, s->force, s->posB, s->velB, s->flag, s->step,
+        s->d_signal, s->loop_seq & 0x7fffffu);
     BBX_HIP_CHECK(hipGetLastError());
     BBX_PROF_END();
     return BBX_OK;
