@@ -527,7 +527,7 @@ __device__ __forceinline__ unsigned long long row_mask(const SimConst &c, float4
 #pragma unroll
         for (int q = 0; q < 8; q++) {
             if (kStaged)
-                pc[q] = row[t0 + q];
+                pc[q] = lds_slot(row + t0 + q);
             else
                 pc[q] = pos[min(a + t0 + q, c.n - 1)];
         }
@@ -549,7 +549,7 @@ __device__ __forceinline__ unsigned long long row_mask(const SimConst &c, float4
     if (bdist <= c.band_w) {
         // candidates inside the band: the exact FP64 rule
         for (int t = 0; t < len; t++) {
-            const float4 pj = kStaged ? row[t] : pos[a + t];
+            const float4 pj = kStaged ? lds_slot(row + t) : pos[a + t];
             if (fabsf(cut_offset(pi, pj, c.band_c)) <= c.band_w) {
                 const unsigned long long bit = 1ull << t;
                 m = within_std_fp64(pi, pj, c.h2d) ? (m | bit) : (m & ~bit);
@@ -643,7 +643,7 @@ __device__ __forceinline__ void walk_cells(const SimConst &c, float4 pi, const i
                 const int sr = sh[dz * 3 + dy];
                 const int e = start[cell + 1];
                 for (int j = start[cell]; j < e; j++) {
-                    const float4 pj = kStaged ? sx[j + sr] : pos[j];
+                    const float4 pj = kStaged ? lds_slot(sx + j + sr) : pos[j];
                     if (in_bucket(c, pi, pj)) bw.emit(j, sr);
                 }
             }
@@ -977,10 +977,11 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
 // a crowded row or more neighbours than the cap is walked cell by cell by its
 // first lane.
 //
-// Used up to kSmallSet.  Measured (us, one lane per particle / four): 25.2 / 12.3
-// at 2k, 28.3 / 14.5 at 16k, 29.7 / 23.2 at 35k, 37.6 / 41.2 at 94k, 62.6 /
-// over 200 at 255k, where the chip is full and the four workgroups' staging
-// and the longer emission count.
+// Used up to kSmallSet.  Measured (us, one lane per particle and the kernel
+// of its tile tables / four): 28.2 / 12.9 at 2k, 31.0 / 14.7 at 16k, 33.5 / 25.5
+// at 35k, 32.1 / 30.5 at 65k, 35.5 / 40.0 at 94k, 71.9 / 121.8 at 255k, where
+// the chip is full and the four workgroups' staging and the longer emission
+// count.
 constexpr int kSplitLanes = 4;
 constexpr int kSplitRows = kBlock / kSplitLanes;  // particles per workgroup
 constexpr int kSplitMax = kBucket;                // bucket entries held in LDS

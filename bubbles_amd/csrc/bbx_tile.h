@@ -87,8 +87,17 @@ constexpr int kFarSlot = kTileCap;
 constexpr unsigned kFarEntry = (unsigned)kFarSlot << kSlotShift;
 static_assert(kFarEntry < 65536u, "entries are 16 bits");
 __device__ __forceinline__ float4 far_particle(float w) { return make_float4(1e15f, 1e15f, 1e15f, w); }
+// A whole slot in one 16-byte read, also where w is not used: loaded through
+// float4's members the compiler drops w and reads 12 bytes (ds_read_b96),
+// which takes the LDS longer.  Per wave and CU: 7.9 against 4.1 ns for slots
+// all over a tile, 5.7 against 2.4 ns for runs of slots.
+typedef float lds_f4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float4 lds_slot(const float4 *p) {
+    const lds_f4 v = *reinterpret_cast<const lds_f4 *>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
 __device__ __forceinline__ float4 lds_at(const float4 *base, int byte_off) {
-    return *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(base) + byte_off);
+    return lds_slot(reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(base) + byte_off));
 }
 
 // storage index of LDS-local index jl (jl < t.total)
