@@ -390,7 +390,7 @@ static void free_all(bbx_solver *s) {
     dfree(s->posA); dfree(s->posB); dfree(s->velA); dfree(s->velB);
     dfree(s->cellA); dfree(s->cellB); dfree(s->home);
     dfree(s->cell_count); dfree(s->cell_start); dfree(s->scan_tmp);
-    dfree(s->key); dfree(s->newc); dfree(s->rank_tmp); dfree(s->tmp_idx); dfree(s->hash_tmp);
+    dfree(s->key); dfree(s->newc); dfree(s->rank_tmp); dfree(s->tmp_idx); dfree(s->hash_tmp); dfree(s->bins);
     dfree(s->nbr16); dfree(s->nbr32); dfree(s->nbr_cnt); dfree(s->tile_tab);
     dfree(s->rho); dfree(s->pres); dfree(s->rho_star); dfree(s->xq); dfree(s->vr);
     dfree(s->force); dfree(s->fp); dfree(s->xstar); dfree(s->feat); dfree(s->pwarm);
@@ -551,6 +551,10 @@ int bbx_solver_create(int kind, const bbx_params *params, const double *pos, con
         s->counters = s->step->counters;
     }
     if (!rc) rc = dalloc(&s->flag, 1);
+    if (!rc && cells <= std::max((size_t)kBinCells, N) && dalloc(&s->bins, grid_bins_words(cells - 1)) != BBX_OK) {
+        s->bins = nullptr;  // no room: the grid pass does without
+        (void)hipGetLastError();
+    }
     // one pinned block (an allocation costs about 100 us): the loop signal,
     // the step block's copy, a flag, and the ring of the field downloads
     const size_t pin_step = 256, pin_flag = pin_step + (sizeof(StepBlock) + 255) / 256 * 256, pin_ring = pin_flag + 256;

@@ -255,6 +255,22 @@ int launch_scan(bbx_solver *s, const int *in, int *out, size_t n) {
 // slot), every new one joins the chain of the cell it hashes into, after the
 // old members in the order added (DistributeByParticleList + AddToChain,
 // src/core/grid.h:358-387,128-140).
+//
+// With kBins (see distribute_grid) the key also goes into its cell's bin at
+// its arrival slot, so that the particle's rank can be counted from the bin
+// and neither a scatter into cell segments nor its index is needed.  A
+// particle that finds the bin full is chained to its cell: the head carries
+// the pass number, so that heads of earlier passes need no clearing.  The
+// particles in no chain, which may be many, are listed by arrival.
+constexpr int kBinCap = 32;
+struct BinKeys {
+    unsigned long long *__restrict__ bin;   // [cells][kBinCap]
+    unsigned long long *__restrict__ head;  // [cells] (pass << 32) | particle
+    int *__restrict__ next;                 // [n] particle, or -1
+    int *__restrict__ none;                 // [n] particles in no chain
+    unsigned pass;
+};
+template <bool kBins>
 __global__ void __launch_bounds__(kBlock) k_hash(SimConst c, const float4 *__restrict__ pos,
                                                  const int *__restrict__ cell_old,
                                                  const int *__restrict__ flag, int force_full,
@@ -262,7 +278,7 @@ __global__ void __launch_bounds__(kBlock) k_hash(SimConst c, const float4 *__res
                                                  int *__restrict__ newc, int *__restrict__ hcell,
                                                  unsigned long long *__restrict__ key,
                                                  int *__restrict__ count,
-                                                 int *__restrict__ rank_tmp) {
+                                                 int *__restrict__ rank_tmp, BinKeys bk) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     const int none = (int)c.g.total;
     const bool valid = s < c.n;
@@ -317,36 +333,62 @@ __global__ void __launch_bounds__(kBlock) k_hash(SimConst c, const float4 *__res
     // a point outside the grid has no home cell: its bucket stays empty
     hcell[s] = bad ? -1 : cid;
     key[s] = k;
-    rank_tmp[s] = base + (lane - head_lane);
+    const int slot = base + (lane - head_lane);
+    if constexpr (kBins) {
+        if (nc == none) {
+            bk.none[slot] = s;
+        } else if (slot < kBinCap) {
+            bk.bin[(size_t)nc * kBinCap + slot] = k;
+        } else {
+            const unsigned long long old =
+                atomicExch(&bk.head[nc], ((unsigned long long)bk.pass << 32) | (unsigned)s);
+            bk.next[s] = (unsigned)(old >> 32) == bk.pass ? (int)(unsigned)old : -1;
+        }
+    } else {
+        rank_tmp[s] = slot;
+    }
+}
+
+size_t grid_bins_words(size_t cells) { return cells * (kBinCap + 1); }
+
+// What the pass reports and leaves behind, done by the last launch that may
+// (thread t of all): statistics, the higher-level flag, the cell counts back
+// at zero for the next pass, and `clear` (a substep's step block behind its
+// counters), which took a launch of their own (4.2 us at 1M).
+struct PassEnd {
+    int *__restrict__ count;
+    size_t cells;
+    int *__restrict__ flag;
+    int force_full, append;
+    int *__restrict__ counters;
+    int *__restrict__ clear;
+    size_t clear_n;
+};
+__device__ __forceinline__ void end_pass(const SimConst &c, const PassEnd &e, const int *__restrict__ start, size_t t) {
+    if (t == 0) {
+        e.counters[CNT_OVERFLOW] = 0;
+        e.counters[CNT_LOST] = c.n - start[c.g.total];
+        if (!e.append) {  // an append leaves the higher-level flag to the next substep
+            e.counters[CNT_FULL] = (e.force_full || *e.flag) ? 1 : 0;
+            *e.flag = 0;  // ResetHigherLevel
+        } else {
+            e.counters[CNT_FULL] = 0;
+        }
+    }
+    if (t < e.cells) e.count[t] = 0;
+    if (t < e.clear_n) e.clear[t] = 0;
 }
 
 // ---------------------------------------------------------------------------
-// 3. scatter into cell segments (arrival order), record full/lost stats
+// 3. scatter into cell segments (arrival order); the cell counts have been
+// read for the last time, so the pass ends here
 // ---------------------------------------------------------------------------
-// The cell counts have been read for the last time: this launch also leaves
-// them at zero for the next pass, and clears `clear` (a substep's step block
-// behind its counters), which took a launch of their own (4.2 us at 1M).
 __global__ void __launch_bounds__(kBlock) k_scatter(SimConst c, const int *__restrict__ newc,
                                                     const int *__restrict__ rank_tmp,
                                                     const int *__restrict__ start,
-                                                    int *__restrict__ count, size_t cells,
-                                                    int *__restrict__ tmp_idx,
-                                                    int *__restrict__ flag, int force_full,
-                                                    int append, int *__restrict__ counters,
-                                                    int *__restrict__ clear, size_t clear_n) {
+                                                    int *__restrict__ tmp_idx, PassEnd end) {
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) {
-        counters[CNT_OVERFLOW] = 0;
-        counters[CNT_LOST] = c.n - start[c.g.total];
-        if (!append) {  // an append leaves the higher-level flag to the next substep
-            counters[CNT_FULL] = (force_full || *flag) ? 1 : 0;
-            *flag = 0;  // ResetHigherLevel
-        } else {
-            counters[CNT_FULL] = 0;
-        }
-    }
-    if (t < cells) count[t] = 0;
-    if (t < clear_n) clear[t] = 0;
+    end_pass(c, end, start, t);
     if (t < (size_t)c.n) tmp_idx[start[newc[t]] + rank_tmp[t]] = (int)t;
 }
 
@@ -420,6 +462,81 @@ __global__ void __launch_bounds__(kBlock) k_rank_move(SimConst c, const int *__r
     vel_out[dest] = vel_in[s];
     cell_out[dest] = cc;
     home_out[dest] = hcell[s];
+}
+
+// 3 and 4 from the bins: a particle's rank is the number of smaller keys in
+// its cell's bin, eight of them (a cell of ordinary density) requested beside
+// its other data, and in the cell's chain behind a full bin.  Workgroups of
+// particles in no chain read those through LDS as k_rank_move does.
+__global__ void __launch_bounds__(kBlock) k_rank_bins(SimConst c, const int *__restrict__ newc,
+                                                      const int *__restrict__ hcell,
+                                                      const unsigned long long *__restrict__ key,
+                                                      const int *__restrict__ start, BinKeys bk,
+                                                      const float4 *__restrict__ pos_in,
+                                                      const float4 *__restrict__ vel_in,
+                                                      float4 *__restrict__ pos_out,
+                                                      float4 *__restrict__ vel_out,
+                                                      int *__restrict__ cell_out,
+                                                      int *__restrict__ home_out, PassEnd end) {
+    __shared__ unsigned long long skey[kBlock];
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    end_pass(c, end, start, t);
+    if ((size_t)blockIdx.x * blockDim.x >= (size_t)c.n) return;  // whole workgroups
+    const bool valid = t < (size_t)c.n;
+    const int total = (int)c.g.total;  // start[total]: the particles in no chain, up to n
+    int cc = 0, home = -1, b = 0, cnt = 0, rank = 0;
+    unsigned long long k = 0ull;
+    float4 p{}, v{};
+    bool lost = false;
+    if (valid) {
+        cc = newc[t];
+        k = key[t];
+        p = pos_in[t];
+        v = vel_in[t];
+        home = hcell[t];
+        lost = cc == total;
+        b = start[cc];
+        if (!lost) {
+            const ulonglong2 *bin = reinterpret_cast<const ulonglong2 *>(bk.bin + (size_t)cc * kBinCap);
+            constexpr int kFirst = 4;  // pairs of keys
+            ulonglong2 q[kFirst];
+#pragma unroll
+            for (int u = 0; u < kFirst; u++) q[u] = bin[u];
+            cnt = start[cc + 1] - b;
+#pragma unroll
+            for (int u = 0; u < kFirst; u++) {
+                rank += 2 * u < cnt && q[u].x < k ? 1 : 0;
+                rank += 2 * u + 1 < cnt && q[u].y < k ? 1 : 0;
+            }
+            const int binned = min(cnt, kBinCap);
+            for (int u = kFirst; 2 * u < binned; u++) {
+                const ulonglong2 w = bin[u];
+                rank += w.x < k ? 1 : 0;
+                rank += 2 * u + 1 < binned && w.y < k ? 1 : 0;
+            }
+            if (cnt > kBinCap)
+                for (int o = (int)(unsigned)bk.head[cc]; o >= 0; o = bk.next[o]) rank += key[o] < k ? 1 : 0;
+        }
+    }
+    if (__syncthreads_or(lost)) {
+        const int lost_n = c.n - start[total];
+        for (int q0 = 0; q0 < lost_n; q0 += kBlock) {
+            const int q = q0 + (int)threadIdx.x;
+            if (q < lost_n) skey[threadIdx.x] = key[bk.none[q]];
+            __syncthreads();
+            if (lost) {
+                const int m = min(kBlock, lost_n - q0);
+                for (int u = 0; u < m; u++) rank += skey[u] < k ? 1 : 0;
+            }
+            __syncthreads();
+        }
+    }
+    if (!valid) return;
+    const int dest = b + rank;
+    pos_out[dest] = p;
+    vel_out[dest] = v;
+    cell_out[dest] = cc;
+    home_out[dest] = home;
 }
 
 // ---------------------------------------------------------------------------
@@ -1288,16 +1405,34 @@ int distribute_grid(bbx_solver *s, bool force_full, int append_from, int *clear,
         BBX_CHECK(launch_fill_int(s, s->counters, 0, CNT_N));
         return clear_n ? launch_fill_int(s, clear, 0, clear_n) : BBX_OK;
     }
-    // k_scatter leaves the counts at zero; not so before the first pass, or
+    // From the bins where the solver has them (grids of up to kBinCells cells,
+    // or one per particle): one launch less, and no index to follow.  Scatter
+    // and rank through the index / rank from the bins (us): 2.6 + 5.3 / 3.4
+    // at 2k, 2.4 + 5.7 / 4.2 at 16k, 2.8 + 7.2 / 4.4 at 94k, 3.1 + 9.4 / 7.1 at
+    // 255k, 5.3 + 20.0 / 21.3 at 1M (where the hash gains 1.8).  A grid with
+    // many more cells than particles would pay for its bins in memory.
+    const bool bins = s->bins != nullptr;
+    // the pass leaves the counts at zero; not so before the first one, or
     // behind one that did not get that far
     if (!s->counts_clear) BBX_CHECK(launch_fill_int(s, s->cell_count, 0, cells));
     s->counts_clear = false;
+    BinKeys bk{};
+    if (bins) {
+        const size_t in_bins = (cells - 1) * kBinCap;
+        if (s->bin_pass + 1u <= 1u) {  // heads hold no pass number yet, or may hold any
+            BBX_CHECK(launch_fill_int(s, reinterpret_cast<int *>(s->bins + in_bins), 0, 2 * (cells - 1)));
+            s->bin_pass = 0;
+        }
+        bk = BinKeys{s->bins, s->bins + in_bins, s->tmp_idx, s->rank_tmp, ++s->bin_pass};
+    }
+    const PassEnd end{s->cell_count, cells, s->flag, force_full ? 1 : 0, append_from >= 0 ? 1 : 0, s->counters,
+                      clear, clear_n};
+    const unsigned end_blocks = (unsigned)((std::max({(size_t)n, cells, clear_n}) + kBlock - 1) / kBlock);
     {
         BBX_PROF_BEGIN("grid_hash");
-        k_hash<<<nblocks(n), kBlock, 0, s->stream>>>(c, s->posA, s->cellA, s->flag,
-                                                     force_full ? 1 : 0, append_from, s->newc,
-                                                     s->hash_tmp, s->key, s->cell_count,
-                                                     s->rank_tmp);
+        (bins ? k_hash<true> : k_hash<false>)<<<nblocks(n), kBlock, 0, s->stream>>>(
+            c, s->posA, s->cellA, s->flag, force_full ? 1 : 0, append_from, s->newc, s->hash_tmp, s->key,
+            s->cell_count, s->rank_tmp, bk);
         BBX_HIP_CHECK(hipGetLastError());
         BBX_PROF_END();
     }
@@ -1306,23 +1441,26 @@ int distribute_grid(bbx_solver *s, bool force_full, int append_from, int *clear,
         BBX_CHECK(launch_scan(s, s->cell_count, s->cell_start, cells));
         BBX_PROF_END();
     }
-    {
-        const size_t items = std::max({(size_t)n, cells, clear_n});
+    if (!bins) {
         BBX_PROF_BEGIN("grid_scatter");
-        k_scatter<<<(unsigned)((items + kBlock - 1) / kBlock), kBlock, 0, s->stream>>>(
-            c, s->newc, s->rank_tmp, s->cell_start, s->cell_count, cells, s->tmp_idx, s->flag, force_full ? 1 : 0,
-            append_from >= 0 ? 1 : 0, s->counters, clear, clear_n);
+        k_scatter<<<end_blocks, kBlock, 0, s->stream>>>(c, s->newc, s->rank_tmp, s->cell_start, s->tmp_idx, end);
         BBX_HIP_CHECK(hipGetLastError());
-        s->counts_clear = true;
         BBX_PROF_END();
     }
     {
         BBX_PROF_BEGIN("grid_rank_move");
-        k_rank_move<<<nblocks(n), kBlock, 0, s->stream>>>(c, s->tmp_idx, s->newc,
-                                                          s->hash_tmp, s->key, s->cell_start,
-                                                          s->posA, s->velA, s->posB,
-                                                          s->velB, s->cellB, s->home);
+        if (bins) {
+            k_rank_bins<<<end_blocks, kBlock, 0, s->stream>>>(c, s->newc, s->hash_tmp, s->key, s->cell_start, bk,
+                                                              s->posA, s->velA, s->posB, s->velB, s->cellB, s->home,
+                                                              end);
+        } else {
+            k_rank_move<<<nblocks(n), kBlock, 0, s->stream>>>(c, s->tmp_idx, s->newc,
+                                                              s->hash_tmp, s->key, s->cell_start,
+                                                              s->posA, s->velA, s->posB,
+                                                              s->velB, s->cellB, s->home);
+        }
         BBX_HIP_CHECK(hipGetLastError());
+        s->counts_clear = true;
         BBX_PROF_END();
     }
     std::swap(s->posA, s->posB);
