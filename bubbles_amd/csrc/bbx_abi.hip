@@ -1540,52 +1540,80 @@ static int published_sph(bbx_solver *s, bbx_stats *st) {
     return BBX_OK;
 }
 
-// timed: also measure the substep's device time, and return when it has
-// ended; without it the substep's last launch may still be running
-static int sph_substep(bbx_solver *s, double dt, bbx_stats *stats, bool timed) {
-    BBX_CHECK(check_setup(s));
-    if (s->kind != BBX_SPH) return fail(BBX_E_INVALID, "not an SPH solver");
-    if (!(dt > 0)) return fail(BBX_E_INVALID, "dt must be > 0");
+// A substep in three parts: what its time step has no part in (grid pass and
+// buckets), the step itself, and its statistics with the largest force.
+static int sph_front(bbx_solver *s) {
+    BBX_CHECK(distribute_grid(s, false, -1, (int *)s->max_force, kStepClear));
+    return build_buckets(s, true, 0, nullptr);
+}
+
+static int sph_back(bbx_solver *s, double dt) {
     s->maxf_cached = false;
     s->loop_seq++;  // numbers this substep's published words
-    if (timed) BBX_HIP_CHECK(hipEventRecord(s->ev0[0], s->stream));
-    BBX_CHECK(distribute_grid(s, false, -1, (int *)s->max_force, kStepClear));
-    BBX_CHECK(build_buckets(s, true, 0, nullptr));
     StepConst st{};
     st.dt = (float)dt;
     st.dt_over_m = (float)(dt / s->mass);
     BBX_CHECK(run_sph_step(s, st));
     BBX_CHECK(swap_after_integrate(s));
-    BBX_CHECK(run_xsph(s, st));
-    if (timed) BBX_HIP_CHECK(hipEventRecord(s->ev1[0], s->stream));
-    bbx_stats local{};
-    if (s->d_signal && s->n > 0)
-        BBX_CHECK(published_sph(s, &local));
-    else
-        BBX_CHECK(read_stats(s, &local));
+    return run_xsph(s, st);
+}
+
+static bool sph_publishes(const bbx_solver *s) { return s->d_signal && s->n > 0; }
+
+static int sph_stats(bbx_solver *s, bbx_stats *st) {
+    BBX_CHECK(sph_publishes(s) ? published_sph(s, st) : read_stats(s, st));
     s->maxf_cached = true;
-    local.max_density_error = 0;
-    if (timed) BBX_CHECK(elapsed_ms(s->ev0[0], s->ev1[0], &local.gpu_ms));
-    if (stats) *stats = local;
-    if (s->prof.enabled) s->prof.resolve();
+    return BBX_OK;
+}
+
+static int check_sph_step(bbx_solver *s, double dt) {
+    BBX_CHECK(check_setup(s));
+    if (s->kind != BBX_SPH) return fail(BBX_E_INVALID, "not an SPH solver");
+    if (!(dt > 0)) return fail(BBX_E_INVALID, "dt must be > 0");
     return BBX_OK;
 }
 extern "C" {
 
-int bbx_sph_substep(bbx_solver *s, double dt, bbx_stats *stats) { return sph_substep(s, dt, stats, true); }
+int bbx_sph_substep(bbx_solver *s, double dt, bbx_stats *stats) {
+    BBX_CHECK(check_sph_step(s, dt));
+    BBX_HIP_CHECK(hipEventRecord(s->ev0[0], s->stream));
+    BBX_CHECK(sph_front(s));
+    BBX_CHECK(sph_back(s, dt));
+    BBX_HIP_CHECK(hipEventRecord(s->ev1[0], s->stream));
+    bbx_stats local{};
+    BBX_CHECK(sph_stats(s, &local));
+    local.max_density_error = 0;
+    BBX_CHECK(elapsed_ms(s->ev0[0], s->ev1[0], &local.gpu_ms));
+    if (stats) *stats = local;
+    if (s->prof.enabled) s->prof.resolve();
+    return BBX_OK;
+}
 
 int bbx_sph_advance(bbx_solver *s, double interval, int *substeps) {
     BBX_CHECK(check_setup(s));
     double remaining = interval;
     int steps = 0;
+    // Whether a substep follows is known before this one's largest force is,
+    // which decides the next one's length alone: the next one's grid pass and
+    // buckets are queued first, and the device works while the host waits for
+    // the force, chooses dt and queues the step (16k particles, Advance(1e-3):
+    // 392 -> 370 us).  Not where the statistics are copied: the grid pass clears them.
+    bool front = false;
     while (remaining > (double)0.0001f) {
         unsigned n = 0;
         BBX_CHECK(time_steps(s, remaining, 1.0, &n));
         if (n == 0) return fail(BBX_E_INVALID, "time-step rule returned 0");
-        double dt = remaining / (double)n;
-        BBX_CHECK(sph_substep(s, dt, nullptr, false));
+        const double dt = remaining / (double)n;
+        BBX_CHECK(check_sph_step(s, dt));
+        if (!front) BBX_CHECK(sph_front(s));
+        BBX_CHECK(sph_back(s, dt));
         remaining -= dt;
         steps++;
+        front = remaining > (double)0.0001f && sph_publishes(s);
+        if (front) BBX_CHECK(sph_front(s));
+        bbx_stats local{};
+        BBX_CHECK(sph_stats(s, &local));
+        if (s->prof.enabled) s->prof.resolve();
     }
     BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
     if (substeps) *substeps = steps;

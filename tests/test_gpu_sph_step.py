@@ -74,3 +74,24 @@ def test_published_statistics_equal_the_copied_ones(bbx, monkeypatch, n, env):
     limit = min(0.4 * inf["kernel_radius"] / s.params.sound_speed,
                 0.25 * np.sqrt(inf["kernel_radius"] * inf["mass"] / fmax))
     assert abs(steps - 1.0 / limit) <= 1 + 1e-6 / limit
+
+
+@pytest.mark.parametrize("signal,xsph", [("1", 0.0), ("0", 0.0), ("1", 2000.0)])
+@pytest.mark.parametrize("n", [1, 300, 66000])
+def test_advance_equals_its_substeps(bbx, monkeypatch, signal, xsph, n):
+    """sph_advance queues the next substep's grid pass before this one's force
+    is known; the state is that of the same substeps one by one."""
+    monkeypatch.setenv("BBX_LOOP_SIGNAL", signal)
+    sc = _scene(n)
+    a, b = (bbx.Solver(sc, kind=bbx.SPH, pseudo_viscosity=xsph) for _ in range(2))
+    for interval in (2.5e-4, 1.2e-3):
+        steps, left = a.sph_advance(interval), interval
+        for _ in range(steps):
+            dt = left / b.number_of_time_steps(left, 1.0)
+            b.sph_substep(dt)
+            left -= dt
+        assert left <= float(np.float32(1e-4)) < left + dt  # the rule's constant is an FP32 one
+        for k in ("position", "velocity", "force", "density"):
+            np.testing.assert_array_equal(a.get(k), b.get(k))
+        for x, y in zip(a.chains(), b.chains()):
+            np.testing.assert_array_equal(x, y)
