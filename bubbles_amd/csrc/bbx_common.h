@@ -43,7 +43,7 @@ constexpr int kTabIntsHost = 48;           // ints per tile table (see bbx_tile.
 // Up to this many particles the chip is not full with one lane per particle,
 // and what a kernel takes is one lane's chain of latencies: the bucket build
 // gives a particle four.
-constexpr int kSmallSet = 65536;
+constexpr int kSmallSet = 224 * kBlock;
 constexpr int kBinCells = 65536;           // grids up to this many cells always get key bins (264 bytes a cell)
 // LDS tile capacity in particles (bbx_tile.h): 2528 float4 (+ the tile
 // table) lets four single-array or two two-array workgroups share a CU's

@@ -879,7 +879,15 @@ __device__ __forceinline__ void warm_start_one(const WarmIn &wi, int i, float4 p
     wi.xq[i] = make_float4(pi.x, pi.y, pi.z, (fabsf(d2) < 1e-8f) ? 0.f : p / d2);
 }
 
-template <bool kPressure, int kFeat>
+// Up to kOwnTables particles -- four workgroups on every CU, all resident at
+// once -- the tables cost one workgroup's latency instead of a launch; above,
+// every round of workgroups would pay it.  Bucket kernel + table kernel / with
+// own tables (us): 30.5 + 5.6 / 31.8 at 94k, 65.5 + 5.4 / 66.9 at 255k,
+// 178.0 + 6.0 / 186.4 at 1M, 224.4 + 6.0 / 235.9 there with the network.
+constexpr int kOwnTables = 4 * 256 * kBlock;
+// kOwnTab: the first wave makes the tile's table here, beside the row-bound
+// loads, instead of a launch before this one.
+template <bool kPressure, int kFeat, bool kOwnTab>
 __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
                                                             const float4 *__restrict__ pos,
                                                             const int *__restrict__ home,
@@ -889,7 +897,7 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
                                                             int *__restrict__ nbr_cnt,
                                                             float *__restrict__ rho,
                                                             float *__restrict__ pres,
-                                                            const int *__restrict__ tile_tab,
+                                                            int *__restrict__ tile_tab,
                                                             int *__restrict__ counters,
                                                             WarmIn wi) {
     // staged candidate positions (16-byte LDS DMA); eight slack slots let
@@ -902,7 +910,7 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
     // below then waits for nothing but it, not for the row bounds requested
     // in between, and needs no workgroup barrier (the LDS copy that the rest
     // of the kernel reads is visible after the barrier behind the staging).
-    const int tw = tab_load_wave(tile_tab + (size_t)tile * kTabInts);
+    const int tw = kOwnTab ? 0 : tab_load_wave(tile_tab + (size_t)tile * kTabInts);
     const int i = tile * kBlock + threadIdx.x;
     const bool valid = i < c.n;
     const int hc = valid ? home[i] : -1;
@@ -944,9 +952,18 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
             for (int q = 0; q < 4; q++) b[r][q] = start[min(max(cx - 1 + q, 0), last)];
         }
     }
-    if (threadIdx.x < kTabWords) reinterpret_cast<int *>(&tt)[threadIdx.x] = tw;
-    const bool staged = tab_word(tw, 1) != 0;
-    if (staged) tab_stage_dma_wave(tw, [&](int j, int e) { lds_dma16(pos + j, sx + e); });
+    bool staged;
+    if constexpr (kOwnTab) {
+        if (threadIdx.x < 64) tile_table(c, home, start, tile, (int)threadIdx.x, tt);
+        __syncthreads();
+        staged = tt.staged != 0;
+        if (staged) tab_stage_dma(tt, [&](int j, int e) { lds_dma16(pos + j, sx + e); });
+        tab_store(tile_tab + (size_t)tile * kTabInts, tt);
+    } else {
+        if (threadIdx.x < kTabWords) reinterpret_cast<int *>(&tt)[threadIdx.x] = tw;
+        staged = tab_word(tw, 1) != 0;
+        if (staged) tab_stage_dma_wave(tw, [&](int j, int e) { lds_dma16(pos + j, sx + e); });
+    }
     if (hc >= 0) {
 #pragma unroll
         for (int r = 0; r < 9; r++) {
@@ -1094,9 +1111,9 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
 // a crowded row or more neighbours than the cap is walked cell by cell by its
 // first lane.
 //
-// Used up to kSmallSet.  Measured (us, one lane per particle and the kernel
-// of its tile tables / four): 28.2 / 12.9 at 2k, 31.0 / 14.7 at 16k, 33.5 / 25.5
-// at 35k, 32.1 / 30.5 at 65k, 35.5 / 40.0 at 94k, 71.9 / 121.8 at 255k, where
+// Used up to kSmallSet.  Measured (us, one lane per particle / four): 25.2 / 12.9
+// at 2k, 27.2 / 15.0 at 16k, 30.2 / 25.6 at 35k, 28.6 / 27.1 at 49k, 29.0 / 28.7
+// at 58k, 29.0 / 30.8 at 65k, 31.8 / 40.0 at 94k, 66.9 / 121.8 at 255k, where
 // the chip is full and the four workgroups' staging and the longer emission
 // count.
 constexpr int kSplitLanes = 4;
@@ -1476,7 +1493,7 @@ int build_buckets(bbx_solver *s, bool with_pressure, int feat_mode, const StepCo
     SimConst &c = s->sc;
     const int n = s->n;
     if (n > 0) {
-        if (n > kSmallSet) {  // smaller sets' bucket kernel makes its own
+        if (n > kOwnTables) {  // smaller sets' bucket kernels make their own
             BBX_PROF_BEGIN("tile_tables");
             k_tile_tables<<<(unsigned)((s->ntiles + kTabWaves - 1) / kTabWaves), kBlock, 0, s->stream>>>(
                 c, s->home, s->cell_start, s->ntiles, s->tile_tab);
@@ -1501,7 +1518,8 @@ int build_buckets(bbx_solver *s, bool with_pressure, int feat_mode, const StepCo
             c, s->posA, s->home, s->cell_start, s->nbr16, s->nbr32, s->nbr_cnt, s->rho, s->pres, s->tile_tab, \
             s->counters, wi);                                                                                 \
     else                                                                                                      \
-        k_buckets_density<P, F><<<nblocks(n), kBlock, 0, s->stream>>>(                                        \
+        (n <= kOwnTables ? k_buckets_density<P, F, true> : k_buckets_density<P, F, false>)                    \
+            <<<nblocks(n), kBlock, 0, s->stream>>>(                                                           \
             c, s->posA, s->home, s->cell_start, s->nbr16, s->nbr32, s->nbr_cnt, s->rho, s->pres, s->tile_tab, \
             s->counters, wi)
         if (with_pressure) {

@@ -1,5 +1,5 @@
 """The bucket build's two kernels: four lanes per particle for small sets (up
-to 65,536 particles) and one lane per particle above.
+to 57,344 particles) and one lane per particle above.
 
 Buckets are exact against the FP64 oracle.  A density is an FP32 sum of at
 most 100 non-negative terms with compensation; each term has a few roundings
@@ -50,10 +50,12 @@ def test_split_buckets_match_oracle(bbx, oracle, n, spacing):
     assert st.bucket_overflows == np.maximum(within - 100, 0).sum()
 
 
-def test_both_kernels_agree_at_the_boundary(bbx):
-    """65,536 particles take the split kernel; the same with one more, far
-    away, the other: the same buckets, features and network pressures."""
-    p = _points(65536, 0.01)
+@pytest.mark.parametrize("n", [57344, 262144])
+def test_both_kernels_agree_at_the_boundary(bbx, n):
+    """57,344 particles take the split kernel, 262,144 the one that makes its
+    tiles' tables; the same with one more, far away, the next kernel: the same
+    buckets, features and network pressures."""
+    p = _points(n, 0.01)
     extra = np.array([[0.9, 0.4, 0.9]], dtype=np.float32).astype(np.float64)
     assert np.abs(p).max() < 0.5
     res = []
@@ -64,7 +66,7 @@ def test_both_kernels_agree_at_the_boundary(bbx):
         s.distribute()
         counts, ids = s.buckets()
         s.pcisph_substep(5e-4, 1, 0.01, bbx.MODE_TEXTBOOK, bbx.WARM_MLP)
-        res.append([x[:65536] for x in (counts, ids, s.get("density"), s.get("features"), s.get("warm_pressure"))])
+        res.append([x[:n] for x in (counts, ids, s.get("density"), s.get("features"), s.get("warm_pressure"))])
         s.close()
     a, b = res
     assert_buckets_equal((a[0], a[1]), (b[0], b[1]))
