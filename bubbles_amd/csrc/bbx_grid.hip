@@ -6,8 +6,10 @@
 // with a counting sort into cell-contiguous storage:
 //
 //   1. hash      one thread per particle: FP64 cell hash, sort key, atomic count
+//                (and the key into its cell's bin)
 //   2. scan      exclusive prefix sum of the cell counts (wave64 shuffles + LDS)
-//   3. scatter   place each particle in its cell's segment (arrival order)
+//   3. scatter   place each particle in its cell's segment (arrival order; not
+//                where there are bins)
 //   4. rank+move rank every particle inside its cell by key and move x, v
 //   5. buckets   per particle, walk the 27 cells in (y,x,z) order, apply the
 //                reference's FP64 cutoff, keep the first 100 -- fused with the

@@ -1,9 +1,9 @@
 // bbx_sph.hip -- SPH / PCISPH gathers, prediction and integration on gfx950.
 //
-// Every kernel is one thread per particle in cell-sorted storage order.  A
-// workgroup's 256 particles form a tile: the tile's candidate intervals
-// (recorded by the bucket kernel) are first copied into LDS with coalesced
-// loads, then each thread walks its bucket -- LDS-local 16-bit indices in
+// Every kernel is one or two threads per particle in cell-sorted storage
+// order.  A workgroup's 256 particles form a tile: the tile's candidate
+// intervals (its table) are first copied into LDS by LDS DMA, then each thread
+// walks its bucket -- LDS-local 16-bit indices in
 // the quad-major table (four entries per load) -- reading neighbours from LDS.
 // Tiles too large to stage walk 32-bit storage indices and read global
 // memory instead.  Fusions relative to the reference's launch sequence
@@ -13,6 +13,7 @@
 //   predicted density + pressure     PredictPressureFor, FP64 max-error reduction
 //   pressure force + predict(k+1)    PredictPressureForceFor + PredictVelocityAndPositionFor
 //   pressure force + integrate       PredictPressureForceFor + AccumulateForcesFor + TimeIntegrationFor
+//   SPH forces + integrate           ComputeAllForcesFor + TimeIntegrationFor
 //
 // Arithmetic is FP32; density and pressure-force sums use Kahan compensation.
 #include "bbx_collider.h"

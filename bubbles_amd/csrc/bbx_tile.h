@@ -5,9 +5,9 @@
 // 27-cell neighbourhoods of a tile's cells [cmin, cmax] are covered by nine
 // contiguous storage ranges, one per (dy, dz) row offset:
 //     cells [cmin + dy*nx + dz*nx*ny - 1, cmax + dy*nx + dz*nx*ny + 1].
-// The bucket kernel merges them into at most nine disjoint intervals,
-// records them per tile, stages the candidates in LDS and writes each
-// bucket as 16-bit LDS-local indices.  Every later gather of the substep
+// They are merged into at most nine disjoint intervals, which the tile's
+// table records; the bucket kernel stages the candidates in LDS and writes
+// each bucket as 16-bit LDS byte offsets.  Every later gather of the substep
 // re-stages the same intervals (coalesced loads) and reads neighbours from
 // LDS.  A tile whose intervals hold more than kTileCap particles keeps
 // 32-bit storage indices and reads neighbours from global memory.

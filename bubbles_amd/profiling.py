@@ -33,7 +33,6 @@ SHORT = {
     "k_hash": "grid_hash", "k_tile_tables": "tile_tables", "k_scatter": "grid_scatter", "k_rank_move": "grid_rank_move",
     "k_rank_bins": "grid_rank_move", "k_scan_small": "grid_scan",
     "k_scan_block": "grid_scan", "k_scan_add": "grid_scan_add", "k_scan_add_reduce": "grid_scan_add",
-    "k_zero_int2": "grid_clear",
     "k_buckets_density<false, 0>": "buckets_density", "k_buckets_density<true, 0>": "buckets_density_tait",
     "k_buckets_density<false, 1>": "buckets_density_features",
     "k_buckets_density<false, 2>": "buckets_density_warm",
@@ -42,15 +41,24 @@ SHORT = {
     "k_mlp_infer": "mlp_infer",
     "k_warm_init": "warm_init", "k_predict_pressure": "predict_pressure",
     "k_pressure_force": "pressure_force", "k_stream_copy": "stream_copy",
-    "k_sph_force": "sph_force", "k_integrate": "integrate", "k_xsph": "xsph",
+    "k_sph_step": "sph_step", "k_xsph": "xsph", "k_by_id": "download",
+    "k_buckets_density_split<false, 0>": "buckets_density", "k_buckets_density_split<true, 0>": "buckets_density_tait",
+    "k_buckets_density_split<false, 1>": "buckets_density_features",
+    "k_buckets_density_split<false, 2>": "buckets_density_warm",
     "k_density": "density", "k_fill_int": "fill",
 }
 
 
 def short_name(kernel: str) -> str:
     base = kernel.split("(")[0].replace("void ", "").strip()
-    base = base.split("::")[-1]
-    return SHORT.get(base, base)
+    base = full = base.split("::")[-1]
+    # variants of one kernel (a collider list, own tile tables, ...) come last
+    # among its template arguments and share its name
+    while base not in SHORT and "<" in base:
+        head, args = base.rstrip(">").split("<")
+        args = args.split(", ")[:-1]
+        base = f"{head}<{', '.join(args)}>" if args else head
+    return SHORT.get(base, full)
 
 
 def loop_kernel_split(trace_csv: str, threshold_us: float = 15.0):
