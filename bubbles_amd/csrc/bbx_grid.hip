@@ -546,20 +546,25 @@ __global__ void __launch_bounds__(kBlock) k_rank_bins(SimConst c, const int *__r
 // ---------------------------------------------------------------------------
 // The tile's home cells span [cmin, cmax]; its nine neighbour rows become at
 // most nine merged storage intervals (tab_row, tab_merge).  Every gather of
-// the substep reads this table.  Storage is sorted by cell except for the
-// particles in no chain (home -1) at its end, so unless the tile's last
-// particle is one of those, cmin and cmax are the homes of its first and
-// last particles (otherwise a wave reduction over the tile finds them).  The
-// row ranges of lanes 0-8 are gathered by shuffles and merged by lane 0.
+// the substep reads this table.  Storage is sorted by cell up to
+// start[total], so for a tile of chained particles cmin and cmax are the
+// homes of its first and last ones.  Behind them lie the particles in no
+// chain in no order: outside the grid (home -1, no neighbours), or inside it
+// after a jump that an incremental pass does not follow.  The latter look
+// for neighbours from homes anywhere and are no candidates themselves, so
+// that their own positions are in no interval: their tiles are not staged.
+// A tile with any particle in no chain takes a wave reduction.  The row
+// ranges of lanes 0-8 are gathered by shuffles and merged by lane 0.
 // (one wave; lane 0's table is complete when the wave has synchronised)
 __device__ __forceinline__ void tile_table(const SimConst &c, const int *__restrict__ home,
                                            const int *__restrict__ start, int tile, int lane, TileTab &tt) {
     const int t0 = tile * kBlock, t1 = min(t0 + kBlock, c.n) - 1;
-    int lo = 0x7fffffff, hi = home[t1];
-    const int first = home[t0];
-    if (hi >= 0) {
-        lo = first;
-    } else {
+    const int chained = start[c.g.total];
+    int lo = home[t0], hi = home[t1], cap = c.tile_cap;
+    if (t1 >= chained) {
+        lo = 0x7fffffff;
+        hi = -1;
+        bool astray = false;
 #pragma unroll
         for (int k = 0; k < kBlock / 64; k++) {
             const int i = t0 + k * 64 + lane;
@@ -567,10 +572,12 @@ __device__ __forceinline__ void tile_table(const SimConst &c, const int *__restr
             if (hc >= 0) {
                 lo = min(lo, hc);
                 hi = max(hi, hc);
+                astray = astray || i >= chained;
             }
         }
         lo = wave_min_i32(lo);
         hi = wave_max_i32(hi);
+        if (__any(astray)) cap = -1;  // no total is within it
     }
     int a = -1, b = -1;
     if (lane < 9) tab_row(c.g, hi >= 0 ? lo : 0, hi, start, lane, a, b);
@@ -580,7 +587,7 @@ __device__ __forceinline__ void tile_table(const SimConst &c, const int *__restr
         ra[r] = __shfl(a, r, 64);
         rb[r] = __shfl(b, r, 64);
     }
-    if (lane == 0 && !tab_merge_ordered(ra, rb, c.tile_cap, tt)) tab_merge(ra, rb, c.tile_cap, tt);
+    if (lane == 0 && !tab_merge_ordered(ra, rb, cap, tt)) tab_merge(ra, rb, cap, tt);
 }
 
 constexpr int kTabWaves = kBlock / 64;
@@ -1049,7 +1056,8 @@ __global__ void __launch_bounds__(kBlock) k_buckets_density(SimConst c,
         // the table this lane has just written (its own quads: no other lane
         // or wave writes them, and no earlier load in this kernel cached them)
         __builtin_amdgcn_s_waitcnt(0);
-        // The particle's own index (its LDS slot in the centre row).  Dead
+        // The particle's own index (its LDS slot in the centre row: a staged
+        // tile's particles with neighbours are all candidates).  Dead
         // entries of the last quad read the particle itself: its staged copy
         // is its position bit for bit, so they add exact zeros to the
         // feature sums below, as the particle's own entry does, and only
