@@ -132,10 +132,10 @@ __device__ __forceinline__ float poly6_w_member(const SimConst &c, float d2) {
     return c.poly6 * x * x * x;
 }
 
-// The same rule as a factor: 1 inside, 0 outside.  Clamping is a modifier of
-// the instruction (v_fma_f32 with clamp takes two cycles a wave; a compare
-// and a select take seven): the next value above -1e-8 maps to 0, -1e-8
-// itself to 2^60 of their distance, far above 1.
+// The same rule as a factor: 1 inside, 0 outside and for a NaN.  Clamping is
+// a modifier of the instruction (v_fma_f32 with clamp takes two cycles a wave;
+// a compare and a select take seven): the next value above -1e-8 maps to 0,
+// -1e-8 itself to 2^60 of their distance, far above 1.
 __device__ __forceinline__ float cutoff_mask(float of) {
     constexpr float kScale = 1152921504606846976.f;                            // 2^60
     constexpr float kAbove = -__builtin_bit_cast(float, __builtin_bit_cast(unsigned, 1e-8f) - 1u);
@@ -151,7 +151,14 @@ __device__ __forceinline__ float one_minus(float a, float scale) {
     return __builtin_amdgcn_fmed3f(fmaf(-a, scale, 1.f), 0.f, 1.f);
 }
 
-// poly6 W of the factor x = 1 - d^2 / h^2, rounded before it enters a sum
+// The factor x = 1 - d^2 / h^2 of poly6 under its own cutoff.  The clamp
+// changes nothing inside; outside it keeps x finite, and a distance that has
+// overflowed or is not a number gives exactly zero, as poly6_w does.
+__device__ __forceinline__ float poly6_x(const SimConst &c, float d2) {
+    return __builtin_amdgcn_fmed3f(1.f - d2 * c.inv_h2, 0.f, 1.f) * cutoff_mask(d2 - c.h2);
+}
+
+// poly6 W of that factor, rounded before it enters a sum
 __device__ __forceinline__ float poly6_of(const SimConst &c, float x) {
 #pragma clang fp contract(off)
     return c.poly6 * x * x * x;
@@ -201,6 +208,15 @@ __device__ __forceinline__ PairFactor pair_factor(const SimConst &c, float dx, f
     const float ir = fast_rsq(d2);
     const float apart = __builtin_amdgcn_fmed3f(fmaf(d2, 1e30f, -1e14f), 0.f, 1.f);
     return PairFactor{one_minus(d2 * ir, c.inv_h), ir * apart};
+}
+
+// a * b, zero where either is zero whatever the other one is (v_mul_legacy_f32)
+extern "C" __device__ float bbx_mul_legacy(float a, float b) __asm("llvm.amdgcn.fmul.legacy");
+
+// t x x ir for a pair's t = kg (q_i + q_j).  The factors that leave a pair out
+// (x = 0, ir = 0) make it an exact zero also where a pressure has overflowed.
+__device__ __forceinline__ float pair_gradient(float t, float x, float ir) {
+    return bbx_mul_legacy(bbx_mul_legacy(t, x) * x, ir);
 }
 
 // Reversed-box collider (ColliderSet3 with one container; CollisionHandle,

@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(kNpThreads) __attribute__((amdgpu_waves_per_eu
                 // kernel's pair rule; with d = x_i - x_j here, f_p = +sum g d
                 const PairFactor f = pair_factor(c, dx, dy, dz);
                 const float xp = kL || live ? f.x : 0.f;
-                const float g = kg * (qi + a.w) * xp * xp * f.ir;
+                const float g = pair_gradient(kg * (qi + a.w), xp, f.ir);
                 kahan_fma(px, epx, g, dx);
                 kahan_fma(py, epy, g, dy);
                 kahan_fma(pz, epz, g, dz);
@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(kPpThreads) k_predict_pressure(SimConst c, Ste
                 const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
                 // poly6; zero outside, and for a dead entry
                 const float d2 = dx * dx + dy * dy + dz * dz;
-                float x = (1.f - d2 * c.inv_h2) * cutoff_mask(d2 - c.h2);
+                float x = poly6_x(c, d2);
                 if (!kS) x = live ? x : 0.f;
                 kahan_add(sum, comp, poly6_of(c, x));
             }, half);
@@ -448,7 +448,7 @@ __global__ void __launch_bounds__(kBlock) k_pressure_force(SimConst c, StepConst
                 const float dx = a.x - xi.x, dy = a.y - xi.y, dz = a.z - xi.z;
                 const PairFactor f = pair_factor(c, dx, dy, dz);
                 const float x = kS || live ? f.x : 0.f;  // zero outside, and for a dead entry
-                const float g = kg * (qi + a.w) * x * x * f.ir;
+                const float g = pair_gradient(kg * (qi + a.w), x, f.ir);
                 kahan_fma(tx, ex, g, dx);
                 kahan_fma(ty, ey, g, dy);
                 kahan_fma(tz, ez, g, dz);
@@ -560,7 +560,7 @@ __global__ void __launch_bounds__(kSphThreads) k_sph_step(SimConst c, StepConst 
                 const float dx = a.x - xi.x, dy = a.y - xi.y, dz = a.z - xi.z;
                 const PairFactor f = pair_factor(c, dx, dy, dz);
                 const float x = kL || live ? f.x : 0.f;
-                const float g = kg * (qi + a.w) * x * x * f.ir;
+                const float g = pair_gradient(kg * (qi + a.w), x, f.ir);
                 kahan_fma(tx, ex, g, dx);
                 kahan_fma(ty, ey, g, dy);
                 kahan_fma(tz, ez, g, dz);
