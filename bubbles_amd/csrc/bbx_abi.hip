@@ -1540,14 +1540,34 @@ static int published_sph(bbx_solver *s, bbx_stats *st) {
     return BBX_OK;
 }
 
-// A substep in three parts: what its time step has no part in (grid pass and
-// buckets), the step itself, and its statistics with the largest force.
-static int sph_front(bbx_solver *s) {
-    BBX_CHECK(distribute_grid(s, false, -1, (int *)s->max_force, kStepClear));
-    return build_buckets(s, true, 0, nullptr);
+// A substep in three parts: the grid pass, which its time step has no part
+// in; buckets and the step itself; its statistics with the largest force.
+static int sph_grid(bbx_solver *s) { return distribute_grid(s, false, -1, (int *)s->max_force, kStepClear); }
+
+// Take back a grid pass that was queued for a step that is not made after
+// all: it wrote to the other halves of the ping-pong, so the state before it
+// is still there; the flag it consumed is in its counters, and the cell table
+// counts the chains of the cells as they were.
+static int sph_grid_undo(bbx_solver *s) {
+    BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
+    std::swap(s->posA, s->posB);
+    std::swap(s->velA, s->velB);
+    std::swap(s->cellA, s->cellB);
+    int full = 0;
+    BBX_HIP_CHECK(hipMemcpy(&full, &s->counters[CNT_FULL], sizeof(int), hipMemcpyDeviceToHost));
+    BBX_CHECK(launch_fill_int(s, s->flag, full, 1));
+    std::vector<int> cell((size_t)s->n), start((size_t)s->grid.total + 1, 0);
+    BBX_HIP_CHECK(hipMemcpy(cell.data(), s->cellA, sizeof(int) * cell.size(), hipMemcpyDeviceToHost));
+    for (int c : cell)
+        if ((unsigned)c < s->grid.total) start[(size_t)c + 1]++;
+    for (size_t c = 1; c < start.size(); c++) start[c] += start[c - 1];
+    BBX_HIP_CHECK(hipMemcpy(s->cell_start, start.data(), sizeof(int) * start.size(), hipMemcpyHostToDevice));
+    BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
+    return BBX_OK;
 }
 
 static int sph_back(bbx_solver *s, double dt) {
+    BBX_CHECK(build_buckets(s, true, 0, nullptr));
     s->maxf_cached = false;
     s->loop_seq++;  // numbers this substep's published words
     StepConst st{};
@@ -1572,12 +1592,44 @@ static int check_sph_step(bbx_solver *s, double dt) {
     if (!(dt > 0)) return fail(BBX_E_INVALID, "dt must be > 0");
     return BBX_OK;
 }
+
+// Advance's substeps.  Whether one follows is known before this one's largest
+// force is, which decides the next one's length alone: the next one's grid
+// pass is queued first, and the device works while the host waits for the
+// force, chooses dt and queues the rest (7 substeps of 16k particles:
+// 409 -> 374 us; 12 of 241k: 2,173 -> 2,119).  Its buckets are not: they
+// overwrite what the last substep left, and an error may end the call here.
+// Not where the statistics are copied: the grid pass clears
+// them.  *queued: a grid pass is queued whose step is not.
+static int sph_substeps(bbx_solver *s, double interval, int *steps, bool *queued) {
+    double remaining = interval;
+    while (remaining > (double)0.0001f) {
+        unsigned n = 0;
+        BBX_CHECK(time_steps(s, remaining, 1.0, &n));
+        if (n == 0) return fail(BBX_E_INVALID, "time-step rule returned 0");
+        const double dt = remaining / (double)n;
+        BBX_CHECK(check_sph_step(s, dt));
+        if (!*queued) BBX_CHECK(sph_grid(s));
+        *queued = false;
+        BBX_CHECK(sph_back(s, dt));
+        remaining -= dt;
+        (*steps)++;
+        if (remaining > (double)0.0001f && sph_publishes(s)) {
+            BBX_CHECK(sph_grid(s));
+            *queued = true;
+        }
+        bbx_stats local{};
+        BBX_CHECK(sph_stats(s, &local));
+        if (s->prof.enabled) s->prof.resolve();
+    }
+    return BBX_OK;
+}
 extern "C" {
 
 int bbx_sph_substep(bbx_solver *s, double dt, bbx_stats *stats) {
     BBX_CHECK(check_sph_step(s, dt));
     BBX_HIP_CHECK(hipEventRecord(s->ev0[0], s->stream));
-    BBX_CHECK(sph_front(s));
+    BBX_CHECK(sph_grid(s));
     BBX_CHECK(sph_back(s, dt));
     BBX_HIP_CHECK(hipEventRecord(s->ev1[0], s->stream));
     bbx_stats local{};
@@ -1591,29 +1643,16 @@ int bbx_sph_substep(bbx_solver *s, double dt, bbx_stats *stats) {
 
 int bbx_sph_advance(bbx_solver *s, double interval, int *substeps) {
     BBX_CHECK(check_setup(s));
-    double remaining = interval;
     int steps = 0;
-    // Whether a substep follows is known before this one's largest force is,
-    // which decides the next one's length alone: the next one's grid pass and
-    // buckets are queued first, and the device works while the host waits for
-    // the force, chooses dt and queues the step (16k particles, Advance(1e-3):
-    // 392 -> 370 us).  Not where the statistics are copied: the grid pass clears them.
-    bool front = false;
-    while (remaining > (double)0.0001f) {
-        unsigned n = 0;
-        BBX_CHECK(time_steps(s, remaining, 1.0, &n));
-        if (n == 0) return fail(BBX_E_INVALID, "time-step rule returned 0");
-        const double dt = remaining / (double)n;
-        BBX_CHECK(check_sph_step(s, dt));
-        if (!front) BBX_CHECK(sph_front(s));
-        BBX_CHECK(sph_back(s, dt));
-        remaining -= dt;
-        steps++;
-        front = remaining > (double)0.0001f && sph_publishes(s);
-        if (front) BBX_CHECK(sph_front(s));
-        bbx_stats local{};
-        BBX_CHECK(sph_stats(s, &local));
-        if (s->prof.enabled) s->prof.resolve();
+    bool queued = false;
+    const int rc = sph_substeps(s, interval, &steps, &queued);
+    if (rc != BBX_OK) {
+        if (queued) {
+            const std::string why = g_last_error;
+            (void)sph_grid_undo(s);
+            g_last_error = why;
+        }
+        return rc;
     }
     BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
     if (substeps) *substeps = steps;
