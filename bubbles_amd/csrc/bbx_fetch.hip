@@ -106,6 +106,14 @@ void fetch_free(bbx_solver *s) {
     s->fetch = nullptr;
 }
 
+// what the kernel saw of the id table; the field is not given out where it is corrupt
+static int check_ids(const bbx_solver *s) {
+    const FetchRing *r = s->fetch;
+    if (__atomic_load_n((const int *)(r->ring + r->bytes), __ATOMIC_ACQUIRE))
+        return fail(BBX_E_INVALID, "corrupt particle id table");
+    return BBX_OK;
+}
+
 namespace {
 
 // Below this many floats the threads' start costs more than they save: with
@@ -133,9 +141,10 @@ struct Pipe {
         BBX_HIP_CHECK(hipEventRecord(s->fetch->ev[c % kFetchSlots], s->stream));
         return BBX_OK;
     }
+    // before any chunk is taken: the kernel has looked at every id by then
     int arrive(int c) const {
         BBX_HIP_CHECK(hipEventSynchronize(s->fetch->ev[c % kFetchSlots]));
-        return BBX_OK;
+        return check_ids(s);
     }
     int one_thread() const {
         for (int c = 0; c < std::min(chunks, kFetchSlots); c++) BBX_CHECK(send(c));
@@ -203,7 +212,8 @@ int fetch_by_id(bbx_solver *s, const FieldSource &f, const FetchTake &take) {
     if (all * sizeof(float) <= r->bytes) {
         BBX_CHECK(launch_by_id(s, f, 0, s->n, (float *)r->d_ring));
         BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
-        if (!__atomic_load_n(bad, __ATOMIC_ACQUIRE)) take.run((const float *)r->ring, 0, all);
+        BBX_CHECK(check_ids(s));
+        take.run((const float *)r->ring, 0, all);
     } else {
         // posB holds nothing between calls: 4 floats a particle
         float *scratch = reinterpret_cast<float *>(s->posB);
@@ -220,7 +230,6 @@ int fetch_by_id(bbx_solver *s, const FieldSource &f, const FetchTake &take) {
             }
         }
     }
-    if (__atomic_load_n(bad, __ATOMIC_ACQUIRE)) return fail(BBX_E_INVALID, "corrupt particle id table");
     return BBX_OK;
 }
 
