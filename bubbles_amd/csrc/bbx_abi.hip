@@ -788,7 +788,8 @@ int bbx_solver_reserve(bbx_solver *s, int capacity) {
     BBX_HIP_CHECK(hipMemcpy(s->home + n, none.data(), sizeof(int) * none.size(), hipMemcpyHostToDevice));
     s->stride = (int)S1;
     fill_sim_const(s);
-    return fetch_grow(s, S1);
+    fetch_grow(s, S1);
+    return BBX_OK;
 }
 
 int bbx_solver_capacity(bbx_solver *s, int *capacity) {

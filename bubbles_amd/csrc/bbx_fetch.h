@@ -37,7 +37,8 @@ protected:
 // bytes of the ring for a solver of that capacity (and 64 for the flag word)
 size_t fetch_ring_bytes(size_t stride);
 int fetch_init(bbx_solver *s, char *pinned, char *device, size_t bytes);
-int fetch_grow(bbx_solver *s, size_t stride);
+// a larger ring for a set that has grown; without one the smaller one serves
+void fetch_grow(bbx_solver *s, size_t stride);
 void fetch_free(bbx_solver *s);
 int fetch_by_id(bbx_solver *s, const FieldSource &f, const FetchTake &take);
 // n FP64 vectors (null: zeros) as FP32 rows of dst, the rest of `rows` zero;

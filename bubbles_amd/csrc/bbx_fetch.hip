@@ -80,20 +80,21 @@ int fetch_init(bbx_solver *s, char *pinned, char *device, size_t bytes) {
     return BBX_OK;
 }
 
-int fetch_grow(bbx_solver *s, size_t stride) {
+void fetch_grow(bbx_solver *s, size_t stride) {
+    FetchRing *r = s->fetch;
     const size_t want = fetch_ring_bytes(stride);
-    if (s->fetch->bytes >= want) return BBX_OK;
+    if (r->bytes >= want) return;
     char *p = nullptr, *d = nullptr;
-    if (hipHostMalloc((void **)&p, want + 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
-        return fail(BBX_E_NOMEM, "pinned alloc");
-    const hipError_t e = hipHostGetDevicePointer((void **)&d, p, 0);
-    if (e != hipSuccess) {
-        (void)hipHostFree(p);
-        return fail(BBX_E_HIP, std::string("fetch ring: ") + hipGetErrorString(e));
+    if (hipHostMalloc((void **)&p, want + 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+        hipHostGetDevicePointer((void **)&d, p, 0) != hipSuccess) {
+        if (p) (void)hipHostFree(p);
+        (void)hipGetLastError();
+        return;
     }
-    if (s->fetch->own) (void)hipHostFree(s->fetch->own);
-    s->fetch->own = p;
-    return fetch_init(s, p, d, want);
+    if (r->own) (void)hipHostFree(r->own);
+    r->own = r->ring = p;
+    r->d_ring = d;
+    r->bytes = want;
 }
 
 void fetch_free(bbx_solver *s) {

@@ -1,6 +1,8 @@
 """Downloads where something failed: a corrupt id table gives an error before
-anything is written, whatever the field's route.  Each case runs in a process
-of its own, where tests/cpp/hip_faults.c stands before the HIP runtime."""
+anything is written, whatever the field's route, and a set that has grown
+without a larger pinned ring comes through the smaller one.  Each case runs in
+a process of its own, where tests/cpp/hip_faults.c stands before the HIP
+runtime."""
 import os
 import subprocess
 import sys
@@ -46,6 +48,31 @@ for field in ("position", "velocity", "density", "features"):
 print("done")
 """
 
+GROWN = """
+sc = scene(13, 5, 3)
+more = scene(36, 36, 36).positions
+parts = [sc.positions, more, more]
+fields = []
+for fail in (1, 0):
+    s = abi.Solver(sc)
+    word("faults_host_malloc").value = fail
+    s.reserve(60000)
+    assert word("faults_host_malloc").value == 0 and s.capacity() >= 60000
+    s.append(more)
+    both = np.concatenate(parts[:2]).astype(np.float32).astype(np.float64)
+    assert np.array_equal(s.get("position"), both)
+    word("faults_host_malloc").value = fail
+    s.append(more)  # grows by itself
+    both = np.concatenate(parts).astype(np.float32).astype(np.float64)
+    assert np.array_equal(s.get("position"), both)
+    s.distribute()
+    fields.append([s.get(f) for f in ("position", "density", "features")])
+    word("faults_host_malloc").value = 0
+for a, b in zip(*fields):
+    assert np.array_equal(a, b)
+print("done")
+"""
+
 
 @pytest.fixture(scope="module")
 def faults(bbx, tmp_path_factory):
@@ -64,3 +91,7 @@ def _run(faults, code, *args):
 @pytest.mark.parametrize("dims", [(20, 15, 10), (100, 60, 60), (100, 50, 101)])
 def test_corrupt_ids_write_nothing(faults, dims):
     _run(faults, CORRUPT, *dims)
+
+
+def test_growth_without_a_larger_ring(faults):
+    _run(faults, GROWN)
