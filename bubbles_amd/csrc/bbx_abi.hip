@@ -418,6 +418,18 @@ static void free_all(bbx_solver *s) {
     s->stream = nullptr;
 }
 
+// Key bins for the solver's grid and capacity, in place of those it has.
+// Without room for them the grid pass does without.
+static void alloc_bins(bbx_solver *s) {
+    const size_t cells = (size_t)s->grid.total + 1, N = (size_t)s->stride;
+    dfree(s->bins);
+    s->bin_pass = 0;
+    if (cells <= std::max((size_t)kBinCells, N) && dalloc(&s->bins, grid_bins_words(cells - 1, N)) != BBX_OK) {
+        s->bins = nullptr;
+        (void)hipGetLastError();
+    }
+}
+
 static int check_solver(bbx_solver *s) {
     if (!s) return fail(BBX_E_INVALID, "null solver");
     return BBX_OK;
@@ -551,10 +563,7 @@ int bbx_solver_create(int kind, const bbx_params *params, const double *pos, con
         s->counters = s->step->counters;
     }
     if (!rc) rc = dalloc(&s->flag, 1);
-    if (!rc && cells <= std::max((size_t)kBinCells, N) && dalloc(&s->bins, grid_bins_words(cells - 1)) != BBX_OK) {
-        s->bins = nullptr;  // no room: the grid pass does without
-        (void)hipGetLastError();
-    }
+    if (!rc) alloc_bins(s);
     // one pinned block (an allocation costs about 100 us): the loop signal,
     // the step block's copy, a flag, and the ring of the field downloads
     const size_t pin_step = 256, pin_flag = pin_step + (sizeof(StepBlock) + 255) / 256 * 256, pin_ring = pin_flag + 256;
@@ -787,6 +796,7 @@ int bbx_solver_reserve(bbx_solver *s, int capacity) {
     BBX_HIP_CHECK(hipMemcpy(s->cellA + n, none.data(), sizeof(int) * none.size(), hipMemcpyHostToDevice));
     BBX_HIP_CHECK(hipMemcpy(s->home + n, none.data(), sizeof(int) * none.size(), hipMemcpyHostToDevice));
     s->stride = (int)S1;
+    alloc_bins(s);
     fill_sim_const(s);
     fetch_grow(s, S1);
     return BBX_OK;

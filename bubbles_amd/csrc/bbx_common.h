@@ -44,7 +44,7 @@ constexpr int kTabIntsHost = 48;           // ints per tile table (see bbx_tile.
 // and what a kernel takes is one lane's chain of latencies: the bucket build
 // gives a particle four.
 constexpr int kSmallSet = 224 * kBlock;
-constexpr int kBinCells = 65536;           // grids up to this many cells always get key bins (264 bytes a cell)
+constexpr int kBinCells = 65536;           // grids up to this many cells always get key bins (256 bytes a cell)
 // LDS tile capacity in particles (bbx_tile.h): 2528 float4 (+ the tile
 // table) lets four single-array or two two-array workgroups share a CU's
 // 160 KB of LDS
@@ -258,8 +258,8 @@ struct bbx_solver {
     // cell table (total + 1 entries, the last one collects particles in no chain)
     int *cell_count = nullptr, *cell_start = nullptr;
     bool counts_clear = false;                 // cell_count is all zeros (a grid pass leaves it so)
-    // keys of each cell's particles and heads of the chains behind full bins
-    // (see k_hash); null for grids of many more cells than particles
+    // keys of each cell's particles and the blocks behind full bins (see
+    // k_hash); null for grids of many more cells than particles
     unsigned long long *bins = nullptr;
     unsigned bin_pass = 0;  // number of the last pass that used them
     int *scan_tmp = nullptr;
@@ -340,7 +340,7 @@ int distribute(bbx_solver *s, bool force_full, bool buckets, bool with_pressure,
 // tile tables + bucket build (the latter is where the warm start is chosen)
 // clear / clear_n: an int range set to zero on the way (the substep's step
 // block behind its counters, which this sets)
-size_t grid_bins_words(size_t cells);  // 8-byte words of the key bins and chain heads
+size_t grid_bins_words(size_t cells, size_t stride);  // 8-byte words of the key bins and the blocks behind them
 int distribute_grid(bbx_solver *s, bool force_full, int append_from, int *clear = nullptr,
                     size_t clear_n = 0);
 int build_buckets(bbx_solver *s, bool with_pressure, int feat_mode, const StepConst *st);
