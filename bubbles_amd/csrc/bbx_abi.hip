@@ -751,6 +751,7 @@ int bbx_solver_reserve(bbx_solver *s, int capacity) {
     if (S1 <= S0) return BBX_OK;
     const size_t n = (size_t)s->n;
     BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
+    dfree(s->bins);  // room for the fields first
     // particle state kept (first n slots), scratch and per-substep tables not
     BBX_CHECK(regrow(s, s->posA, S1, n));
     BBX_CHECK(regrow(s, s->velA, S1, n));
