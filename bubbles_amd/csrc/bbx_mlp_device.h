@@ -48,7 +48,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ unsigned short f2bf(float f) {
     return __builtin_bit_cast(unsigned short, (__bf16)f);
 }
-__device__ __forceinline__ float bf2f(unsigned short b) { return __uint_as_float((unsigned)b << 16); }
 
 __device__ __forceinline__ bf16x4 pack4(float a, float b, float c, float d) {
     typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
@@ -107,61 +106,7 @@ constexpr int kW1Row = kF + 4;                          // 20
 constexpr int kW2Row = kH + 4;                          // 68
 constexpr int kLdsWeights = kH * kW1Row + kH * kW2Row;  // BF16 entries
 
-// Staging for a 512-thread workgroup, split in two: the global loads are
-// issued early (before a long loop, to hide their latency) and the LDS
-// stores later.  P is 16-byte aligned (its own allocation), and so are both
-// weight blocks.  Thread t holds W1 float4 t (t < 256) and W2 float4s t and
-// t + 512, the layer biases and output weight of unit t (t < 64), and the
-// feature normalisation of its MFMA lane.
-struct InferPrefetch {
-    float4 w1, w2a, w2b;
-    float b1, b2, w3;
-    float mean[4], istd[4];
-};
-constexpr int kPrefetchThreads = 512;
-static_assert(kH * kF / 4 <= kPrefetchThreads && kH * kH / 4 == 2 * kPrefetchThreads && kH <= kPrefetchThreads,
-              "prefetch split");
-
-__device__ __forceinline__ void prefetch_infer(const float *__restrict__ P, int tid, InferPrefetch &f) {
-    const float4 *w1 = reinterpret_cast<const float4 *>(P + OFF_W1);
-    const float4 *w2 = reinterpret_cast<const float4 *>(P + OFF_W2);
-    f.w1 = tid < kH * kF / 4 ? w1[tid] : make_float4(0.f, 0.f, 0.f, 0.f);
-    f.w2a = w2[tid];
-    f.w2b = w2[tid + kPrefetchThreads];
-    f.b1 = f.b2 = f.w3 = 0.f;
-    if (tid < kH) {
-        f.b1 = P[OFF_B1 + tid];
-        f.b2 = P[OFF_B2 + tid];
-        f.w3 = P[OFF_W3 + tid];
-    }
-    const int q = (tid & 63) >> 4;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        f.mean[v] = P[OFF_MEAN + 4 * q + v];
-        f.istd[v] = P[OFF_ISTD + 4 * q + v];
-    }
-}
-
-// LDS side: BF16 weights into lw (one rounding of the FP32 parameters), b1 | b2 | w3 into lb
-__device__ __forceinline__ void store_infer_prefetch(const InferPrefetch &f, unsigned short *lw, float *lb,
-                                                     int tid) {
-    if (tid < kH * kF / 4)
-        *reinterpret_cast<bf16x4 *>(lw + (tid / (kF / 4)) * kW1Row + 4 * (tid % (kF / 4))) =
-            pack4(f.w1.x, f.w1.y, f.w1.z, f.w1.w);
-    unsigned short *lw2 = lw + kH * kW1Row;
-    const int ka = tid, kb = tid + kPrefetchThreads;
-    *reinterpret_cast<bf16x4 *>(lw2 + (ka / (kH / 4)) * kW2Row + 4 * (ka % (kH / 4))) =
-        pack4(f.w2a.x, f.w2a.y, f.w2a.z, f.w2a.w);
-    *reinterpret_cast<bf16x4 *>(lw2 + (kb / (kH / 4)) * kW2Row + 4 * (kb % (kH / 4))) =
-        pack4(f.w2b.x, f.w2b.y, f.w2b.z, f.w2b.w);
-    if (tid < kH) {
-        lb[tid] = f.b1;
-        lb[kH + tid] = f.b2;
-        lb[2 * kH + tid] = f.w3;
-    }
-}
-
-// The same LDS image written by a block of any size straight from the FP32
+// The LDS image of the weights, written by a block of any size from the FP32
 // parameters (each weight rounded to BF16 once): W1, W2, then b1 | b2 | w3.
 __device__ __forceinline__ void stage_infer_weights(const float *__restrict__ P, unsigned short *lw, float *lb,
                                                     int tid, int nthreads) {

@@ -70,13 +70,6 @@ __device__ __forceinline__ void tab_load_shared(const int *__restrict__ g, TileT
     if (threadIdx.x < kTabWords) dst[threadIdx.x] = g[threadIdx.x];
 }
 
-// LDS position of storage index j (j inside one of the intervals)
-__device__ __forceinline__ int tab_local(const TileTab &t, int j) {
-    for (int k = 0; k < t.n_ivl; k++)
-        if (j >= t.start[k] && j < t.start[k] + t.len[k]) return t.off[k] + (j - t.start[k]);
-    return -1;
-}
-
 // A staged tile's bucket entries are LDS byte offsets (slot << kSlotShift,
 // slot < kTileCap, so they fit 16 bits): a gather adds no shift per entry.
 constexpr int kSlotShift = 4;  // 16-byte slots
