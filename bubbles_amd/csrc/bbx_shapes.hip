@@ -23,8 +23,17 @@ struct bbx_sdf {
 
 namespace {
 
-constexpr int kSdfWaves = 4;  // waves that share a brick of 4 x 4 x 4 nodes
-constexpr int kSdfBlock = 64 * kSdfWaves;
+// Routes of a mesh's SDF, by triangles and nodes; whole from_mesh calls in us.
+// Up to kSdfFew triangles, or twice that on a grid that leaves the chip idle,
+// every pair is evaluated: bounds / all pairs 1 triangle 33 / 30, 8 and 1M nodes
+// 157 / 158, 12 and 16k nodes 48 / 42, 12 and 275k 70 / 81.  Up to a triangle per
+// lane, one wave has a brick of 4 x 4 x 4 nodes; above, four share it: four /
+// one 20 triangles and 730k nodes 181 / 109, 60 and 100k 177 / 140, 320 and 110k
+// 178 / 302.
+constexpr int kSdfFew = 8;
+constexpr long long kSdfFewNodes = 1 << 17;
+constexpr int kSdfOneWave = 64;
+constexpr int kSdfWaves = 4;
 
 __device__ __forceinline__ double sgn_d(double a) { return a > 0 ? 1.0 : (a < 0 ? -1.0 : 0.0); }
 __device__ __forceinline__ double clamp_d(double v, double lo, double hi) {
@@ -116,11 +125,8 @@ __device__ __forceinline__ float lane_of(float v, int l) {
 // grid.  A triangle that tri_dist2 cannot measure (an edge of no length, no
 // area, coordinates that are not finite) gets an infinite radius: it is never
 // passed over and bounds nothing.
-__global__ void __launch_bounds__(256) k_tri_spheres(const double *__restrict__ tri, int ntri, double ox, double oy,
-                                                     double oz, float slack, float4 *__restrict__ sphere) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ntri) return;
-    const double *v = tri + 9 * (size_t)t;
+__device__ __forceinline__ float4 tri_sphere(const double *__restrict__ v, double ox, double oy, double oz,
+                                             float slack) {
     const double cx = (v[0] + v[3] + v[6]) / 3.0, cy = (v[1] + v[4] + v[7]) / 3.0, cz = (v[2] + v[5] + v[8]) / 3.0;
     double r2 = 0.0, e2 = DBL_MAX;
     for (int k = 0; k < 3; k++) {
@@ -132,8 +138,34 @@ __global__ void __launch_bounds__(256) k_tri_spheres(const double *__restrict__ 
     const double wx = v[6] - v[0], wy = v[7] - v[1], wz = v[8] - v[2];
     const double nx = uy * wz - uz * wy, ny = uz * wx - ux * wz, nz = ux * wy - uy * wx;
     const bool sound = e2 > 0.0 && nx * nx + ny * ny + nz * nz > 0.0 && r2 < 1e30 && fabs(cx) + fabs(cy) + fabs(cz) < 1e30;
-    sphere[t] = make_float4((float)(cx - ox), (float)(cy - oy), (float)(cz - oz),
-                            sound ? (float)sqrt(r2) * 1.000001f + slack : __builtin_inff());
+    return make_float4((float)(cx - ox), (float)(cy - oy), (float)(cz - oz),
+                       sound ? (float)sqrt(r2) * 1.000001f + slack : __builtin_inff());
+}
+
+__global__ void __launch_bounds__(256) k_tri_spheres(const double *__restrict__ tri, int ntri, double ox, double oy,
+                                                     double oz, float slack, float4 *__restrict__ sphere) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < ntri) sphere[t] = tri_sphere(tri + 9 * (size_t)t, ox, oy, oz, slack);
+}
+
+// Every triangle's distance and solid angle at every node, a node per lane: what
+// the kernel below saves itself, for meshes and grids so small that its bounds
+// only lengthen each lane's chain.
+__global__ void __launch_bounds__(64) k_sdf_all_pairs(const double *__restrict__ tri, int ntri, int nx, int ny, int nz,
+                                                      double ox, double oy, double oz, double dx,
+                                                      float *__restrict__ out) {
+#pragma clang fp contract(off)
+    const unsigned node = blockIdx.x * 64u + threadIdx.x, row = node / (unsigned)nx;
+    if (node >= (unsigned)nx * ny * nz) return;  // below 2^31
+    const double px = ox + dx * (double)(node % (unsigned)nx), py = oy + dx * (double)(row % (unsigned)ny),
+                 pz = oz + dx * (double)(row / (unsigned)ny);
+    double best = DBL_MAX, wind = 0.0;
+    for (int t = 0; t < ntri; t++) {
+        best = fmin(best, tri_dist2(tri + 9 * t, px, py, pz));
+        wind += tri_solid_angle(tri + 9 * t, px, py, pz);
+    }
+    const double psd = fmax(sqrt(best), 0.00001);
+    out[node] = (float)(fabs(wind) > 2.0 * M_PI ? -psd : psd);  // |winding number| > 1/2
 }
 
 // SetNodeSDFKernel (src/core/shape.cpp:411-424) for a mesh: distance to the
@@ -142,7 +174,7 @@ __global__ void __launch_bounds__(256) k_tri_spheres(const double *__restrict__ 
 // mesh's bounds centre, src/core/shape.cpp:356-373).
 //
 // A workgroup holds a brick of 4 x 4 x 4 nodes, one per lane in each of its
-// waves, and splits the triangles between the waves.  FP64 distances and solid angles
+// waves, and splits the triangles between them.  FP64 distances and solid angles
 // of every (node, triangle) pair bounded the kernel (4.03 ms at 229k nodes
 // and 1,280 triangles, about 2,100 cycles per pair of a wave), so most pairs
 // get neither (0.31 ms; 34 to 2.1 ms at 572k nodes and 5,120 triangles of a
@@ -159,16 +191,18 @@ __global__ void __launch_bounds__(256) k_tri_spheres(const double *__restrict__ 
 //    node of a mesh that is not closed (or has a triangle without area),
 //    takes the whole sum in triangle order: at the surface and in an opening
 //    the winding number is 1/2 up to its rounding.
-__global__ void __launch_bounds__(kSdfBlock) k_sdf_from_mesh(const double *__restrict__ tri,
-                                                             const float4 *__restrict__ sphere, int ntri, int nx,
-                                                             int ny, int nz, double ox, double oy, double oz,
-                                                             double dx, float slack, int closed,
-                                                             float *__restrict__ out) {
+template <int kWaves>
+__global__ void __launch_bounds__(64 * kWaves) k_sdf_from_mesh(const double *__restrict__ tri,
+                                                               const float4 *__restrict__ sphere, int ntri, int nx,
+                                                               int ny, int nz, double ox, double oy, double oz,
+                                                               double dx, float slack, int closed,
+                                                               float *__restrict__ out) {
 #pragma clang fp contract(off)
+    constexpr int kSdfBlock = 64 * kWaves;
     __shared__ unsigned near_up[64];   // per node: bits of the smallest bound so far
-    __shared__ double part[kSdfWaves][64];
-    __shared__ float red[3][kSdfWaves];
-    __shared__ int red_at[kSdfWaves];
+    __shared__ double part[kWaves][64];
+    __shared__ float red[3][kWaves];
+    __shared__ int red_at[kWaves];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int bx = (nx + 3) / 4, by = (ny + 3) / 4;
     const int brick = (int)blockIdx.x;
@@ -181,10 +215,20 @@ __global__ void __launch_bounds__(kSdfBlock) k_sdf_from_mesh(const double *__res
     const float half = 1.5f * (float)dx;
     const float cx = __shfl(fx, 0, 64) + half, cy = __shfl(fy, 0, 64) + half, cz = __shfl(fz, 0, 64) + half;
     const float brad = 1.7321f * half + slack;
+    // a small mesh's spheres are made here, a triangle per lane, without a launch before this one
+    float4 own = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (kWaves == 1)
+        if (lane < ntri) own = tri_sphere(tri + 9 * (size_t)lane, ox, oy, oz, slack);
+    auto sphere_of = [&](int t) {
+        if constexpr (kWaves == 1)
+            return own;
+        else
+            return t < ntri ? sphere[t] : make_float4(0.f, 0.f, 0.f, 0.f);
+    };
     float c2 = __builtin_inff(), rmax = 0.f, edge = 0.f;
     int nearest = 0;
     for (int t = wave * 64 + lane; t < ntri; t += kSdfBlock) {
-        const float4 s = sphere[t];
+        const float4 s = sphere_of(t);
         const float ax = cx - s.x, ay = cy - s.y, az = cz - s.z, d2 = ax * ax + ay * ay + az * az;
         const bool sound = s.w < 3.4e38f;
         if (sound && d2 < c2) {
@@ -212,7 +256,7 @@ __global__ void __launch_bounds__(kSdfBlock) k_sdf_from_mesh(const double *__res
     }
     if (wave == 0) near_up[lane] = 0x7f800000u;
     __syncthreads();
-    for (int w = 0; w < kSdfWaves; w++) {
+    for (int w = 0; w < kWaves; w++) {
         if (red[0][w] < c2) {
             c2 = red[0][w];
             nearest = red_at[w];
@@ -233,7 +277,7 @@ __global__ void __launch_bounds__(kSdfBlock) k_sdf_from_mesh(const double *__res
     };
     measure(nearest);
     for (int t0 = wave * 64; t0 < ntri; t0 += kSdfBlock) {
-        const float4 s = t0 + lane < ntri ? sphere[t0 + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4 s = sphere_of(t0 + lane);
         const float ax = cx - s.x, ay = cy - s.y, az = cz - s.z, reach = brick_up + s.w;
         // both tests are written so that a NaN keeps the triangle
         unsigned long long keep =
@@ -251,7 +295,7 @@ __global__ void __launch_bounds__(kSdfBlock) k_sdf_from_mesh(const double *__res
     }
     part[wave][lane] = best;
     __syncthreads();
-    for (int w = 0; w < kSdfWaves; w++) best = fmin(best, part[w][lane]);
+    for (int w = 0; w < kWaves; w++) best = fmin(best, part[w][lane]);
     __syncthreads();
     const double dist = sqrt(best);
     bool interior = false;
@@ -271,7 +315,7 @@ __global__ void __launch_bounds__(kSdfBlock) k_sdf_from_mesh(const double *__res
         double number = 0.0;
         bool unsure = false;
         for (int t0 = wave * 64; t0 < ntri; t0 += kSdfBlock) {
-            const float4 s = t0 + lane < ntri ? sphere[t0 + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+            const float4 s = sphere_of(t0 + lane);
             const float ax = cx - s.x, ay = cy - s.y, az = cz - s.z, reach = brad + s.w;
             unsigned long long near = __ballot(t0 + lane < ntri && !(ax * ax + ay * ay + az * az > reach * reach * 1.00001f));
             for (; near; near &= near - 1) {
@@ -287,13 +331,16 @@ __global__ void __launch_bounds__(kSdfBlock) k_sdf_from_mesh(const double *__res
         part[wave][lane] = (unsure ? 1e6 : 0.0) + number + turns / (4.0 * M_PI);
         __syncthreads();
         double sum = 0.0;
-        for (int w = 0; w < kSdfWaves; w++) sum += part[w][lane];
+        for (int w = 0; w < kWaves; w++) sum += part[w][lane];
         number = rint(sum);
         interior = fabs(number) > 0.5;
         todo &= __ballot(!(fabs(sum - number) < 1e-3) || fabs(number) > 5e5);
     }
     if (wave > 0) return;
-    if (__popcll(todo) > 24) {  // every node for itself is cheaper then
+    // Every node for itself, or one after the other by the whole wave, 64
+    // triangles at a time, whose additions in order cost as much as two more
+    // solid angles: the latter for few nodes and many triangles.
+    if (__popcll(todo) > (kWaves == 1 ? 3 * ntri / 8 : 24)) {
         double wind = 0.0;
         for (int t = 0; t < ntri; t++) wind += tri_solid_angle(tri + 9 * (size_t)t, px, py, pz);
         if (todo >> lane & 1ull) interior = fabs(wind) > 2.0 * M_PI;  // |winding number| > 1/2
@@ -305,9 +352,15 @@ __global__ void __launch_bounds__(kSdfBlock) k_sdf_from_mesh(const double *__res
         double wind = 0.0;
         for (int t0 = 0; t0 < ntri; t0 += 64) {
             const double a = t0 + lane < ntri ? tri_solid_angle(tri + 9 * (size_t)(t0 + lane), qx, qy, qz) : 0.0;
-            for (int l = 0; l < 64; l++)
+            auto add = [&](int l) {
                 wind += __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(a), l),
                                          __builtin_amdgcn_readlane(__double2loint(a), l));
+            };
+            if (ntri - t0 >= 64) {
+                for (int l = 0; l < 64; l++) add(l);
+            } else {
+                for (int l = 0; l < ntri - t0; l++) add(l);
+            }
         }
         if (lane == rep) interior = fabs(wind) > 2.0 * M_PI;
     }
@@ -562,12 +615,19 @@ int bbx_sdf_from_mesh(const double *vertices, int nvertices, const int *triangle
     if (e == hipSuccess) e = hipMemcpy(dtri, tri.data(), sizeof(double) * tri.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) {
         float4 *sphere = (float4 *)((char *)dtri + tri_bytes);
-        k_tri_spheres<<<(unsigned)((ntriangles + 255) / 256), 256>>>(dtri, ntriangles, pmin[0], pmin[1], pmin[2],
-                                                                     slack, sphere);
+        const bool direct = ntriangles <= kSdfFew || (ntriangles <= 2 * kSdfFew && total <= kSdfFewNodes);
+        const int waves = ntriangles <= kSdfOneWave ? 1 : kSdfWaves;
+        if (waves > 1)
+            k_tri_spheres<<<(unsigned)((ntriangles + 255) / 256), 256>>>(dtri, ntriangles, pmin[0], pmin[1], pmin[2],
+                                                                         slack, sphere);
         const long long bricks = (long long)((s->nodes[0] + 3) / 4) * ((s->nodes[1] + 3) / 4) * ((s->nodes[2] + 3) / 4);
-        k_sdf_from_mesh<<<(unsigned)bricks, kSdfBlock>>>(
-            dtri, sphere, ntriangles, s->nodes[0], s->nodes[1], s->nodes[2], pmin[0], pmin[1], pmin[2], sp, slack,
-            closed ? 1 : 0, s->field);
+        if (direct)
+            k_sdf_all_pairs<<<(unsigned)((total + 63) / 64), 64>>>(dtri, ntriangles, s->nodes[0], s->nodes[1],
+                                                                   s->nodes[2], pmin[0], pmin[1], pmin[2], sp, s->field);
+        else
+            (waves == 1 ? k_sdf_from_mesh<1> : k_sdf_from_mesh<kSdfWaves>)<<<(unsigned)bricks, 64 * waves>>>(
+                dtri, sphere, ntriangles, s->nodes[0], s->nodes[1], s->nodes[2], pmin[0], pmin[1], pmin[2], sp, slack,
+                closed ? 1 : 0, s->field);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipDeviceSynchronize();
