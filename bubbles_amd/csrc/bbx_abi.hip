@@ -386,11 +386,16 @@ static void dfree(T *&p) {
     p = nullptr;
 }
 
+static void drop_bins(bbx_solver *s) {
+    dfree(s->bins);
+    dfree(s->blocks);
+}
+
 static void free_all(bbx_solver *s) {
     dfree(s->posA); dfree(s->posB); dfree(s->velA); dfree(s->velB);
     dfree(s->cellA); dfree(s->cellB); dfree(s->home);
     dfree(s->cell_count); dfree(s->cell_start); dfree(s->scan_tmp);
-    dfree(s->key); dfree(s->newc); dfree(s->rank_tmp); dfree(s->tmp_idx); dfree(s->hash_tmp); dfree(s->bins);
+    dfree(s->key); dfree(s->newc); dfree(s->rank_tmp); dfree(s->tmp_idx); dfree(s->hash_tmp); drop_bins(s);
     dfree(s->nbr16); dfree(s->nbr32); dfree(s->nbr_cnt); dfree(s->tile_tab);
     dfree(s->rho); dfree(s->pres); dfree(s->rho_star); dfree(s->xq); dfree(s->vr);
     dfree(s->force); dfree(s->fp); dfree(s->xstar); dfree(s->feat); dfree(s->pwarm);
@@ -418,14 +423,13 @@ static void free_all(bbx_solver *s) {
     s->stream = nullptr;
 }
 
-// Key bins for the solver's grid and capacity, in place of those it has.
-// Without room for them the grid pass does without.
-static void alloc_bins(bbx_solver *s) {
-    const size_t cells = (size_t)s->grid.total + 1, N = (size_t)s->stride;
-    dfree(s->bins);
+// The blocks behind the key bins for the solver's capacity, in place of those
+// it has.  Without room for them the grid pass does without bins.
+static void alloc_blocks(bbx_solver *s) {
     s->bin_pass = 0;
-    if (cells <= std::max((size_t)kBinCells, N) && dalloc(&s->bins, grid_bins_words(cells - 1, N)) != BBX_OK) {
-        s->bins = nullptr;
+    dfree(s->blocks);
+    if (s->bins && dalloc(&s->blocks, grid_block_words((size_t)s->stride)) != BBX_OK) {
+        drop_bins(s);
         (void)hipGetLastError();
     }
 }
@@ -563,7 +567,10 @@ int bbx_solver_create(int kind, const bbx_params *params, const double *pos, con
         s->counters = s->step->counters;
     }
     if (!rc) rc = dalloc(&s->flag, 1);
-    if (!rc) alloc_bins(s);
+    if (!rc && cells <= std::max((size_t)kBinCells, N)) {
+        if (dalloc(&s->bins, grid_bin_words(cells - 1)) != BBX_OK) (void)hipGetLastError();
+        alloc_blocks(s);
+    }
     // one pinned block (an allocation costs about 100 us): the loop signal,
     // the step block's copy, a flag, and the ring of the field downloads
     const size_t pin_step = 256, pin_flag = pin_step + (sizeof(StepBlock) + 255) / 256 * 256, pin_ring = pin_flag + 256;
@@ -611,8 +618,8 @@ int bbx_solver_create(int kind, const bbx_params *params, const double *pos, con
     }
     // FP64 -> FP32, id in pos.w, velocity w = 0 (no previous pressure);
     // fields at zero, and every slot in no chain until Setup distributes
-    rc = upload_vec4(s, s->posA, pos, (size_t)n, N, true);
-    if (!rc) rc = upload_vec4(s, s->velA, vel, (size_t)n, N, false);
+    rc = upload_vec4(s, s->posA, pos, (size_t)n, N, 0);
+    if (!rc) rc = upload_vec4(s, s->velA, vel, (size_t)n, N, -1);
     if (!rc) rc = launch_fill_int(s, (int *)s->step, 0, sizeof(StepBlock) / sizeof(int));
     if (!rc) rc = launch_fill_int(s, s->flag, 0, 1);
     if (!rc) rc = launch_init_fields(s);
@@ -723,21 +730,108 @@ int bbx_solver_download(bbx_solver *s, int field, double *out) {
 // ---------------------------------------------------------------------------
 }  // extern "C"
 namespace {
-// replace *p by a buffer of new_n elements holding the first keep elements
+// What has grown when a first attempt runs out of memory is not grown again.
+struct Progress {
+    int at = 0, done = 0;
+    bool due() { return at++ >= done; }
+    int ok() {
+        done = at;
+        return BBX_OK;
+    }
+};
+
+// replace *p by a buffer of new_n elements (the stream is idle)
 template <typename T>
-int regrow(bbx_solver *s, T *&p, size_t new_n, size_t keep) {
+int renew(Progress &pr, T *&p, size_t new_n) {
+    if (!pr.due()) return BBX_OK;
     T *q = nullptr;
     BBX_CHECK(dalloc(&q, new_n));
-    if (keep && p) {
-        hipError_t e = hipMemcpyAsync(q, p, sizeof(T) * keep, hipMemcpyDeviceToDevice, s->stream);
-        if (e != hipSuccess) {
-            dfree(q);
-            return fail(BBX_E_HIP, std::string("regrow copy: ") + hipGetErrorString(e));
-        }
-    }
-    BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
     dfree(p);
     p = q;
+    return pr.ok();
+}
+
+// Buffers that keep their first elements: the copies are queued, and the old
+// buffers freed behind one synchronisation.
+struct Regrow {
+    bbx_solver *s;
+    Progress &pr;
+    std::vector<void *> old;
+    Regrow(bbx_solver *solver, Progress &progress) : s(solver), pr(progress) { old.reserve(16); }
+    ~Regrow() {
+        (void)hipStreamSynchronize(s->stream);
+        for (void *p : old) (void)hipFree(p);
+    }
+    template <typename T>
+    int operator()(T *&p, size_t new_n, size_t keep) {
+        if (!pr.due()) return BBX_OK;
+        T *q = nullptr;
+        BBX_CHECK(dalloc(&q, new_n));
+        if (keep) {
+            const hipError_t e = hipMemcpyAsync(q, p, sizeof(T) * keep, hipMemcpyDeviceToDevice, s->stream);
+            if (e != hipSuccess) {
+                dfree(q);
+                return fail(BBX_E_HIP, std::string("regrow copy: ") + hipGetErrorString(e));
+            }
+        }
+        old.push_back(p);
+        p = q;
+        return pr.ok();
+    }
+};
+
+int grow_fields(bbx_solver *s, size_t S0, size_t S1, Progress &pr) {
+    const size_t n = (size_t)s->n;
+    pr.at = 0;
+    // particle state kept (first n slots), scratch and per-substep tables not
+    {
+        Regrow regrow(s, pr);
+        BBX_CHECK(regrow(s->posA, S1, n));
+        BBX_CHECK(regrow(s->velA, S1, n));
+        BBX_CHECK(regrow(s->cellA, S1, n));
+        BBX_CHECK(regrow(s->home, S1, n));
+        BBX_CHECK(regrow(s->force, S1, n));
+        BBX_CHECK(regrow(s->fp, S1, n));
+        BBX_CHECK(regrow(s->xstar, S1, n));
+        BBX_CHECK(regrow(s->xq, S1, n));
+        BBX_CHECK(regrow(s->rho, S1, n));
+        BBX_CHECK(regrow(s->pres, S1, n));
+        BBX_CHECK(regrow(s->rho_star, S1, n));
+        BBX_CHECK(regrow(s->pwarm, S1, n));
+    }
+    BBX_CHECK(renew(pr, s->posB, S1));
+    BBX_CHECK(renew(pr, s->velB, S1));
+    if (s->vr) BBX_CHECK(renew(pr, s->vr, S1));
+    BBX_CHECK(renew(pr, s->cellB, S1));
+    BBX_CHECK(renew(pr, s->key, S1));
+    BBX_CHECK(renew(pr, s->newc, S1));
+    BBX_CHECK(renew(pr, s->rank_tmp, S1));
+    BBX_CHECK(renew(pr, s->tmp_idx, S1));
+    BBX_CHECK(renew(pr, s->hash_tmp, S1));
+    BBX_CHECK(renew(pr, s->nbr16, S1 * kBucket));
+    BBX_CHECK(renew(pr, s->nbr32, S1 * kBucket));
+    BBX_CHECK(renew(pr, s->nbr_cnt, S1));
+    // features are feature-major with the row stride: copy row by row
+    if (pr.due()) {
+        float *q = nullptr;
+        BBX_CHECK(dalloc(&q, S1 * BBX_NFEAT));
+        for (int f = 0; f < BBX_NFEAT && n; f++)
+            BBX_HIP_CHECK(hipMemcpyAsync(q + (size_t)f * S1, s->feat + (size_t)f * S0, sizeof(float) * n,
+                                         hipMemcpyDeviceToDevice, s->stream));
+        BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
+        dfree(s->feat);
+        s->feat = q;
+        pr.ok();
+    }
+    const size_t ntiles = (S1 + kBlock - 1) / kBlock;
+    BBX_CHECK(renew(pr, s->tile_tab, ntiles * kTabIntsHost));
+    s->ntiles = (int)ntiles;
+    BBX_CHECK(launch_fill_int(s, s->nbr_cnt, 0, S1));
+    BBX_CHECK(launch_fill_int(s, s->tile_tab, 0, ntiles * kTabIntsHost));
+    // slots beyond n are in no chain
+    BBX_CHECK(launch_fill_int(s, s->cellA + n, (int)s->grid.total, S1 - n));
+    BBX_CHECK(launch_fill_int(s, s->home + n, (int)s->grid.total, S1 - n));
+    BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
     return BBX_OK;
 }
 }  // namespace
@@ -749,57 +843,17 @@ int bbx_solver_reserve(bbx_solver *s, int capacity) {
     const size_t S0 = (size_t)s->stride;
     const size_t S1 = (size_t)(((capacity + 63) / 64) * 64);
     if (S1 <= S0) return BBX_OK;
-    const size_t n = (size_t)s->n;
     BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
-    dfree(s->bins);  // room for the fields first
-    // particle state kept (first n slots), scratch and per-substep tables not
-    BBX_CHECK(regrow(s, s->posA, S1, n));
-    BBX_CHECK(regrow(s, s->velA, S1, n));
-    BBX_CHECK(regrow(s, s->cellA, S1, n));
-    BBX_CHECK(regrow(s, s->home, S1, n));
-    BBX_CHECK(regrow(s, s->force, S1, n));
-    BBX_CHECK(regrow(s, s->fp, S1, n));
-    BBX_CHECK(regrow(s, s->xstar, S1, n));
-    BBX_CHECK(regrow(s, s->xq, S1, n));
-    BBX_CHECK(regrow(s, s->rho, S1, n));
-    BBX_CHECK(regrow(s, s->pres, S1, n));
-    BBX_CHECK(regrow(s, s->rho_star, S1, n));
-    BBX_CHECK(regrow(s, s->pwarm, S1, n));
-    BBX_CHECK(regrow(s, s->posB, S1, 0));
-    BBX_CHECK(regrow(s, s->velB, S1, 0));
-    if (s->vr) BBX_CHECK(regrow(s, s->vr, S1, 0));
-    BBX_CHECK(regrow(s, s->cellB, S1, 0));
-    BBX_CHECK(regrow(s, s->key, S1, 0));
-    BBX_CHECK(regrow(s, s->newc, S1, 0));
-    BBX_CHECK(regrow(s, s->rank_tmp, S1, 0));
-    BBX_CHECK(regrow(s, s->tmp_idx, S1, 0));
-    BBX_CHECK(regrow(s, s->hash_tmp, S1, 0));
-    BBX_CHECK(regrow(s, s->nbr16, S1 * kBucket, 0));
-    BBX_CHECK(regrow(s, s->nbr32, S1 * kBucket, 0));
-    BBX_CHECK(regrow(s, s->nbr_cnt, S1, 0));
-    // features are feature-major with the row stride: copy row by row
-    {
-        float *q = nullptr;
-        BBX_CHECK(dalloc(&q, S1 * BBX_NFEAT));
-        for (int f = 0; f < BBX_NFEAT && n; f++)
-            BBX_HIP_CHECK(hipMemcpyAsync(q + (size_t)f * S1, s->feat + (size_t)f * S0, sizeof(float) * n,
-                                         hipMemcpyDeviceToDevice, s->stream));
-        BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
-        dfree(s->feat);
-        s->feat = q;
+    Progress pr;
+    int rc = grow_fields(s, S0, S1, pr);
+    if (rc == BBX_E_NOMEM && s->bins) {  // the fields come before the bins
+        drop_bins(s);
+        rc = grow_fields(s, S0, S1, pr);
     }
-    s->ntiles = (int)((S1 + kBlock - 1) / kBlock);
-    BBX_CHECK(regrow(s, s->tile_tab, (size_t)s->ntiles * kTabIntsHost, 0));
-    BBX_HIP_CHECK(hipMemset(s->nbr_cnt, 0, sizeof(int) * S1));
-    BBX_HIP_CHECK(hipMemset(s->tile_tab, 0, sizeof(int) * (size_t)s->ntiles * kTabIntsHost));
-    // slots beyond n are in no chain
-    std::vector<int> none(S1 - n, (int)s->grid.total);
-    BBX_HIP_CHECK(hipMemcpy(s->cellA + n, none.data(), sizeof(int) * none.size(), hipMemcpyHostToDevice));
-    BBX_HIP_CHECK(hipMemcpy(s->home + n, none.data(), sizeof(int) * none.size(), hipMemcpyHostToDevice));
+    BBX_CHECK(rc);
     s->stride = (int)S1;
-    alloc_bins(s);
+    alloc_blocks(s);
     fill_sim_const(s);
-    fetch_grow(s, S1);
     return BBX_OK;
 }
 
@@ -821,21 +875,12 @@ int bbx_solver_append(bbx_solver *s, const double *pos, const double *vel, int c
     BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
     // AppendData (src/core/particle.h:232-240): ids n0.., zero force, and
     // no previous pressure for the warm start
-    std::vector<float4> hp((size_t)count), hv((size_t)count);
-    for (int k = 0; k < count; k++) {
-        const int id = n0 + k;
-        float idf;
-        std::memcpy(&idf, &id, sizeof(int));
-        hp[k] = make_float4((float)pos[3 * (size_t)k], (float)pos[3 * (size_t)k + 1], (float)pos[3 * (size_t)k + 2], idf);
-        hv[k] = vel ? make_float4((float)vel[3 * (size_t)k], (float)vel[3 * (size_t)k + 1], (float)vel[3 * (size_t)k + 2], 0.f)
-                    : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    BBX_HIP_CHECK(hipMemcpy(s->posA + n0, hp.data(), sizeof(float4) * count, hipMemcpyHostToDevice));
-    BBX_HIP_CHECK(hipMemcpy(s->velA + n0, hv.data(), sizeof(float4) * count, hipMemcpyHostToDevice));
-    BBX_HIP_CHECK(hipMemset(s->force + n0, 0, sizeof(float4) * count));
-    BBX_HIP_CHECK(hipMemset(s->fp + n0, 0, sizeof(float4) * count));
-    BBX_HIP_CHECK(hipMemset(s->rho + n0, 0, sizeof(float) * count));
-    BBX_HIP_CHECK(hipMemset(s->pres + n0, 0, sizeof(float) * count));
+    BBX_CHECK(upload_vec4(s, s->posA + n0, pos, (size_t)count, (size_t)count, n0));
+    BBX_CHECK(upload_vec4(s, s->velA + n0, vel, (size_t)count, (size_t)count, -1));
+    BBX_CHECK(launch_fill_int(s, (int *)(s->force + n0), 0, 4 * (size_t)count));
+    BBX_CHECK(launch_fill_int(s, (int *)(s->fp + n0), 0, 4 * (size_t)count));
+    BBX_CHECK(launch_fill_int(s, (int *)(s->rho + n0), 0, (size_t)count));
+    BBX_CHECK(launch_fill_int(s, (int *)(s->pres + n0), 0, (size_t)count));
     s->n = n0 + count;
     fill_sim_const(s);
     // DistributeByParticleList (src/core/grid.h:358-387): each new particle

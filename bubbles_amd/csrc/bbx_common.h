@@ -260,7 +260,7 @@ struct bbx_solver {
     bool counts_clear = false;                 // cell_count is all zeros (a grid pass leaves it so)
     // keys of each cell's particles and the blocks behind full bins (see
     // k_hash); null for grids of many more cells than particles
-    unsigned long long *bins = nullptr;
+    unsigned long long *bins = nullptr, *blocks = nullptr;
     unsigned bin_pass = 0;  // number of the last pass that used them
     int *scan_tmp = nullptr;
     size_t scan_tmp_elems = 0;
@@ -340,7 +340,8 @@ int distribute(bbx_solver *s, bool force_full, bool buckets, bool with_pressure,
 // tile tables + bucket build (the latter is where the warm start is chosen)
 // clear / clear_n: an int range set to zero on the way (the substep's step
 // block behind its counters, which this sets)
-size_t grid_bins_words(size_t cells, size_t stride);  // 8-byte words of the key bins and the blocks behind them
+size_t grid_bin_words(size_t cells);     // 8-byte words of the key bins
+size_t grid_block_words(size_t stride);  // and of the blocks behind them
 int distribute_grid(bbx_solver *s, bool force_full, int append_from, int *clear = nullptr,
                     size_t clear_n = 0);
 int build_buckets(bbx_solver *s, bool with_pressure, int feat_mode, const StepConst *st);

@@ -80,9 +80,21 @@ int fetch_init(bbx_solver *s, char *pinned, char *device, size_t bytes) {
     return BBX_OK;
 }
 
-void fetch_grow(bbx_solver *s, size_t stride) {
+void fetch_free(bbx_solver *s) {
     FetchRing *r = s->fetch;
-    const size_t want = fetch_ring_bytes(stride);
+    if (!r) return;
+    for (hipEvent_t e : r->ev)
+        if (e) (void)hipEventDestroy(e);
+    if (r->own) (void)hipHostFree(r->own);
+    delete r;
+    s->fetch = nullptr;
+}
+
+// A larger ring for a set that has grown; without one the smaller one serves.
+// Not before a field wants it: pinned memory of 2 MB or more takes 300 us.
+static void fetch_grow(bbx_solver *s) {
+    FetchRing *r = s->fetch;
+    const size_t want = fetch_ring_bytes((size_t)s->stride);
     if (r->bytes >= want) return;
     char *p = nullptr, *d = nullptr;
     if (hipHostMalloc((void **)&p, want + 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
@@ -95,16 +107,6 @@ void fetch_grow(bbx_solver *s, size_t stride) {
     r->own = r->ring = p;
     r->d_ring = d;
     r->bytes = want;
-}
-
-void fetch_free(bbx_solver *s) {
-    FetchRing *r = s->fetch;
-    if (!r) return;
-    for (hipEvent_t e : r->ev)
-        if (e) (void)hipEventDestroy(e);
-    if (r->own) (void)hipHostFree(r->own);
-    delete r;
-    s->fetch = nullptr;
 }
 
 // what the kernel saw of the id table; the field is not given out where it is corrupt
@@ -207,9 +209,9 @@ struct Pipe {
 int fetch_by_id(bbx_solver *s, const FieldSource &f, const FetchTake &take) {
     if (s->n == 0) return BBX_OK;
     FetchRing *r = s->fetch;
-    int *bad = (int *)(r->ring + r->bytes);
-    __atomic_store_n(bad, 0, __ATOMIC_RELEASE);
     const size_t all = (size_t)s->n * f.width;
+    if (all * sizeof(float) > r->bytes) fetch_grow(s);
+    __atomic_store_n((int *)(r->ring + r->bytes), 0, __ATOMIC_RELEASE);
     if (all * sizeof(float) <= r->bytes) {
         BBX_CHECK(launch_by_id(s, f, 0, s->n, (float *)r->d_ring));
         BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
@@ -234,7 +236,7 @@ int fetch_by_id(bbx_solver *s, const FieldSource &f, const FetchTake &take) {
     return BBX_OK;
 }
 
-int upload_vec4(bbx_solver *s, float4 *dst, const double *xyz, size_t n, size_t rows, bool with_ids) {
+int upload_vec4(bbx_solver *s, float4 *dst, const double *xyz, size_t n, size_t rows, int first_id) {
     FetchRing *r = s->fetch;
     const size_t slot = r->bytes / kFetchSlots, per = slot / sizeof(float4);
     size_t c = 0;
@@ -246,8 +248,8 @@ int upload_vec4(bbx_solver *s, float4 *dst, const double *xyz, size_t n, size_t 
         for (size_t i = lo; i < hi; i++) {
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
             if (i < n && xyz) v = make_float4((float)xyz[3 * i], (float)xyz[3 * i + 1], (float)xyz[3 * i + 2], 0.f);
-            if (i < n && with_ids) {
-                const int id = (int)i;
+            if (i < n && first_id >= 0) {
+                const int id = first_id + (int)i;
                 std::memcpy(&v.w, &id, sizeof(int));
             }
             h[i - lo] = v;

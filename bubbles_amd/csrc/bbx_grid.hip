@@ -391,9 +391,10 @@ __global__ void __launch_bounds__(kBlock) k_hash(SimConst c, const float4 *__res
     }
 }
 
-// bins, then the table of blocks, then the blocks (see BinKeys)
+size_t grid_bin_words(size_t cells) { return cells * kBinCap; }
+// the table of blocks, then the blocks (see BinKeys)
 static size_t bin_blocks(size_t stride) { return stride / (kBinCap / 2) + 64; }
-size_t grid_bins_words(size_t cells, size_t stride) { return cells * kBinCap + bin_blocks(stride) * (kBinCap + 1); }
+size_t grid_block_words(size_t stride) { return bin_blocks(stride) * (kBinCap + 1); }
 
 // What the pass reports and leaves behind, done by the last launch that may
 // (thread t of all): statistics, the higher-level flag, the cell counts back
@@ -1552,12 +1553,11 @@ int distribute_grid(bbx_solver *s, bool force_full, int append_from, int *clear,
     BinKeys bk{};
     if (bins) {
         const size_t nblk = bin_blocks((size_t)s->stride);
-        unsigned long long *tag = s->bins + (cells - 1) * kBinCap;
         if (s->bin_pass == 0 || s->bin_pass + 1 == 1u << kTagPassBits) {  // the table holds nothing yet, or any pass
-            BBX_CHECK(launch_fill_int(s, reinterpret_cast<int *>(tag), 0, 2 * nblk));
+            BBX_CHECK(launch_fill_int(s, reinterpret_cast<int *>(s->blocks), 0, 2 * nblk));
             s->bin_pass = 0;
         }
-        bk = BinKeys{s->bins, tag, tag + nblk, s->tmp_idx, (unsigned)nblk, ++s->bin_pass};
+        bk = BinKeys{s->bins, s->blocks, s->blocks + nblk, s->tmp_idx, (unsigned)nblk, ++s->bin_pass};
     }
     const PassEnd end{s->cell_count, cells, s->flag, force_full ? 1 : 0, append_from >= 0 ? 1 : 0, s->counters,
                       clear, clear_n};
