@@ -99,7 +99,7 @@ __device__ __forceinline__ void integrate_one(const SimConst &c, float dt, float
 // streams: the bucket kernel writes the pairs xq and vr (vr in the half of
 // the velocity ping-pong that the integration fills later), which costs it
 // 2 us at 1M particles.  Put together here, through registers, they cost this
-// kernel 15 us of 90.
+// kernel 15 us of 90; mode 0, which runs on whatever the fields hold, does that.
 //
 // Two lanes per particle: the two LDS arrays allow only two workgroups per
 // CU, so each particle's bucket is split between lanes 2p and 2p + 1 (even
@@ -107,6 +107,9 @@ __device__ __forceinline__ void integrate_one(const SimConst &c, float dt, float
 // added with one lane exchange.
 // ---------------------------------------------------------------------------
 constexpr int kNpThreads = 2 * kBlock;
+struct Pair {
+    float4 x, v;
+};
 
 template <int kMode, bool kList>
 __global__ void __launch_bounds__(kNpThreads) __attribute__((amdgpu_waves_per_eu(4))) k_nonpressure(SimConst c, StepConst st, NbrTab nb,
@@ -147,12 +150,23 @@ __global__ void __launch_bounds__(kNpThreads) __attribute__((amdgpu_waves_per_eu
         if (kWarm) qi = xq[i].w;
         first = nbr_prefetch<2, 2>(nb.n16, nb.n32, staged, i, c.stride, half);
     }
+    auto pair_of = [&](int j) {  // mode 0: from the fields as they are
+        const float4 v = vel[j];
+        return Pair{pos[j], make_float4(v.x, v.y, v.z, fast_rcp(rho[j]))};
+    };
     if (in_lds) {
-        tab_stage_dma(tt, [&](int j, int e) {
-            lds_dma16(xq + j, sx + e);
-            lds_dma16(vr + j, sv + e);
-        });
-        lds_dma_wait();
+        if constexpr (kMode == 0) {
+            tab_stage_with(tt, pair_of, [&](int e, const Pair &p) {
+                sx[e] = p.x;
+                sv[e] = p.v;
+            });
+        } else {
+            tab_stage_dma(tt, [&](int j, int e) {
+                lds_dma16(xq + j, sx + e);
+                lds_dma16(vr + j, sv + e);
+            });
+            lds_dma_wait();
+        }
     }
     __syncthreads();
     if (!valid) return;  // the lane pair shares validity
@@ -169,8 +183,14 @@ __global__ void __launch_bounds__(kNpThreads) __attribute__((amdgpu_waves_per_eu
                 b = lds_at(sv, j);
             } else {
                 const int g = staged ? (live ? tab_global(tt, j >> kSlotShift) : i) : j;
-                a = xq[g];
-                b = vr[g];
+                if constexpr (kMode == 0) {
+                    const Pair p = pair_of(g);
+                    a = p.x;
+                    b = p.v;
+                } else {
+                    a = xq[g];
+                    b = vr[g];
+                }
             }
             const float dx = xi.x - a.x, dy = xi.y - a.y, dz = xi.z - a.z;
             // no branches and no masks: the cutoff is the clamped factor x,
@@ -695,25 +715,8 @@ static NbrTab nbr_tab(const bbx_solver *s) {
     return NbrTab{s->nbr16, s->nbr32, s->nbr_cnt, s->tile_tab};
 }
 
-// the gather's inputs from the fields as they are now (a substep's come from
-// its bucket kernel)
-__global__ void __launch_bounds__(kBlock) k_pair_inputs(int n, const float4 *__restrict__ pos,
-                                                        const float4 *__restrict__ vel,
-                                                        const float *__restrict__ rho, float4 *__restrict__ xq,
-                                                        float4 *__restrict__ vr) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 x = pos[i], v = vel[i];
-    xq[i] = make_float4(x.x, x.y, x.z, 0.f);
-    vr[i] = make_float4(v.x, v.y, v.z, fast_rcp(rho[i]));
-}
-
 int run_nonpressure(bbx_solver *s, const StepConst &st, int mode) {
     if (s->n == 0) return BBX_OK;
-    if (mode == 0) {
-        k_pair_inputs<<<nblocks(s->n), kBlock, 0, s->stream>>>(s->n, s->posA, s->velA, s->rho, s->xq, s->velB);
-        BBX_HIP_CHECK(hipGetLastError());
-    }
     const unsigned nb = nblocks(s->n);
     const NbrTab t = nbr_tab(s);
 #define BBX_NP(M)                                                                                            \
