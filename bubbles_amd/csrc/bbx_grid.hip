@@ -285,23 +285,28 @@ struct BinKeys {
         return __umulhi(h * 0x2C1B3C6Du, nblk);
     }
     __device__ __forceinline__ unsigned after(unsigned h) const { return h + 1 < nblk ? h + 1 : 0u; }
-    // the block, entered if it is new
+    // The block, entered if it is new.  The table is never full and a block
+    // that is read has been entered, so both searches end at it; the bound on
+    // their steps only says that they end.
     __device__ __forceinline__ unsigned enter(int cell, unsigned block) const {
         const unsigned long long w = want(cell, block);
-        for (unsigned h = home(cell, block);; h = after(h)) {
+        unsigned h = home(cell, block);
+        for (unsigned k = 0; k < nblk; k++, h = after(h)) {
             unsigned long long v = __hip_atomic_load(&tag[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (v != w && (unsigned)(v >> (64 - kTagPassBits)) != pass) {
                 const unsigned long long old = atomicCAS(&tag[h], v, w);
                 v = old == v ? w : old;  // an entry changes once in a pass
             }
-            if (v == w) return h;
+            if (v == w) break;
         }
+        return h;
     }
     // a block that an earlier launch entered, given what its home holds
     __device__ __forceinline__ unsigned find(int cell, unsigned block, unsigned long long at_home) const {
         const unsigned long long w = want(cell, block);
         unsigned h = home(cell, block);
-        for (unsigned long long v = at_home; v != w; v = tag[h]) h = after(h);
+        unsigned long long v = at_home;
+        for (unsigned k = 0; v != w && k < nblk; k++, v = tag[h]) h = after(h);
         return h;
     }
 };
