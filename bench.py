@@ -50,12 +50,12 @@ PEAK_HBM_GBS = 8000.0
 # the particle's own fields read and written once, excluding neighbour
 # re-reads and the neighbour table.
 KERNEL_BYTES = {
-    "grid_hash": 36,                   # x, old cell -> new cell, key, rank, hash
+    "grid_hash": 40,                   # x, old cell -> new cell, key, the key in its bin, hash
     "grid_scatter": 16,                # new cell, rank, start -> slot index
-    "grid_rank_move": 76,              # slot, x+id, v+p -> x+id, v+p, cell, home
+    "grid_rank_move": 96,              # new cell, key, bin, x+id, v+p, hash -> x+id, v+p, cell, home
     "tile_tables": 4,                  # home -> per-tile interval tables
-    "buckets_density": 20,             # x -> rho, count; + 2 B per bucket entry (see below)
-    "buckets_density_warm": 64,        # x, v -> rho, count, p0, p_warm, rho*, (x, q0); + bucket
+    "buckets_density": 64,             # x, v -> rho, count, (x, q), (v, 1/rho); + 2 B per bucket entry (see below)
+    "buckets_density_warm": 80,        # x, v+p -> rho, count, p0, p_warm, rho*, (x, q0), (v, 1/rho); + bucket
     "nonpressure_predict": 56,         # x, v, rho -> f, x*, rho*
     "nonpressure_warm": 60,            # x, q0, v, rho -> f, x*, rho*
     "mlp_infer": 68,                   # 16 features -> p
