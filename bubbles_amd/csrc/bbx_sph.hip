@@ -500,7 +500,7 @@ __global__ void __launch_bounds__(kBlock) k_pressure_force(SimConst c, StepConst
 // particle, as in the non-pressure gather: with one lane, the pairs put
 // together through registers (a division for every staged neighbour), IEEE
 // divisions per pair and a second launch for the moves it took 15.1 + 4.1 us
-// at 16k particles and 40.4 + 9.9 us at 241k; now 8.8 and 23.1 us.
+// at 16k particles and 40.4 + 9.9 us at 241k; now 9.2 and 23.0 us.
 //
 // The last workgroup to finish publishes the substep's statistics and its
 // largest force to the host (LoopSignal), which waits for them to choose the
