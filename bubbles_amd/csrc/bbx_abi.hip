@@ -618,8 +618,8 @@ int bbx_solver_create(int kind, const bbx_params *params, const double *pos, con
     }
     // FP64 -> FP32, id in pos.w, velocity w = 0 (no previous pressure);
     // fields at zero, and every slot in no chain until Setup distributes
-    rc = upload_vec4(s, s->posA, pos, (size_t)n, N, 0);
-    if (!rc) rc = upload_vec4(s, s->velA, vel, (size_t)n, N, -1);
+    rc = upload_vec4(s, s->posA, pos, (size_t)n, N, true);
+    if (!rc) rc = upload_vec4(s, s->velA, vel, (size_t)n, N, false);
     if (!rc) rc = launch_fill_int(s, (int *)s->step, 0, sizeof(StepBlock) / sizeof(int));
     if (!rc) rc = launch_fill_int(s, s->flag, 0, 1);
     if (!rc) rc = launch_init_fields(s);
@@ -875,8 +875,17 @@ int bbx_solver_append(bbx_solver *s, const double *pos, const double *vel, int c
     BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
     // AppendData (src/core/particle.h:232-240): ids n0.., zero force, and
     // no previous pressure for the warm start
-    BBX_CHECK(upload_vec4(s, s->posA + n0, pos, (size_t)count, (size_t)count, n0));
-    BBX_CHECK(upload_vec4(s, s->velA + n0, vel, (size_t)count, (size_t)count, -1));
+    std::vector<float4> hp((size_t)count), hv((size_t)count);
+    for (int k = 0; k < count; k++) {
+        const int id = n0 + k;
+        float idf;
+        std::memcpy(&idf, &id, sizeof(int));
+        hp[k] = make_float4((float)pos[3 * (size_t)k], (float)pos[3 * (size_t)k + 1], (float)pos[3 * (size_t)k + 2], idf);
+        hv[k] = vel ? make_float4((float)vel[3 * (size_t)k], (float)vel[3 * (size_t)k + 1], (float)vel[3 * (size_t)k + 2], 0.f)
+                    : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    BBX_HIP_CHECK(hipMemcpy(s->posA + n0, hp.data(), sizeof(float4) * count, hipMemcpyHostToDevice));
+    BBX_HIP_CHECK(hipMemcpy(s->velA + n0, hv.data(), sizeof(float4) * count, hipMemcpyHostToDevice));
     BBX_CHECK(launch_fill_int(s, (int *)(s->force + n0), 0, 4 * (size_t)count));
     BBX_CHECK(launch_fill_int(s, (int *)(s->fp + n0), 0, 4 * (size_t)count));
     BBX_CHECK(launch_fill_int(s, (int *)(s->rho + n0), 0, (size_t)count));

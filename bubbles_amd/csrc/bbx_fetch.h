@@ -40,9 +40,8 @@ int fetch_init(bbx_solver *s, char *pinned, char *device, size_t bytes);
 void fetch_free(bbx_solver *s);
 int fetch_by_id(bbx_solver *s, const FieldSource &f, const FetchTake &take);
 // n FP64 vectors (null: zeros) as FP32 rows of dst, the rest of `rows` zero;
-// first_id >= 0: row i's fourth word holds first_id + i.  Chunk by chunk
-// through the ring: two whole host copies cost 7.8 ms in first-touched pages
-// at 1M particles.
-int upload_vec4(bbx_solver *s, float4 *dst, const double *xyz, size_t n, size_t rows, int first_id);
+// with_ids: row i's fourth word holds i.  Chunk by chunk through the ring: two
+// whole host copies cost 7.8 ms in first-touched pages at 1M particles.
+int upload_vec4(bbx_solver *s, float4 *dst, const double *xyz, size_t n, size_t rows, bool with_ids);
 
 }  // namespace bbx

@@ -236,7 +236,7 @@ int fetch_by_id(bbx_solver *s, const FieldSource &f, const FetchTake &take) {
     return BBX_OK;
 }
 
-int upload_vec4(bbx_solver *s, float4 *dst, const double *xyz, size_t n, size_t rows, int first_id) {
+int upload_vec4(bbx_solver *s, float4 *dst, const double *xyz, size_t n, size_t rows, bool with_ids) {
     FetchRing *r = s->fetch;
     const size_t slot = r->bytes / kFetchSlots, per = slot / sizeof(float4);
     size_t c = 0;
@@ -248,8 +248,8 @@ int upload_vec4(bbx_solver *s, float4 *dst, const double *xyz, size_t n, size_t 
         for (size_t i = lo; i < hi; i++) {
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
             if (i < n && xyz) v = make_float4((float)xyz[3 * i], (float)xyz[3 * i + 1], (float)xyz[3 * i + 2], 0.f);
-            if (i < n && first_id >= 0) {
-                const int id = first_id + (int)i;
+            if (i < n && with_ids) {
+                const int id = (int)i;
                 std::memcpy(&v.w, &id, sizeof(int));
             }
             h[i - lo] = v;
