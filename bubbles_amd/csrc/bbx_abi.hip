@@ -808,6 +808,9 @@ int grow_fields(bbx_solver *s, size_t S0, size_t S1, Progress &pr) {
     BBX_CHECK(renew(pr, s->rank_tmp, S1));
     BBX_CHECK(renew(pr, s->tmp_idx, S1));
     BBX_CHECK(renew(pr, s->hash_tmp, S1));
+    // no counts without their tables, should the memory end here
+    BBX_CHECK(launch_fill_int(s, s->nbr_cnt, 0, S0));
+    BBX_HIP_CHECK(hipStreamSynchronize(s->stream));
     BBX_CHECK(renew(pr, s->nbr16, S1 * kBucket));
     BBX_CHECK(renew(pr, s->nbr32, S1 * kBucket));
     BBX_CHECK(renew(pr, s->nbr_cnt, S1));

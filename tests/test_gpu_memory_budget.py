@@ -1,5 +1,6 @@
 """A set grows wherever its fields have room: the key bins of the grid pass, an
-option that many cells make large, give way.  Runs in a process of its own,
+option that many cells make large, give way.  Where the fields have none, the
+set goes on as it was, whichever of them the memory ended at.  Runs in a process of its own,
 where tests/cpp/hip_faults.c stands before the HIP runtime and refuses device
 memory beyond a budget."""
 import pytest
@@ -48,3 +49,38 @@ print("done")
 
 def test_growth_within_the_fields_own_memory(faults):  # noqa: F811
     _run(faults, BUDGET)
+
+
+FAILED = """
+size = lambda name: word(name, C.c_size_t)
+sc = scene(16, 8, 16)
+a, b = abi.Solver(sc), abi.Solver(sc)
+for s in (a, b):
+    s.pcisph_substep(sc.dt, 3, 1e-9, abi.MODE_TEXTBOOK)
+fields = ("position", "velocity", "force", "density", "pressure")
+full = 950 * 60000
+for part in range(1, 20):  # the memory ends after more and more of the fields
+    size("faults_budget").value = size("faults_live").value + full * part // 20
+    try:
+        a.reserve(60000)
+    except abi.BbxError:
+        pass
+    else:
+        break
+    finally:
+        size("faults_budget").value = 0
+    assert a.capacity() == b.capacity()
+    for f in fields:
+        assert np.array_equal(a.get(f), b.get(f)), (part, f)
+    a.stage_density()  # buckets are as they were or empty
+    for s in (a, b):
+        s.pcisph_substep(sc.dt, 3, 1e-9, abi.MODE_TEXTBOOK)
+    for f in fields:
+        assert np.array_equal(a.get(f), b.get(f)), (part, f)
+assert part > 5
+print("done")
+"""
+
+
+def test_failed_growth_leaves_a_sound_solver(faults):  # noqa: F811
+    _run(faults, FAILED)
